@@ -42,6 +42,37 @@ def test_quantiser_bit_exact(dev, dtype, dist):
     assert np.array_equal(s.float().cpu().numpy(), rs)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("N,K", [(1, 8), (5, 504), (1023, 512), (1024, 520), (1027, 1024),
+                                 (1025, 2056), (3, 8192), (1030, 8192), (2, 8200), (2, 32768),
+                                 (2, 32776), (6, 1001)])
+def test_quantiser_row_widths_ties_and_specials(dev, dtype, N, K):
+    """Both sides of every width and row-count line of the vector kernel, with
+    rows whose quotients are exact ties, all zero, tiny (fp16: scale 0) or not finite."""
+    from src.quant_utils import quantize_weight_symmetric_per_channel
+    g = torch.Generator("cpu").manual_seed(N * 7 + K)
+    w = (torch.randn(N, K, generator=g) * 0.02).to(dtype)
+    ties = (torch.randint(-254, 255, (K,), generator=g).float() * 0.5 / 64).to(dtype)
+    ties[0] = 127.0 / 64                       # scale 1/64: w/s is k or k + 0.5
+    w[0] = ties
+    if N > 4:
+        w[1] = 0
+        w[2] = 6e-8 if dtype == torch.float16 else 1e-30
+        w[3, K // 2] = float("inf")
+        w[4, K - 1] = float("nan")
+    q, s = quantize_weight_symmetric_per_channel(w.to(dev))
+    name = "bfloat16" if dtype == torch.bfloat16 else "float16"
+    keep = [i for i in range(N) if not (N > 4 and i == 4)]
+    rq, rs = oq.quantize_per_channel(w[keep].float().numpy(), name)
+    assert np.array_equal(q.cpu().numpy()[keep], rq)
+    assert np.array_equal(s.float().cpu().numpy()[keep], rs)
+    if N > 4:    # a NaN weight is written as 0 and does not enter the row maximum
+        rest = w[4:5].float().numpy()
+        rest[0, K - 1] = 0
+        rq, rs = oq.quantize_per_channel(rest, name)
+        assert np.array_equal(q.cpu().numpy()[4:5], rq) and np.array_equal(s.float().cpu().numpy()[4:5], rs)
+
+
 def _check_linear(dev, M, K, N, dtype, dist="normal", x_nc=False, seed=42):
     from src.quant_linear import W8A16Linear
     from src.quant_utils import quantize_weight_symmetric_per_channel
