@@ -19,15 +19,14 @@
 // reference's separate ops do (src/rope.py:85-86, src/model.py:23, :113-127).
 //
 // GEMV design (MI355X): the int8 weights are the only large operand and are
-// read once.  A workgroup owns a tile of RPB (8 or 16) output rows of one (or,
-// for SwiGLU, two) weight matrices; its NW waves split K.  The products run on
-// v_mfma_f32_16x16x32_{bf16,f16}: the A operand is 16 weight rows x 32 k
-// (int8 converted exactly in registers), the B operand is x^T with the
-// columns beyond M zero.  Each lane loads 16 contiguous int8 of one row; a
-// wave issues every weight load of its K slice before its first MFMA, so the
-// whole matrix is in flight at once (these GEMVs are latency-bound: a few MB
-// each).  With the RMSNorm prologue the normalised rows are staged in LDS and
-// the B operands are read from there; otherwise straight from global memory.
+// read once.  A workgroup owns a few tiles of 8 (up to 8 token rows) or 16
+// output rows of one (or, for SwiGLU, two) weight matrices and its waves split
+// K.  The products run on v_mfma_f32_16x16x32_{bf16,f16}: weight rows are the A
+// operand (int8 converted exactly in registers), x^T the B operand with the
+// columns beyond M zero.  A wave issues every load of its K slice before its
+// first MFMA, so the whole matrix is in flight at once (these GEMVs are
+// latency-bound: a few MB each).  With the RMSNorm prologue each wave
+// normalises its own slice of x in registers.
 #include <math.h>
 #include <type_traits>
 
@@ -129,291 +128,6 @@ __device__ inline float dl_lane_xor(float x, int lane) {
     auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false,
                                                false);
     return __uint_as_float((lane & 32) ? sw[0] : sw[1]);
-  }
-}
-
-// Weight row of tile row r (0..15) for tile `tile`: rows 0..RPB-1 of the tile;
-// for the RoPE epilogue a tile holds 8 rotation pairs: rows i and i+8 are head
-// dims d and d + D/2.
-template <int EPI, int RPB>
-__device__ inline int tile_row(int tile_in_mat, int r, int D) {
-  if constexpr (EPI == kEpiQkvRope) {
-    const int half = D >> 1, tiles_per_head = half >> 3;
-    const int head = tile_in_mat / tiles_per_head, j = tile_in_mat % tiles_per_head;
-    return head * D + 8 * j + (r & 7) + ((r >> 3) ? half : 0);
-  } else {
-    return tile_in_mat * RPB + r;
-  }
-}
-
-template <typename T, int NW, bool NORM, int EPI, int RPB, int MR>
-__global__ __launch_bounds__(64 * NW) void layer_gemv_kernel(LayerGemvArgs a) {
-  using MM = LMfma<T>;
-  typedef typename MM::v8 v8;
-  constexpr int NMAT = EPI == kEpiSwiglu ? 2 : 1;      // A streams per tile
-  constexpr int MAXC = 8;          // 64-k chunks per wave: K = 512 * NW (host-checked)
-  // MR: rows of x the RMSNorm prologue holds (>= M)
-  extern __shared__ __align__(16) unsigned char smem[];
-  T* xs = reinterpret_cast<T*>(smem);                   // NORM: [M][K] normalised x
-  float* red_ss = reinterpret_cast<float*>(smem + (NORM ? (size_t)a.M * a.K * sizeof(T) : 0));
-  f32x4* red = reinterpret_cast<f32x4*>(smem + (NORM ? (size_t)a.M * a.K * sizeof(T) +
-                                                           (size_t)NW * MR * sizeof(float)
-                                                     : 0));
-
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int r = lane & 15, g = lane >> 4;    // A: weight row in tile / k group
-  const int m = lane & 15;                   // B: x row
-  const bool m_ok = m < a.M;
-
-  // ---- RMSNorm prologue, part 1: this thread's 16-byte column chunk of every
-  //      x row (and of the norm weight), requested before any weight load so
-  //      the statistics do not wait behind the weight stream (vmcnt retires
-  //      in order).  K = 8 * 64 * NW: one chunk per thread per row.
-  //      Every load in this kernel is unconditional (rows beyond M or N read
-  //      a clamped row and are discarded by the epilogue): a load under a
-  //      branch forces the compiler's vmcnt waits to assume it was skipped,
-  //      which would make the first wait cover the whole weight stream.
-  u32x4 xv[NORM ? MR : 1], nwv = {0, 0, 0, 0};
-  if constexpr (NORM) {
-#pragma unroll
-    for (int row = 0; row < MR; ++row)
-      xv[row] = load16(reinterpret_cast<const T*>(a.x) + (int64_t)min(row, a.M - 1) * a.x_sm +
-                       tid * 8);
-    nwv = load16(reinterpret_cast<const T*>(a.norm_w) + tid * 8);
-  }
-
-  // device position of the QKV epilogue (a scalar load, needed for the
-  // RoPE table addresses below)
-  const int64_t pos = EPI == kEpiQkvRope ? *a.pos : 0;
-
-  // ---- which matrix / tile this block owns
-  int tile = blockIdx.x;
-  int mat = 0;
-  if constexpr (EPI == kEpiQkvRope) {
-    if (tile >= a.n_tiles0) {
-      tile -= a.n_tiles0;
-      mat = 1;
-      if (tile >= a.n_tiles1) { tile -= a.n_tiles1; mat = 2; }
-    }
-  }
-  const int8_t* wm = mat == 0 ? a.w0 : (mat == 1 ? a.w1 : a.w2);
-  const int64_t w_sn = mat == 0 ? a.w_sn0 : (mat == 1 ? a.w_sn1 : a.w_sn2);
-  const int n_in_mat = tile_row<EPI, RPB>(tile, r, a.D);   // this lane's weight row
-  const int n_valid = EPI == kEpiQkvRope ? (mat == 0 ? a.Hq : a.Hkv) * a.D : a.N;
-  const bool row_ok = r < RPB && n_in_mat < n_valid;
-  // weight rows through buffer resources (host-checked: the matrix spans < 2^31 bytes):
-  // lanes of padding rows (r >= RPB, n >= N) get an out-of-range offset and
-  // load zeros without a memory access
-  const buf_rsrc wr0 = make_rsrc(wm, (uint32_t)((int64_t)(n_valid - 1) * w_sn + a.K));
-  const uint32_t wo0 = row_ok ? (uint32_t)((int64_t)n_in_mat * w_sn) : kOobOffset;
-  const buf_rsrc wr1 = make_rsrc(NMAT == 2 ? a.w1 : wm,
-                                 NMAT == 2 ? (uint32_t)((int64_t)(a.N - 1) * a.w_sn1 + a.K) : 0u);
-  const uint32_t wo1 = NMAT == 2 && row_ok ? (uint32_t)((int64_t)n_in_mat * a.w_sn1) : kOobOffset;
-
-  // ---- without the prologue the B operands come straight from global memory:
-  //      request them all first (L2 hits, they retire ahead of the weights)
-  const int c_lo = w * MAXC;
-  const int mc = min(m, a.M - 1);             // columns m >= M are discarded
-  u32x4 xr[NORM ? 1 : MAXC][2];
-  if constexpr (!NORM) {
-    // x through a buffer resource (host-checked: ((M-1)*x_sm + K)*2 < 2^31):
-    // the B-operand columns m >= M load zeros without a memory access
-    const buf_rsrc xrs = make_rsrc(a.x, (uint32_t)(((int64_t)(a.M - 1) * a.x_sm + a.K) * sizeof(T)));
-    const uint32_t xo = m_ok ? (uint32_t)((int64_t)m * a.x_sm * sizeof(T)) : kOobOffset;
-#pragma unroll
-    for (int i = 0; i < MAXC; ++i) {
-      const int k0 = (c_lo + i) * 64 + 16 * g;
-      xr[i][0] = buf_load16(xrs, xo + (uint32_t)(k0 * sizeof(T)));
-      xr[i][1] = buf_load16(xrs, xo + (uint32_t)((k0 + 8) * sizeof(T)));
-    }
-  }
-
-  // ---- issue every weight load of this wave's K slice (MAXC chunks of 64)
-  u32x4 wq[NMAT][MAXC];
-#pragma unroll
-  for (int i = 0; i < MAXC; ++i) {
-    const int k0 = (c_lo + i) * 64 + 16 * g;
-    wq[0][i] = buf_load16_nt(wr0, wo0 + (uint32_t)k0);
-    if constexpr (NMAT == 2) wq[1][i] = buf_load16_nt(wr1, wo1 + (uint32_t)k0);
-  }
-  // ---- epilogue operands (row scales, residual, RoPE table entries), issued
-  //      behind the weights so the epilogue does not start with a round trip;
-  //      unconditional, from clamped indices (lanes beyond M / N discard them)
-  T e_s0[4], e_s1[4], e_res[4], e_cos[4], e_sin[4];
-  auto load_epilogue = [&]() {
-  if constexpr (EPI == kEpiQkvRope) {
-    const T* sc = reinterpret_cast<const T*>(mat == 0 ? a.s0 : (mat == 1 ? a.s1 : a.s2));
-    const int half = a.D >> 1, tph = half >> 3;
-    const int head = tile / tph, j8 = tile % tph;
-    // rows outside the table are clamped (callers keep positions in range)
-    const int64_t crow = min(max(pos - a.rope_row0, (int64_t)0), a.rope_rows - 1);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int rr = 4 * g + i;
-      e_s0[i] = sc[head * a.D + 8 * j8 + (rr & 7) + ((rr >> 3) ? half : 0)];
-      const int ii = 8 * j8 + 4 * (g & 1) + i;
-      e_cos[i] = reinterpret_cast<const T*>(a.cos)[crow * a.c_ss + ii];
-      e_sin[i] = reinterpret_cast<const T*>(a.sin)[crow * a.c_ss + ii];
-    }
-  } else {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int nc = min(tile * RPB + 4 * g + i, a.N - 1);
-      e_s0[i] = reinterpret_cast<const T*>(a.s0)[nc];
-      if constexpr (EPI == kEpiSwiglu) e_s1[i] = reinterpret_cast<const T*>(a.s1)[nc];
-      if constexpr (EPI == kEpiResidual)
-        e_res[i] = reinterpret_cast<const T*>(a.res)[(int64_t)mc * a.res_sm + nc];
-    }
-  }
-  };
-  // 1024-thread blocks (128 VGPRs) with a prologue or two weight streams have
-  // no registers to spare: they load these at the epilogue instead
-  constexpr bool kPrefetchEpi = !(NW >= 16 && (NORM || NMAT == 2));
-  if constexpr (kPrefetchEpi) load_epilogue();
-  // keep the whole load stream issued before the prologue's first wait
-  __builtin_amdgcn_sched_barrier(0);
-
-  // ---- RMSNorm prologue, part 2: per-row sum of squares (wave shuffles, then
-  //      LDS across waves), normalised rows into LDS, rounded to T
-  if constexpr (NORM) {
-    float ss[MR];
-#pragma unroll
-    for (int row = 0; row < MR; ++row) {
-      float v[8];
-      Chunk<T>::unpack(xv[row], v);
-      float t = 0.f;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) t = fmaf(v[e], v[e], t);
-#pragma unroll
-      for (int off = 32; off >= 1; off >>= 1) t += shfl_xor_f32(t, off);
-      ss[row] = t;
-    }
-    if (lane == 0) {
-#pragma unroll
-      for (int row = 0; row < MR; ++row) red_ss[w * MR + row] = ss[row];
-    }
-    __syncthreads();
-    float wn[8];
-    Chunk<T>::unpack(nwv, wn);
-#pragma unroll
-    for (int row = 0; row < MR; ++row) {
-      if (row < a.M) {
-        float tot = 0.f;
-  #pragma unroll
-        for (int ww = 0; ww < NW; ++ww) tot += red_ss[ww * MR + row];
-        const float rstd = 1.0f / sqrtf(tot / (float)a.K + a.eps);
-        float v[8];
-        Chunk<T>::unpack(xv[row], v);
-        typedef T t8 __attribute__((ext_vector_type(8)));
-        t8 o;
-  #pragma unroll
-        for (int e = 0; e < 8; ++e) o[e] = Elem<T>::from_f32(v[e] * rstd * wn[e]);
-        *reinterpret_cast<t8*>(xs + (int64_t)row * a.K + tid * 8) = o;
-      }
-    }
-    __syncthreads();
-  }
-
-  // ---- MFMAs over the slice
-  f32x4 acc[NMAT];
-#pragma unroll
-  for (int t = 0; t < NMAT; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-  for (int i = 0; i < MAXC; ++i) {
-    const int k0 = (c_lo + i) * 64 + 16 * g;
-    v8 xb0, xb1;
-    if constexpr (NORM) {
-      const T* xp = xs + (int64_t)mc * a.K + k0;
-      xb0 = __builtin_bit_cast(v8, load16(xp));
-      xb1 = __builtin_bit_cast(v8, load16(xp + 8));
-    } else {
-      xb0 = __builtin_bit_cast(v8, xr[i][0]);
-      xb1 = __builtin_bit_cast(v8, xr[i][1]);
-    }
-#pragma unroll
-    for (int t = 0; t < NMAT; ++t) {
-      acc[t] = MM::mma(i8x8_cvt<T, v8>(wq[t][i].x, wq[t][i].y), xb0, acc[t]);
-      acc[t] = MM::mma(i8x8_cvt<T, v8>(wq[t][i].z, wq[t][i].w), xb1, acc[t]);
-    }
-  }
-
-  // ---- reduce the NW waves' partial sums
-  if (w != 0) {
-#pragma unroll
-    for (int t = 0; t < NMAT; ++t) red[((w - 1) * NMAT + t) * 64 + lane] = acc[t];
-  }
-  __syncthreads();
-  if (w != 0) return;
-#pragma unroll
-  for (int ww = 1; ww < NW; ++ww)
-#pragma unroll
-    for (int t = 0; t < NMAT; ++t) acc[t] += red[((ww - 1) * NMAT + t) * 64 + lane];
-
-  if constexpr (!kPrefetchEpi) load_epilogue();
-  // acc[t][i] = C[tile row 4*g + i][x row m]
-  auto f32_of = [](T v) { return Elem<T>::to_f32(v); };
-  if constexpr (EPI == kEpiQkvRope) {
-    // rows 4g+i (g < 2) are dims d = 8j + 4g + i, their partners (rows +8) sit
-    // in lane + 32: swap the rounded projections across the lane halves
-    const int half = a.D >> 1, tph = half >> 3;
-    const int head = tile / tph, j8 = tile % tph;
-    float yv[4], yp[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-      yv[i] = Elem<T>::to_f32(Elem<T>::from_f32(acc[0][i] * f32_of(e_s0[i])));
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(yv[i]), __float_as_uint(yv[i]),
-                                                 false, false);
-      yp[i] = __uint_as_float(lane < 32 ? sw[1] : sw[0]);
-    }
-    if (!m_ok) return;
-    const int64_t p = pos;
-    const bool hi = g >= 2;                       // rows 8..15: second half of the pair
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int ii = 8 * j8 + 4 * (g & 1) + i;    // rotation index, 0 <= ii < half
-      const int d = ii + (hi ? half : 0);
-      T out;
-      if (mat == 2) {
-        out = Elem<T>::from_f32(yv[i]);           // v: appended unrotated (bitwise)
-      } else {
-        const float cs = f32_of(e_cos[i]), sn = f32_of(e_sin[i]);
-        const float x1 = hi ? yp[i] : yv[i], x2 = hi ? yv[i] : yp[i];
-        T y1, y2;
-        {
-#pragma clang fp contract(off)
-          const float x1c = x1 * cs, x2s = x2 * sn, x2c = x2 * cs, x1s = x1 * sn;
-          y1 = Elem<T>::from_f32(x1c - x2s);
-          y2 = Elem<T>::from_f32(x2c + x1s);
-        }
-        out = hi ? y2 : y1;
-      }
-      if (mat == 0) {
-        reinterpret_cast<T*>(a.y)[((int64_t)m * a.Hq + head) * a.D + d] = out;
-      } else if (p >= 0 && p < a.capacity) {
-        T* c = reinterpret_cast<T*>(mat == 1 ? a.ck : a.cv);
-        c[(int64_t)m * a.c_sb + (int64_t)head * a.c_sh + p * a.c_st + d] = out;
-      }
-    }
-  } else {
-    if (!m_ok) return;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int rr = 4 * g + i;
-      const int n = tile * RPB + rr;
-      if (rr >= RPB || n >= a.N) continue;
-      float v = Elem<T>::to_f32(Elem<T>::from_f32(acc[0][i] * f32_of(e_s0[i])));
-      if constexpr (EPI == kEpiResidual) {
-        v = Elem<T>::to_f32(Elem<T>::from_f32(f32_of(e_res[i]) + v));
-      } else if constexpr (EPI == kEpiSwiglu) {
-        const float b = Elem<T>::to_f32(Elem<T>::from_f32(acc[1][i] * f32_of(e_s1[i])));
-        const float sa = Elem<T>::to_f32(Elem<T>::from_f32(silu_f32(v)));
-        v = sa * b;
-      }
-      reinterpret_cast<T*>(a.y)[(int64_t)m * a.y_sm + n] = Elem<T>::from_f32(v);
-    }
   }
 }
 
@@ -691,61 +405,302 @@ __global__ __launch_bounds__(64 * NW) void dgemv_kernel(LayerGemvArgs a) {
   }
 }
 
+// A lane's 16 bytes of weight row r for the first / second 64 k of a 128-k pair
+// of chunks, from the two loads of the pair: a holds rows 0..7 and b rows 8..15,
+// lanes r < 8 the first 64 k and lanes r >= 8 the second (each load reads whole
+// 128-byte lines of 8 rows).  One DPP row rotate by 8 per word.
+__device__ inline u32x4 rows_lo(const u32x4& a, const u32x4& b) {
+  u32x4 o;
+#pragma unroll
+  for (int i = 0; i < 4; ++i)   // lanes 8..15 take b of lane r - 8
+    o[i] = (uint32_t)__builtin_amdgcn_update_dpp((int)a[i], (int)b[i], 0x128, 0xF, 0xC, false);
+  return o;
+}
+__device__ inline u32x4 rows_hi(const u32x4& a, const u32x4& b) {
+  u32x4 o;
+#pragma unroll
+  for (int i = 0; i < 4; ++i)   // lanes 0..7 take a of lane r + 8
+    o[i] = (uint32_t)__builtin_amdgcn_update_dpp((int)b[i], (int)a[i], 0x128, 0xF, 0x3, false);
+  return o;
+}
+
+// ---------------------------------------------------------------------------
+// GEMV for 9..16 token rows.
+//
+// With more than 8 token rows the B operand of v_mfma_f32_16x16x32 is full, so
+// an A tile is 16 weight rows: lane (r, g) feeds 16 consecutive k of weight row
+// r and of token row r for each 64-k chunk (two MFMAs); the weights of a pair of
+// chunks are loaded as whole 128-byte lines of 8 rows (rows_lo / rows_hi).  A block has NW waves
+// that split K (SC consecutive chunks each, K = 64 * NW * SC) and owns TPB
+// 16-row tiles of each of its NMAT matrices: every wave reads its slice of x
+// once, straight into the B registers, for all of the block's tiles.  x is what
+// bounds these calls, not the weights: a block with one tile reads twice as
+// many bytes of x (16 rows of 2 bytes) as of int8 weights, so tiles are grouped
+// until the grid is about one block per CU, and all weight loads are issued
+// before the first wait.  With the RMSNorm prologue each wave normalises its
+// own x slice in registers.  The waves' sums meet in LDS.
+// MI355X, M = 16, per call in a graph over rotating weights, against one tile per
+// block with 64-byte pieces of 16 rows per load (8-row tiles for N < 3840):
+// [3072, 3072] 10.8 -> 6.3 us, [3072, 8192] 25.2 -> 14.6, SwiGLU 2 x [8192, 3072]
+// 17.9 -> 13.0 (3.9 TB/s), SwiGLU 2 x [8192, 2048] 11.7 -> 9.5, [3072, 2048] 6.9 -> 4.9.
+// What is left is x: the same calls with all 16 rows at one address take 1 to 3 us less.
+template <typename T, int NW, int SC, bool NORM, int EPI, int TPB>
+__global__ __launch_bounds__(64 * NW) void rows_gemv_kernel(LayerGemvArgs a) {
+  using MM = LMfma<T>;
+  typedef typename MM::v8 v8;
+  constexpr int NMAT = EPI == kEpiSwiglu ? 2 : 1;
+  constexpr int NT = NMAT * TPB;                       // 16-row A tiles per block
+  constexpr int NOUT = 256 * TPB;                      // outputs of a block
+  constexpr int NO = (NOUT + 64 * NW - 1) / (64 * NW); // outputs of a thread
+  __shared__ __align__(16) float red[NW][NT][16][16];  // [wave][tile][token][row]
+  __shared__ float ssq[NORM ? NW : 1][16];             // per-wave sums of squares
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r = lane & 15, g = lane >> 4;   // A: tile row / B: token row; k group
+  // K slice of this wave, rotated by block (concurrent blocks read different x lines)
+  const int kw = ((w + (int)blockIdx.x) % NW) * SC * 64;
+  const int kx = kw + 16 * g;
+
+  // ---- the block's tiles.  QKV: tiles of wq, then wk, then wv in one list,
+  //      each 8 rotation pairs of a head (rows 0..7 dims d, rows 8..15 d + D/2)
+  const int half = a.D >> 1, tph = EPI == kEpiQkvRope ? half >> 3 : 1;
+  const int n_tiles = EPI == kEpiQkvRope ? a.n_tiles0 + 2 * a.n_tiles1 : (a.N + 15) >> 4;
+  auto mat_of = [&](int tile) -> int {
+    if constexpr (EPI != kEpiQkvRope) return 0;
+    return tile < a.n_tiles0 ? 0 : tile < a.n_tiles0 + a.n_tiles1 ? 1 : 2;
+  };
+  auto w_row = [&](int tile, int mat, int row) -> int {
+    if constexpr (EPI == kEpiQkvRope) {
+      const int tim = mat == 0 ? tile : tile - a.n_tiles0 - (mat == 2 ? a.n_tiles1 : 0);
+      const int head = tim / tph, j = tim - head * tph;
+      return head * a.D + 8 * j + (row & 7) + ((row >> 3) ? half : 0);
+    } else {
+      return tile * 16 + row;
+    }
+  };
+  // weight rows through buffer resources (host-checked: each matrix spans < 2^31
+  // bytes); rows past N and tiles past the list load zeros without an access
+  buf_rsrc wr[NT];
+  uint32_t woff[NT][2];
+#pragma unroll
+  for (int t = 0; t < NT; ++t) {
+    const int tile = blockIdx.x * TPB + t % TPB, mat = mat_of(tile);
+    const bool b3 = t >= TPB;                          // SwiGLU's second matrix
+    const int8_t* wm = b3 || mat == 1 ? a.w1 : mat == 2 ? a.w2 : a.w0;
+    const int64_t sn = b3 || mat == 1 ? a.w_sn1 : mat == 2 ? a.w_sn2 : a.w_sn0;
+    const int rows = EPI == kEpiQkvRope && mat != 0 ? a.Hkv * a.D : a.N;
+    wr[t] = make_rsrc(wm, (uint32_t)((int64_t)(rows - 1) * sn + a.K));
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int n = w_row(tile, mat, 8 * h + (r & 7));
+      woff[t][h] = (tile < n_tiles && n < rows ? (uint32_t)((int64_t)n * sn) : kOobOffset) +
+                   (r >> 3) * 64 + 16 * g;
+    }
+  }
+
+  // ---- x (rows >= M read zeros), norm weights, then every weight load
+  const buf_rsrc xrs =
+      make_rsrc(a.x, (uint32_t)(((int64_t)(a.M - 1) * a.x_sm + a.K) * sizeof(T)));
+  const uint32_t xo = r < a.M ? (uint32_t)((int64_t)r * a.x_sm * sizeof(T)) : kOobOffset;
+  u32x4 xr[SC][2];
+#pragma unroll
+  for (int s = 0; s < SC; ++s) {
+    xr[s][0] = buf_load16(xrs, xo + (uint32_t)((kx + s * 64) * sizeof(T)));
+    xr[s][1] = buf_load16(xrs, xo + (uint32_t)((kx + s * 64 + 8) * sizeof(T)));
+  }
+  u32x4 nr[NORM ? SC : 1][2];
+  if constexpr (NORM) {
+#pragma unroll
+    for (int s = 0; s < SC; ++s) {
+      const T* np = reinterpret_cast<const T*>(a.norm_w) + kx + s * 64;
+      nr[s][0] = load16(np);
+      nr[s][1] = load16(np + 8);
+    }
+  }
+  u32x4 wq[NT][SC];
+#pragma unroll
+  for (int s = 0; s < SC; ++s)
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+      wq[t][s] = buf_load16_nt(wr[t], woff[t][s & 1] + (uint32_t)(kw + (s >> 1) * 128));
+
+  // ---- epilogue operands behind the weights, from clamped indices
+  T e_s0[NO], e_s1[NO], e_res[NO], e_cos[NO], e_sin[NO];
+  const int64_t pos = EPI == kEpiQkvRope ? *a.pos : 0;
+#pragma unroll
+  for (int o = 0; o < NO; ++o) {
+    const int i = min(tid + o * 64 * NW, NOUT - 1);
+    const int tile = min((int)blockIdx.x * TPB + (i >> 8), n_tiles - 1);
+    const int row = i & 15, m = min((i >> 4) & 15, a.M - 1);
+    if constexpr (EPI == kEpiQkvRope) {
+      const int mat = mat_of(tile), n = w_row(tile, mat, row);
+      const T* sc = reinterpret_cast<const T*>(mat == 0 ? a.s0 : mat == 1 ? a.s1 : a.s2);
+      e_s0[o] = sc[n];
+      e_s1[o] = sc[w_row(tile, mat, row ^ 8)];
+      const int64_t crow = min(max(pos - a.rope_row0, (int64_t)0), a.rope_rows - 1);
+      const int ii = (n % a.D) % half;
+      e_cos[o] = reinterpret_cast<const T*>(a.cos)[crow * a.c_ss + ii];
+      e_sin[o] = reinterpret_cast<const T*>(a.sin)[crow * a.c_ss + ii];
+    } else {
+      const int n = min(tile * 16 + row, a.N - 1);
+      e_s0[o] = reinterpret_cast<const T*>(a.s0)[n];
+      if constexpr (EPI == kEpiSwiglu) e_s1[o] = reinterpret_cast<const T*>(a.s1)[n];
+      if constexpr (EPI == kEpiResidual)
+        e_res[o] = reinterpret_cast<const T*>(a.res)[(int64_t)m * a.res_sm + n];
+    }
+  }
+  __builtin_amdgcn_sched_barrier(0);
+
+  // ---- RMSNorm: a token row's sum of squares over this lane's k, the k groups
+  //      and the waves; then x * rstd * w rounded once to T, in place
+  if constexpr (NORM) {
+    float ss = 0.f;
+#pragma unroll
+    for (int s = 0; s < SC; ++s)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        float v[8];
+        Chunk<T>::unpack(xr[s][h], v);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) ss = fmaf(v[e], v[e], ss);
+      }
+    ss += dl_lane_xor<16>(ss, lane);
+    ss += dl_lane_xor<32>(ss, lane);
+    if (lane < 16) ssq[w][lane] = ss;
+    __syncthreads();
+    float tot = 0.f;
+#pragma unroll
+    for (int ww = 0; ww < NW; ++ww) tot += ssq[ww][r];
+    const float rstd = 1.0f / sqrtf(tot / (float)a.K + a.eps);
+#pragma unroll
+    for (int s = 0; s < SC; ++s)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        float v[8], wn[8];
+        Chunk<T>::unpack(xr[s][h], v);
+        Chunk<T>::unpack(nr[s][h], wn);
+        typedef T t8 __attribute__((ext_vector_type(8)));
+        t8 o;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) o[e] = Elem<T>::from_f32(v[e] * rstd * wn[e]);
+        xr[s][h] = __builtin_bit_cast(u32x4, o);
+      }
+  }
+
+  // ---- MFMAs over the wave's chunks; acc[i] = C[tile row 4g + i][token r]
+  f32x4 acc[NT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int s = 0; s < SC; ++s) {
+    const v8 xb0 = __builtin_bit_cast(v8, xr[s][0]);
+    const v8 xb1 = __builtin_bit_cast(v8, xr[s][1]);
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      const u32x4 wv = s & 1 ? rows_hi(wq[t][s - 1], wq[t][s]) : rows_lo(wq[t][s], wq[t][s + 1]);
+      acc[t] = MM::mma(i8x8_cvt<T, v8>(wv.x, wv.y), xb0, acc[t]);
+      acc[t] = MM::mma(i8x8_cvt<T, v8>(wv.z, wv.w), xb1, acc[t]);
+    }
+  }
+#pragma unroll
+  for (int t = 0; t < NT; ++t) *reinterpret_cast<f32x4*>(&red[w][t][r][4 * g]) = acc[t];
+  __syncthreads();
+
+  auto wsum = [&](int t, int m, int row) -> float {
+    float v = 0.f;
+#pragma unroll
+    for (int ww = 0; ww < NW; ++ww) v += red[ww][t][m][row];
+    return v;
+  };
+  auto f32_of = [](T v) { return Elem<T>::to_f32(v); };
+  auto rnd = [](float v) { return Elem<T>::to_f32(Elem<T>::from_f32(v)); };
+#pragma unroll
+  for (int o = 0; o < NO; ++o) {
+    const int i = tid + o * 64 * NW;
+    const int t = i >> 8, tile = blockIdx.x * TPB + t, row = i & 15, m = (i >> 4) & 15;
+    if (i >= NOUT || tile >= n_tiles || m >= a.M) continue;
+    if constexpr (EPI == kEpiQkvRope) {
+      const int mat = mat_of(tile), n = w_row(tile, mat, row);
+      const float yv = rnd(wsum(t, m, row) * f32_of(e_s0[o]));
+      const float yp = rnd(wsum(t, m, row ^ 8) * f32_of(e_s1[o]));
+      const int head = n / a.D, d = n - head * a.D;
+      T out;
+      if (mat == 2) {
+        out = Elem<T>::from_f32(yv);                  // v: appended unrotated (bitwise)
+      } else {
+        const bool hi = row >= 8;
+        T y1, y2;
+        rope_rotate<T, T>(hi ? yp : yv, hi ? yv : yp, e_cos[o], e_sin[o], y1, y2);
+        out = hi ? y2 : y1;
+      }
+      if (mat == 0) {
+        reinterpret_cast<T*>(a.y)[((int64_t)m * a.Hq + head) * a.D + d] = out;
+      } else if (pos >= 0 && pos < a.capacity) {
+        T* c = reinterpret_cast<T*>(mat == 1 ? a.ck : a.cv);
+        c[(int64_t)m * a.c_sb + (int64_t)head * a.c_sh + pos * a.c_st + d] = out;
+      }
+    } else {
+      const int n = tile * 16 + row;
+      if (n >= a.N) continue;
+      float v = rnd(wsum(t, m, row) * f32_of(e_s0[o]));
+      if constexpr (EPI == kEpiResidual) {
+        v = f32_of(e_res[o]) + v;
+      } else if constexpr (EPI == kEpiSwiglu) {
+        const float b = rnd(wsum(TPB + t, m, row) * f32_of(e_s1[o]));
+        v = rnd(silu_f32(v)) * b;
+      }
+      reinterpret_cast<T*>(a.y)[(int64_t)m * a.y_sm + n] = Elem<T>::from_f32(v);
+    }
+  }
+}
+
 namespace {
 
-template <typename T, int NW, bool NORM, int EPI, int RPB, int MR>
-hipError_t launch_layer_gemv(const LayerGemvArgs& a, int n_blocks, hipStream_t st) {
-  size_t smem = (size_t)(NW - 1) * (EPI == kEpiSwiglu ? 2 : 1) * 64 * sizeof(f32x4);
-  if (NORM) smem += (size_t)a.M * a.K * sizeof(T) + (size_t)NW * MR * sizeof(float);
-  hipLaunchKernelGGL((layer_gemv_kernel<T, NW, NORM, EPI, RPB, MR>), dim3((unsigned)n_blocks),
-                     dim3(64 * NW), smem, st, a);
+template <typename T, bool NORM, int EPI, int TPB, int NW, int SC>
+hipError_t launch_rows(const LayerGemvArgs& a, int n_tiles, hipStream_t st) {
+  hipLaunchKernelGGL((rows_gemv_kernel<T, NW, SC, NORM, EPI, TPB>),
+                     dim3((unsigned)((n_tiles + TPB - 1) / TPB)), dim3(64 * NW), 0, st, a);
   return hipGetLastError();
 }
 
-// Waves per block: K = 512 * NW (each wave owns 8 chunks of 64 k).  The
-// RMSNorm prologue keeps MR (8 or 16 >= M) rows of one column chunk per thread.
-template <typename T, bool NORM, int EPI, int RPB>
-hipError_t dispatch_nw(const LayerGemvArgs& a, int n_blocks, hipStream_t st) {
-  constexpr int MR = 8;
-  if (NORM && a.M > MR) {
-    switch (a.K) {
-      case 512: return launch_layer_gemv<T, 1, NORM, EPI, RPB, 16>(a, n_blocks, st);
-      case 1024: return launch_layer_gemv<T, 2, NORM, EPI, RPB, 16>(a, n_blocks, st);
-      case 2048: return launch_layer_gemv<T, 4, NORM, EPI, RPB, 16>(a, n_blocks, st);
-      default: return hipErrorInvalidValue;  // host checks exclude the rest
-    }
-  }
+// Waves and chunks per wave from K = 64 * NW * SC, at most 16 waves.
+template <typename T, bool NORM, int EPI, int TPB>
+hipError_t dispatch_rows_k(const LayerGemvArgs& a, int n_tiles, hipStream_t st) {
   switch (a.K) {
-    case 512: return launch_layer_gemv<T, 1, NORM, EPI, RPB, MR>(a, n_blocks, st);
-    case 1024: return launch_layer_gemv<T, 2, NORM, EPI, RPB, MR>(a, n_blocks, st);
-    case 1536: return launch_layer_gemv<T, 3, NORM, EPI, RPB, MR>(a, n_blocks, st);
-    case 2048: return launch_layer_gemv<T, 4, NORM, EPI, RPB, MR>(a, n_blocks, st);
-    case 3072: return launch_layer_gemv<T, 6, NORM, EPI, RPB, MR>(a, n_blocks, st);
-    case 4096: return launch_layer_gemv<T, 8, NORM, EPI, RPB, MR>(a, n_blocks, st);
+    case 512: return launch_rows<T, NORM, EPI, TPB, 4, 2>(a, n_tiles, st);
+    case 1024: return launch_rows<T, NORM, EPI, TPB, 8, 2>(a, n_tiles, st);
+    case 1536: return launch_rows<T, NORM, EPI, TPB, 12, 2>(a, n_tiles, st);
+    case 2048: return launch_rows<T, NORM, EPI, TPB, 8, 4>(a, n_tiles, st);
     default: break;
   }
-  if constexpr (EPI != kEpiSwiglu) {  // two weight streams: K <= 4096 (host-checked)
+  if constexpr (!NORM) {   // the prologue serves K <= 2048 (host-checked)
     switch (a.K) {
-      case 6144: return launch_layer_gemv<T, 12, NORM, EPI, RPB, MR>(a, n_blocks, st);
-      case 8192: return launch_layer_gemv<T, 16, NORM, EPI, RPB, MR>(a, n_blocks, st);
+      case 3072: return launch_rows<T, NORM, EPI, TPB, 12, 4>(a, n_tiles, st);
+      // 16 waves have 128 registers each: one tile of two matrices at a time
+      case 4096: return launch_rows<T, NORM, EPI, EPI == kEpiSwiglu ? 1 : TPB, 16, 4>(a, n_tiles, st);
       default: break;
+    }
+    if constexpr (EPI != kEpiSwiglu) {  // two weight streams: K <= 4096 (host-checked)
+      switch (a.K) {
+        case 6144: return launch_rows<T, NORM, EPI, 1, 16, 6>(a, n_tiles, st);
+        case 8192: return launch_rows<T, NORM, EPI, 1, 16, 8>(a, n_tiles, st);
+        default: break;
+      }
     }
   }
   return hipErrorInvalidValue;
 }
 
-template <typename T, int EPI, int RPB>
-hipError_t dispatch_norm(const LayerGemvArgs& a, int n_blocks, hipStream_t st) {
-  return a.norm_w != nullptr ? dispatch_nw<T, true, EPI, RPB>(a, n_blocks, st)
-                             : dispatch_nw<T, false, EPI, RPB>(a, n_blocks, st);
-}
-
-// Row tiles of 16 when that already makes a few hundred blocks, else of 8
-// (the A rows beyond 8 are zero) so that small-N projections use every CU.
+// 9..16 rows: two tiles per block when one per block is more than a block per CU.
 template <typename T, int EPI>
-hipError_t dispatch_tile(const LayerGemvArgs& a, hipStream_t st) {
-  if (a.N / 16 >= 240) return dispatch_norm<T, EPI, 16>(a, (a.N + 15) / 16, st);
-  return dispatch_norm<T, EPI, 8>(a, (a.N + 7) / 8, st);
+hipError_t dispatch_rows(const LayerGemvArgs& a, int n_tiles, hipStream_t st) {
+  const bool two = n_tiles > device_cu_count();
+  if (a.norm_w != nullptr)
+    return two ? dispatch_rows_k<T, true, EPI, 2>(a, n_tiles, st)
+               : dispatch_rows_k<T, true, EPI, 1>(a, n_tiles, st);
+  return two ? dispatch_rows_k<T, false, EPI, 2>(a, n_tiles, st)
+             : dispatch_rows_k<T, false, EPI, 1>(a, n_tiles, st);
 }
 
 // Diagonal-packed kernel (M <= 8): waves and superchunks per wave from K =
@@ -792,15 +747,15 @@ hipError_t dispatch_dg(const LayerGemvArgs& a, int n_blocks, hipStream_t st) {
 }
 
 // Store / residual / SwiGLU projections: the diagonal-packed kernel for M <= 8
-// (one 8-row tile per block; SwiGLU two tiles of each matrix), else the
-// 16-column kernel above.
+// (one 8-row tile per block; SwiGLU two tiles of each matrix), else the 16-row
+// kernel.
 template <typename T, int EPI>
 hipError_t dispatch_linear(const LayerGemvArgs& a, hipStream_t st) {
   if (a.M <= 8) {
     constexpr int TPB = EPI == kEpiSwiglu ? 2 : 1;
     return dispatch_dg<T, EPI, TPB>(a, (a.N + 8 * TPB - 1) / (8 * TPB), st);
   }
-  return dispatch_tile<T, EPI>(a, st);
+  return dispatch_rows<T, EPI>(a, (a.N + 15) / 16, st);
 }
 
 bool k_supported(int64_t K) {
@@ -979,9 +934,9 @@ extern "C" int32_t mi_w8a16_qkv_rope_append(
     const int tph = (int)(head_dim / 16);   // tiles (8 rotation pairs each) per head
     a.n_tiles0 = (int32_t)(n_heads * tph);
     a.n_tiles1 = (int32_t)(n_kv_heads * tph);
-    const int n_blocks = a.n_tiles0 + 2 * a.n_tiles1;
-    e = dtype == MI_DTYPE_BF16 ? dispatch_norm<bf16_t, kEpiQkvRope, 16>(a, n_blocks, s)
-                               : dispatch_norm<f16_t, kEpiQkvRope, 16>(a, n_blocks, s);
+    const int n_tiles = a.n_tiles0 + 2 * a.n_tiles1;
+    e = dtype == MI_DTYPE_BF16 ? dispatch_rows<bf16_t, kEpiQkvRope>(a, n_tiles, s)
+                               : dispatch_rows<f16_t, kEpiQkvRope>(a, n_tiles, s);
   }
   if (e != hipSuccess) {
     set_last_error("%s: launch failed: %s", what, hipGetErrorString(e));

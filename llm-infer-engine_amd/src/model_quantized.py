@@ -31,11 +31,18 @@ class QuantizedFeedForward(FeedForward):
         super().__init__(dim, hidden_dim, linear)
 
     def forward(self, x, *, residual=None):
-        """Prefill-sized inputs: silu(w1(x)) * w3(x) in one GEMM launch (the
-        same rounding points, neither projection written out) when its tiles
-        fill the GPU; otherwise the op chain of src/model.py:23."""
+        """silu(w1(x)) * w3(x) in one launch (the same rounding points, neither
+        projection written out): up to 16 rows in the decode projection
+        kernels, prefill-sized inputs in the GEMM when its tiles fill the GPU;
+        otherwise the op chain of src/model.py:23."""
         x2 = x.reshape(-1, x.shape[-1])
         w1, w3 = self.w1, self.w3
+        if _rows_fusable(x2, w1, swiglu=True) and _rows_fusable(x2, w3):
+            torch.cuda.nvtx.range_push("FFN")
+            h = decode_layer.linear_fused(x2, w1, lin_b=w3)
+            out = self.down(h.view(*x.shape[:-1], w1.out_features), residual)
+            torch.cuda.nvtx.range_pop()
+            return out
         if not quant_linear.swiglu_worth(x2.shape[0], x2.shape[1], w1.out_features, x.device):
             return super().forward(x, residual=residual)
         torch.cuda.nvtx.range_push("FFN")
@@ -48,10 +55,23 @@ class QuantizedFeedForward(FeedForward):
         return _project_residual(self.w2, h, residual)
 
 
+def _rows_fusable(x2, lin, *, swiglu=False) -> bool:
+    """Whether the decode projection kernels take rows x2 [M <= 16, K] through `lin`."""
+    return (1 <= x2.shape[0] <= 16
+            and decode_layer.supported(x2.shape[0], x2.shape[1], x2.dtype, lin, swiglu=swiglu)
+            and decode_layer.aligned(x2))
+
+
 def _project_residual(lin, h, residual):
-    """lin(h) + residual with the add in the GEMM epilogue at GEMM sizes (the
-    same roundings as the separate ops); otherwise the two ops."""
+    """lin(h) + residual with the add in the epilogue of the decode projection
+    (up to 16 rows) or of the GEMM (the same roundings as the separate ops);
+    otherwise the two ops."""
     h2 = h.reshape(-1, h.shape[-1])
+    if (residual is not None and residual.dtype == h.dtype
+            and residual.shape == (*h.shape[:-1], lin.out_features) and _rows_fusable(h2, lin)):
+        res2 = residual.reshape(-1, lin.out_features)
+        if res2.stride(1) == 1:
+            return decode_layer.linear_fused(h2, lin, residual=res2).view(residual.shape)
     if residual is None or not quant_linear.gemm_supported(h2.shape[0], h2.shape[1]):
         out = lin(h)
         return out if residual is None else residual + out
@@ -103,13 +123,21 @@ class QuantizedTransformerBlock(TransformerBlock):
             return False
         dt, sup = x.dtype, decode_layer.supported
         n_o = attn.n_heads * attn.head_dim
-        return (decode_layer.aligned(x.view(B, dim))
-                and sup(B, dim, dt, attn.wq, self.attention_norm.weight)
+        return (decode_layer.aligned(x.view(B, dim)) and sup(B, dim, dt, attn.wq)
                 and sup(B, dim, dt, attn.wk) and sup(B, dim, dt, attn.wv)
                 and sup(B, n_o, dt, attn.wo)
-                and sup(B, dim, dt, ff.w1, self.ffn_norm.weight, swiglu=True)
+                and sup(B, dim, dt, ff.w1, swiglu=True)
                 and sup(B, dim, dt, ff.w3)
                 and sup(B, ff.w1.out_features, dt, ff.w2))
+
+    @staticmethod
+    def _norm_in(x2, lin, norm, *, swiglu=False):
+        """(rows, norm weight) for a projection of the normalised rows: the
+        projection's own RMSNorm prologue where it takes these sizes, else the
+        rows normalised by a launch of their own and no prologue."""
+        if decode_layer.supported(x2.shape[0], x2.shape[1], x2.dtype, lin, norm.weight, swiglu=swiglu):
+            return x2, norm.weight
+        return norm(x2), None
 
     def forward(self, x, rope_cos, rope_sin, layer_idx=None, start_pos=0, kv_cache=None,
                 use_cuda_graph=False, scatter_positions=None, decode_attn_mask=None, **ext):
@@ -130,16 +158,16 @@ class QuantizedTransformerBlock(TransformerBlock):
         else:
             pos = torch.full((1,), int(start_pos), dtype=torch.int64, device=x.device)
             row0 = 0 if by_pos else int(start_pos)
-        q = decode_layer.qkv_rope_append(x2, attn, self.attention_norm.weight,
-                                         self.attention_norm.eps, rope_cos, rope_sin, row0, pos,
-                                         kv_cache, layer_idx)
+        h, nw = self._norm_in(x2, attn.wq, self.attention_norm)
+        q = decode_layer.qkv_rope_append(h, attn, nw, self.attention_norm.eps, rope_cos, rope_sin,
+                                         row0, pos, kv_cache, layer_idx)
         ck, cv = kv_cache.k[layer_idx, :B], kv_cache.v[layer_idx, :B]
         if positions is None:
             ck, cv = ck[:, :, :int(start_pos) + 1], cv[:, :, :int(start_pos) + 1]
         o = flash_decode(q, ck, cv, mask=decode_attn_mask, seq_lens=ext.get("seq_lens"))
         h = decode_layer.linear_fused(o.view(B, -1), attn.wo, residual=x2)
-        g = decode_layer.linear_fused(h, ff.w1, norm_weight=self.ffn_norm.weight,
-                                      eps=self.ffn_norm.eps, lin_b=ff.w3)
+        n, nw = self._norm_in(h, ff.w1, self.ffn_norm, swiglu=True)
+        g = decode_layer.linear_fused(n, ff.w1, norm_weight=nw, eps=self.ffn_norm.eps, lin_b=ff.w3)
         y = decode_layer.linear_fused(g, ff.w2, residual=h)
         return y.view(B, 1, dim)
 

@@ -129,6 +129,74 @@ def test_qkv_rope_append(dev, dtype, M, Hq, Hkv, D, by_position):
     _close(q, uq, 1e-2)
 
 
+@pytest.mark.parametrize("M", [9, 13, 16])
+@pytest.mark.parametrize("K,N", [(512, 16), (1536, 4112), (2048, 250), (3072, 4100), (4096, 4112),
+                                 (6144, 40), (8192, 4112)])
+def test_rows_gemv_widths_and_tile_edges(dev, M, K, N):
+    """9..16 rows: every wave split of K, one and two tiles per block (N past
+    16 x 256 rows), a last tile and a last pair that are not full; the sums run
+    over the same products as the unfused kernel in another order."""
+    from src import decode_layer
+    from src.quant_linear import w8a16_gemv_launch
+    dtype = torch.bfloat16
+    lin = _linear(dev, K, N, dtype, 51)
+    x, res = randn((M, K), 52, dtype, dev), randn((M, N), 53, dtype, dev)
+    y = decode_layer.linear_fused(x, lin)
+    un = w8a16_gemv_launch(x, lin.weight, lin.scales)
+    _close(y, oq.w8a16(x, lin.weight, lin.scales), 2e-2)
+    _close(y, un, 1e-2)
+    _close(decode_layer.linear_fused(x, lin, residual=res), res + un, 1e-2)
+    if K <= 4096:
+        lin3 = _linear(dev, K, N, dtype, 54)
+        g = decode_layer.linear_fused(x, lin, lin_b=lin3)
+        _close(g, torch.nn.functional.silu(un) * w8a16_gemv_launch(x, lin3.weight, lin3.scales), 1e-2)
+
+
+@pytest.mark.parametrize("M,dim,Hq,Hkv,D", [(16, 3072, 24, 8, 128), (9, 2048, 32, 8, 64),
+                                            (11, 1024, 3, 1, 48)])
+def test_block_of_9_to_16_rows_matches_op_chain(dev, M, dim, Hq, Hkv, D):
+    """The fused block at batches above 8 (RMSNorm as its own launch where the
+    prologue does not take the size) against its op-by-op form."""
+    from src.config import ModelArgs
+    from src.kv_cache import KVCache
+    from src.model_quantized import QuantizedTransformerBlock, build_random_quantized
+    if dim != Hq * D:      # heads that do not fill dim: not a model shape, keep the QKV kernel only
+        from src import decode_layer
+        from src.rope import DeviceRopeTable, apply_rotary
+        attn = _Attn(dev, dim, Hq, Hkv, D, torch.bfloat16)
+        cache = _Cache(dev, 1, M, Hkv, 32, D, torch.bfloat16)
+        t = DeviceRopeTable(orope.freqs_cis(D, 32, 500000.0), torch.bfloat16, dev)
+        x = randn((M, dim), 61, torch.bfloat16, dev)
+        pos = torch.full((1,), 5, dtype=torch.int64, device=dev)
+        q = decode_layer.qkv_rope_append(x, attn, None, 0.0, t.cos, t.sin, 0, pos, cache, 0)
+        rot = lambda l, h: apply_rotary(l(x).view(M, 1, h, D).transpose(1, 2), *t.rows(5, 1))  # noqa: E731
+        _close(q, rot(attn.wq, Hq), 1e-2)
+        _close(cache.k[0, :, :, 5], rot(attn.wk, Hkv)[:, :, 0], 1e-2)
+        _close(cache.v[0, :, :, 5], attn.wv(x).view(M, Hkv, D), 1e-2)
+        return
+    args = ModelArgs(dim=dim, n_layers=1, n_heads=Hq, n_kv_heads=Hkv, vocab_size=64, hidden_dim=4096,
+                     max_batch_size=M, max_seq_len=64, device=str(dev))
+    block = build_random_quantized(args, seed=3, device=str(dev)).layers[0]
+    kv = [KVCache(args, dtype=torch.bfloat16) for _ in range(2)]
+    kv[0].k.normal_(generator=torch.Generator(device=dev).manual_seed(1))
+    kv[0].v.normal_(generator=torch.Generator(device=dev).manual_seed(2))
+    kv[1].k.copy_(kv[0].k)
+    kv[1].v.copy_(kv[0].v)
+    x = randn((M, 1, dim), 62, torch.bfloat16, dev)
+    cos, sin = orope.cos_sin(orope.freqs_cis(D, 64, 500000.0)[40:41], torch.bfloat16)
+    ys = []
+    with torch.no_grad():
+        for c, fused in zip(kv, (True, False)):
+            QuantizedTransformerBlock.fused_decode = fused
+            try:
+                ys.append(block(x, cos.to(dev), sin.to(dev), layer_idx=0, start_pos=40, kv_cache=c))
+            finally:
+                QuantizedTransformerBlock.fused_decode = True
+    _close(ys[0], ys[1], 1e-2)
+    _close(kv[0].k, kv[1].k, 1e-2)
+    _close(kv[0].v, kv[1].v, 1e-2)
+
+
 def test_unsupported_shapes_are_rejected(dev):
     """K outside the built set, M > 16: the C side refuses (nothing launched)
     and the model-level predicate routes such calls to the op chain."""
