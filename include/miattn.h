@@ -409,6 +409,30 @@ int32_t mi_w8a16_gemm_multi(const void* x, int64_t m, int64_t k, int64_t x_sm,
                             int32_t dtype, int32_t sdtype, void* stream);
 
 /*
+ * GEMMs of a few rows to a few hundred (a chat prompt, a large decode batch),
+ * x [m, k] times 1..3 int8 matrices [n_i, k] in one launch (arrays as in
+ * mi_w8a16_gemm_multi).  Epilogues, with the roundings of the separate ops:
+ *   0  y_i = dtype((x w_i^T) * s_i)
+ *   1  y_0 = dtype(res + dtype((x w_0^T) * s_0))               (one matrix)
+ *   2  y_0 = dtype(dtype(silu(dtype((x w_0^T) s_0))) * dtype((x w_1^T) s_1))
+ * m <= 65535; k a multiple of 256 (m <= 64) or of 128.  One matrix may split K:
+ * mi_w8a16_small_gemm_splits(m, n, k) > 1 asks for a workspace of splits * m * n
+ * fp32 (a second launch adds the splits in order); a matrix that splits has no
+ * fused form (epilogue 2, or n_mats > 1).  Up to 64 rows a matrix gives the same
+ * bits alone and fused.  Other requirements as mi_w8a16_gemm.  Replaces w8a16_gemm_kernel +
+ * w8a16_gemm_launch at these sizes  src/quant_linear.py:123-188, :191-247.
+ */
+int64_t mi_w8a16_small_gemm_splits(int64_t m, int64_t n, int64_t k);
+int32_t mi_w8a16_small_gemm(const void* x, int64_t m, int64_t k, int64_t x_sm,
+                            int32_t n_mats, const int8_t* const* w,
+                            const void* const* scales, void* const* y,
+                            const int64_t* n, const int64_t* w_sn,
+                            const int64_t* s_sn, const int64_t* y_sm,
+                            int32_t epilogue, const void* res, int64_t res_sm,
+                            float* part, int64_t part_elems, int32_t dtype,
+                            int32_t sdtype, void* stream);
+
+/*
  * Fused decode-step projection (1 <= m <= 16 rows; k one of 512, 1024, 1536,
  * 2048, 3072, 4096, 6144, 8192):
  *   a   = rmsnorm(x, norm_w, eps) if norm_w != NULL else x   (rounded to dtype)

@@ -36,6 +36,8 @@
 //  * Tiles are ordered so that concurrently resident workgroups of one XCD
 //    (blocks are dealt to the 8 XCDs round-robin) cover a patch of 8 m-tiles
 //    and share their operand rows in that XCD's L2.
+#include <type_traits>
+
 #include "common.hpp"
 
 namespace mi {
@@ -553,6 +555,347 @@ __global__ __launch_bounds__(256) void w8a16_splitk_reduce_kernel(GemmArgs a, in
   }
 }
 
+// ---------------------------------------------------------------------------
+// Small-M GEMM: 17 rows up to a few hundred (a chat prompt, a large decode batch).
+//
+// Here the weights (and the re-reads of x) decide: a 128 x 256 tile grid leaves
+// CUs idle, and gemm_tile_body's one stage of prefetch exposes a memory round
+// trip per 64 k when a CU has one workgroup.  So:
+//  * 8 waves per workgroup, NG = 8 / KG of them side by side in n (32 columns
+//    each) and KG behind each other in k (64 k of every stage), all on the same
+//    BM = 32 MB rows; the tile is 32 MB x 32 NG and its k groups meet in LDS at
+//    the end, in k-group order.
+//  * x and the int8 weights both come by LDS DMA into a ring of S stages of
+//    64 KG k (96 to 144 KB, one workgroup per CU), S - 1 of them in flight; the
+//    wait counts this wave's own copies (vmcnt), one barrier per stage publishes
+//    them and frees the slot that the next copy overwrites.
+//  * the two operands use the widening of the large GEMM; their 16-byte chunks are
+//    XOR-swizzled by the row so that an LDS read of 8 rows covers all banks.
+//  * a stage's operands are read from LDS one step ahead of their MFMAs.
+// What bounds it: per 128 k a CU spends about 0.4 us (widening, 24 VALU ops per 16 k
+// of 32 columns, and the barrier) plus 0.17 us per 32-row block (its MFMAs and LDS
+// reads).  MI355X, per call in a graph over rotating weights, against split K and
+// separate silu and product launches: 300 rows SwiGLU 2 x [8192, 2048] 73.3 -> 30.7 us
+// (655 TFLOP/s), [2048, 8192] + residual 31.9 -> 25.6, [2048, 2048] 21.4 -> 10.6; 48
+// rows SwiGLU 2 x [8192, 3072] 44.7 -> 16.3 (3.1 TB/s), [3072, 8192] 27.7 -> 15.1.
+constexpr int kMidMats = 3;
+struct MidMat {
+  const unsigned char* w;   // [N, K] int8, rows w_sn bytes apart
+  const void* scales;       // [N], element stride s_sn
+  void* y;                  // [M, N] (SwiGLU: of matrix 0 only)
+  int64_t w_sn, s_sn, y_sm;
+  int32_t N, col0;          // columns; first tile column of the matrix in the grid
+  int32_t y_vec;            // rows of y take 8-byte stores of 4 columns
+};
+struct MidArgs {
+  MidMat mat[kMidMats];
+  const unsigned char* x;   // [M, K], rows x_sm elements apart
+  const void* res;          // residual [M, N], rows res_sm elements apart, or null
+  float* part;              // split-K sums [split][M][N] or null
+  int64_t x_sm, res_sm;
+  int32_t M, K, n_mats, tiles_m, tiles_n, split_stages, res_vec, part_vec;
+};
+enum : int { kMidStore = 0, kMidPartial = 1, kMidSwiglu = 2 };
+
+template <int MB, int KG> struct MidShape {
+  // k of a k group in a stage: 32 where 64 would leave two stages in the ring and
+  // no registers for the operands read ahead
+  static constexpr int kKP = MB > 3 ? 32 : 64;
+  static constexpr int kNG = 8 / KG, kBM = 32 * MB, kBN = 32 * kNG, kBK = kKP * KG;
+  static constexpr int kXBytes = kBM * kBK * 2, kWBytes = kBN * kBK;   // per stage
+  static constexpr int kStage = kXBytes + kWBytes;
+  static constexpr int kS = 147456 / kStage > 8 ? 8 : 147456 / kStage;
+  // 1 KB copies per stage; of x a wave makes kXDma, or one less (waves 4..7 where
+  // MB is odd and the x copies do not divide by 8)
+  static constexpr int kXAll = kXBytes / 1024, kXDma = (kXAll + 7) / 8, kWDma = kWBytes / 1024 / 8;
+  static constexpr bool kXEven = kXAll % 8 == 0;
+  static constexpr size_t kLds = (size_t)kS * kStage + kBN * sizeof(float);   // + column scales
+  static_assert(kS >= 2, "ring of two stages at least");
+};
+
+template <int N>
+__device__ __forceinline__ void vm_wait() {
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+
+template <typename T, typename ST, int MB, int KG, int EPI>
+__global__ __launch_bounds__(512) void w8a16_mid_kernel(MidArgs a) {
+  using OP = GemmOps<T>;
+  using SH = MidShape<MB, KG>;
+  typedef typename OP::v8 v8;
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  const int lane = threadIdx.x & 63, r = lane & 31, h = lane >> 5;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int ng = wv % SH::kNG, kg = wv / SH::kNG;
+
+  // ---- tile: ids dealt round-robin to the 8 XCDs become consecutive per XCD,
+  //      m fastest, so that an XCD's tiles share weight rows in its L2
+  const int G = a.tiles_m * a.tiles_n;
+  const int split = EPI == kMidPartial ? (int)blockIdx.x / G : 0;
+  int b = (int)blockIdx.x - split * G;
+  {
+    const int xcd = b & 7, q = G >> 3, rem = G & 7;
+    b = xcd * q + min(xcd, rem) + (b >> 3);
+  }
+  const int tm = b % a.tiles_m, tn = b / a.tiles_m;
+  int mi = 0;
+  if constexpr (EPI == kMidStore) {
+#pragma unroll
+    for (int j = 1; j < kMidMats; ++j)
+      if (j < a.n_mats && tn >= a.mat[j].col0) mi = j;
+  }
+  const MidMat& mt = a.mat[mi];
+  constexpr int kCols = EPI == kMidSwiglu ? SH::kBN / 2 : SH::kBN;   // output columns
+  const int m0 = tm * SH::kBM, n0 = (tn - (EPI == kMidStore ? mt.col0 : 0)) * kCols;
+
+  // ---- copies of this wave: 1 KB of consecutive LDS each, lane t the 16 bytes
+  //      at 16 t; the swizzle chooses which chunk of the row that is.  Rows past
+  //      M or N are clamped and never stored.
+  constexpr int XC = SH::kBK / 8, WC = SH::kBK / 16;   // 16-byte chunks of a row
+  // chunk swizzle of a row: 8 consecutive rows' equal chunks fall in 8 different
+  // 16-byte columns of the 128 bytes that LDS serves at once
+  auto swz = [](int row, int chunks) { return chunks >= 8 ? row & 7 : (row >> 1) & 3; };
+  uint32_t x_off[SH::kXDma], w_off[SH::kWDma];
+  const unsigned char* w_base[SH::kWDma];
+#pragma unroll
+  for (int i = 0; i < SH::kXDma; ++i) {
+    const int row = (8 * i + wv) * (64 / XC) + lane / XC;
+    const int c = (lane % XC) ^ swz(row, XC);
+    x_off[i] = (uint32_t)((int64_t)(min(m0 + row, a.M - 1) - m0) * a.x_sm * 2 + c * 16);
+  }
+#pragma unroll
+  for (int i = 0; i < SH::kWDma; ++i) {
+    const int row0 = (SH::kWDma * wv + i) * (64 / WC);       // wave-uniform first row
+    const int row = row0 + lane / WC;
+    const int c = (lane % WC) ^ swz(row, WC);
+    if constexpr (EPI == kMidSwiglu) {
+      // 32 rows of a wave: 16 of w1, then the same 16 output columns' rows of w3
+      const MidMat& ms = a.mat[(row0 >> 4) & 1];
+      const int n = min(n0 + 16 * (row >> 5) + (row & 15), mt.N - 1) - n0;
+      w_base[i] = ms.w + (int64_t)n0 * ms.w_sn;
+      w_off[i] = (uint32_t)((int64_t)n * ms.w_sn + c * 16);
+    } else {
+      w_base[i] = mt.w + (int64_t)n0 * mt.w_sn;
+      w_off[i] = (uint32_t)((int64_t)(min(n0 + row, mt.N - 1) - n0) * mt.w_sn + c * 16);
+    }
+  }
+  const unsigned char* x_base = a.x + (int64_t)m0 * a.x_sm * 2;
+  const uint32_t lds0 = lds_addr(smem_raw);
+  const int nk_all = a.K / SH::kBK;
+  const int s0 = EPI == kMidPartial ? split * a.split_stages : 0;
+  const int nk = EPI == kMidPartial ? min(s0 + a.split_stages, nk_all) : nk_all;
+  auto issue = [&](int s, int slot) {
+    const uint32_t l = lds0 + (uint32_t)slot * SH::kStage;
+#pragma unroll
+    for (int i = 0; i < SH::kWDma; ++i)
+      lds_dma16(w_base[i] + (int64_t)s * SH::kBK, w_off[i],
+                l + SH::kXBytes + (SH::kWDma * wv + i) * 1024);
+#pragma unroll
+    for (int i = 0; i < SH::kXDma; ++i)
+      if (SH::kXEven || i + 1 < SH::kXDma || wv < 4)
+        lds_dma16(x_base + (int64_t)s * SH::kBK * 2, x_off[i], l + (8 * i + wv) * 1024);
+  };
+
+  // ---- operand reads: weight row 32 ng + r and activation row 32 mb + r, the
+  //      k of the k group: lane half h the h-th half of them
+  constexpr int KJ = SH::kKP / 16, WE = SH::kKP / 32;   // MFMA k steps; weight chunks of a lane
+  int w_rd[WE], x_rd[KJ];
+  {
+    const int row = 32 * ng + r;
+#pragma unroll
+    for (int e = 0; e < WE; ++e)
+      w_rd[e] = SH::kXBytes + row * SH::kBK + 16 * ((2 * WE * kg + WE * h + e) ^ swz(row, WC));
+#pragma unroll
+    for (int j = 0; j < KJ; ++j)
+      x_rd[j] = r * SH::kBK * 2 + 16 * ((2 * KJ * kg + KJ * h + j) ^ swz(r, XC));
+  }
+
+  // the tile's column scales (SwiGLU: w1's, then w3's): loaded ahead of the copies,
+  // put in LDS for the epilogue after the main loop
+  float* const sc_lds = reinterpret_cast<float*>(smem_raw + SH::kS * SH::kStage);
+  ST sc_raw = (ST)0.f;
+  if (EPI != kMidPartial && threadIdx.x < SH::kBN) {
+    const MidMat& ms = a.mat[EPI == kMidSwiglu ? (threadIdx.x >= kCols) : mi];
+    const int n = min(n0 + (int)(threadIdx.x % kCols), ms.N - 1);
+    sc_raw = reinterpret_cast<const ST*>(ms.scales)[(int64_t)n * ms.s_sn];
+  }
+
+  f32x16 acc[MB];
+#pragma unroll
+  for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) acc[mb][i] = 0.f;
+
+  // Stage s's operands are read from LDS one step before its MFMAs, so that the
+  // reads (and the copies behind them) run under the MFMAs of stage s - 1: with
+  // the waves in step at the barrier, reads and MFMAs would otherwise take turns.
+  struct Ops { u32x4 q[WE]; v8 xa[KJ][MB]; };
+  // this wave's copies landed, but for the last `later` stages' worth (a constant:
+  // a chain of branches over run-time counts cost 200 cycles per stage)
+  auto wait = [&](auto later) {
+    constexpr int L = decltype(later)::value;
+    if (SH::kXEven || wv < 4) vm_wait<L * (SH::kXDma + SH::kWDma)>();
+    else vm_wait<L * (SH::kXDma + SH::kWDma - 1)>();
+  };
+  auto read = [&](int slot, Ops& o) {
+    const unsigned char* st = smem_raw + slot * SH::kStage;
+#pragma unroll
+    for (int e = 0; e < WE; ++e) o.q[e] = *reinterpret_cast<const u32x4*>(st + w_rd[e]);
+#pragma unroll
+    for (int j = 0; j < KJ; ++j)
+#pragma unroll
+      for (int mb = 0; mb < MB; ++mb)
+        o.xa[j][mb] = __builtin_bit_cast(
+            v8, *reinterpret_cast<const u32x4*>(st + x_rd[j] + mb * 32 * SH::kBK * 2));
+  };
+  auto mul = [&](const Ops& o) {
+#pragma unroll
+    for (int j = 0; j < KJ; ++j) {
+      const u32x4& q = o.q[j >> 1];
+      const v8 wb = (j & 1) ? OP::widen(q.z, q.w) : OP::widen(q.x, q.y);
+#pragma unroll
+      for (int mb = 0; mb < MB; ++mb) acc[mb] = OP::mma(wb, o.xa[j][mb], acc[mb]);
+    }
+  };
+  int slot = 0;   // of stage s
+  constexpr int S = SH::kS, kHalf = (S - 1) / 2;
+  auto step = [&](auto steady, int s, const Ops& cur, Ops& next) {
+    const int old = slot;
+    slot = slot + 1 == S ? 0 : slot + 1;
+    if (decltype(steady)::value || s + 1 < nk) {
+      if (decltype(steady)::value) wait(std::integral_constant<int, S - 2>());
+      else if (nk - 2 - s >= kHalf) wait(std::integral_constant<int, kHalf>());
+      else wait(std::integral_constant<int, 0>());
+      // stage s + 1 is published, and every wave has read stage s: its slot is free
+      block_sync_lds();
+      read(slot, next);
+      if (decltype(steady)::value) issue(s + S, old);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    mul(cur);
+  };
+#pragma unroll
+  for (int p = 0; p < S; ++p)
+    if (s0 + p < nk) issue(s0 + p, p);
+  if (nk - s0 >= S) wait(std::integral_constant<int, S - 1>());
+  else wait(std::integral_constant<int, 0>());
+  block_sync_lds();
+  Ops oa, ob;
+  read(0, oa);
+  int s = s0;
+  for (; s + S + 1 < nk; s += 2) {   // stages s and s + 1 each have an (s + S)-th to fetch
+    step(std::true_type(), s, oa, ob);
+    step(std::true_type(), s + 1, ob, oa);
+  }
+  if (s + S < nk) {                  // one more
+    step(std::true_type(), s, oa, ob);
+    ++s;
+    oa = ob;
+  }
+  for (; s + 1 < nk; s += 2) {
+    step(std::false_type(), s, oa, ob);
+    step(std::false_type(), s + 1, ob, oa);
+  }
+  if (s < nk) step(std::false_type(), s, oa, ob);
+
+  // ---- the k groups' sums: unit (mb, g) = columns 8 g + 4 h .. + 3 of rows 32 mb + r
+  //      is finished by one owner wave of the n group, which adds the KG sums in
+  //      k-group order; the others hand theirs over in LDS (the ring, once every
+  //      wave has read its last stage)
+  auto owner = [](int mb, int g) { return KG == 2 ? (g & 1) : ((2 * mb + (g & 1)) & (KG - 1)); };
+  constexpr int UPO = KG == 2 ? 2 * MB : 2;    // units of an owner
+  auto unit_at = [&](int mb, int g, int src) -> f32x4* {
+    const int own = owner(mb, g), local = KG == 2 ? 2 * mb + (g >> 1) : (g >> 1);
+    const int k = src < own ? src : src - 1;
+    return reinterpret_cast<f32x4*>(smem_raw) +
+           ((((ng * KG + own) * UPO + local) * (KG - 1) + k) * 64 + lane);
+  };
+  block_sync_lds();
+  if (EPI != kMidPartial && threadIdx.x < SH::kBN) sc_lds[threadIdx.x] = Elem<ST>::to_f32(sc_raw);
+#pragma unroll
+  for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+    for (int g = 0; g < 4; ++g)
+      if (owner(mb, g) != kg)
+        *unit_at(mb, g, kg) = f32x4{acc[mb][4 * g], acc[mb][4 * g + 1], acc[mb][4 * g + 2],
+                                    acc[mb][4 * g + 3]};
+  block_sync_lds();
+  auto unit = [&](int mb, int g) -> f32x4 {
+    const f32x4 own = f32x4{acc[mb][4 * g], acc[mb][4 * g + 1], acc[mb][4 * g + 2], acc[mb][4 * g + 3]};
+    f32x4 t = kg == 0 ? own : *unit_at(mb, g, 0);
+#pragma unroll
+    for (int src = 1; src < KG; ++src) t += src == kg ? own : *unit_at(mb, g, src);
+    return t;
+  };
+
+  if constexpr (EPI == kMidPartial) {
+    float* pp = a.part + (int64_t)split * a.M * mt.N;
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        if (owner(mb, g) != kg) continue;
+        const f32x4 t = unit(mb, g);
+        const int nb = n0 + 32 * ng + 8 * g + 4 * h, m = m0 + 32 * mb + r;
+        if (m >= a.M) continue;
+        float* q = pp + (int64_t)m * mt.N + nb;
+        if (a.part_vec && nb + 3 < mt.N) {
+          *reinterpret_cast<f32x4*>(q) = t;
+        } else {
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            if (nb + i < mt.N) q[i] = t[i];
+        }
+      }
+    return;
+  }
+  typedef T t4 __attribute__((ext_vector_type(4)));
+  auto rnd = [](float v) { return Elem<T>::to_f32(Elem<T>::from_f32(v)); };
+  T* const y = reinterpret_cast<T*>(mt.y);
+  constexpr int GO = EPI == kMidSwiglu ? 2 : 4;   // column groups of the output
+#pragma unroll
+  for (int g = 0; g < GO; ++g) {
+    const int nb = n0 + (EPI == kMidSwiglu ? 16 : 32) * ng + 8 * g + 4 * h;
+    const f32x4 s1 = *reinterpret_cast<const f32x4*>(sc_lds + nb - n0);
+    f32x4 s3 = s1;
+    if constexpr (EPI == kMidSwiglu) s3 = *reinterpret_cast<const f32x4*>(sc_lds + kCols + nb - n0);
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb) {
+      if (owner(mb, g) != kg) continue;
+      const f32x4 t = unit(mb, g);
+      t4 v;
+      if constexpr (EPI == kMidSwiglu) {
+        const f32x4 u = unit(mb, g + 2);   // same owner: owner() looks at g's low bit
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          v[i] = Elem<T>::from_f32(rnd(silu_f32(rnd(t[i] * s1[i]))) * rnd(u[i] * s3[i]));
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = Elem<T>::from_f32(t[i] * s1[i]);
+      }
+      const int m = m0 + 32 * mb + r;
+      if (m >= a.M) continue;
+      T* yp = y + (int64_t)m * mt.y_sm + nb;
+      const T* rp = reinterpret_cast<const T*>(a.res) + (int64_t)m * a.res_sm + nb;
+      if (mt.y_vec && nb + 3 < mt.N && (a.res == nullptr || a.res_vec)) {
+        if (a.res != nullptr) {
+          const t4 rv = *reinterpret_cast<const t4*>(rp);
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            v[i] = Elem<T>::from_f32(Elem<T>::to_f32(rv[i]) + Elem<T>::to_f32(v[i]));
+        }
+        *reinterpret_cast<t4*>(yp) = v;
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          if (nb + i < mt.N)
+            yp[i] = a.res == nullptr
+                        ? v[i] : Elem<T>::from_f32(Elem<T>::to_f32(rp[i]) + Elem<T>::to_f32(v[i]));
+      }
+    }
+  }
+}
+
 }  // namespace mi
 
 using namespace mi;
@@ -870,4 +1213,202 @@ extern "C" int32_t mi_w8a16_gemm_residual(const void* x, const int8_t* w, const 
   if (rc != MI_OK) return rc;
   launch_reduce(a, (int32_t)used, dtype, sdtype, st);
   return launch_status(what);
+}
+
+// ---- small-M GEMM: shape rules and launch ---------------------------------
+
+namespace {
+
+// k groups per workgroup: 4 (64-column tiles) up to 64 rows, where x is cheap
+// to re-read and every CU should stream weights; 2 (128 columns) above.
+int mid_kg(int64_t m) { return m <= 64 ? 4 : 2; }
+
+// K granularity: a stage of the tallest-stage kernels
+int mid_bk(int kg) { return 64 * kg; }
+
+// K splits of one matrix: 2048 k per split at least, about one workgroup per CU.
+int64_t mid_splits(int64_t m, int64_t n, int64_t k) {
+  const int kg = mid_kg(m);
+  const int64_t bn = 256 / kg, mmax = kg == 4 ? 64 : 160;
+  const int64_t tiles = ((m + mmax - 1) / mmax) * ((n + bn - 1) / bn);
+  int64_t s = device_cu_count() / (tiles > 0 ? tiles : 1);
+  if (s > k / 2048) s = k / 2048;
+  if (s > 8) s = 8;
+  while (s > 1 && s * m * n * 4 > (64LL << 20)) --s;
+  if (s <= 1) return 1;
+  const int64_t nk = k / mid_bk(kg), per = (nk + s - 1) / s;
+  return (nk + per - 1) / per;
+}
+
+// 32-row blocks per tile: the least rounds of the grid times the bytes that a
+// workgroup copies per stage, over the sizes that are built.
+int mid_mb(int64_t m, int64_t tiles_n, int kg) {
+  const int cus = device_cu_count(), top = kg == 4 ? 2 : 5;
+  int best = 1;
+  int64_t cost = INT64_MAX;
+  for (int mb = 1; mb <= top; ++mb) {
+    const int64_t tiles = (m + 32 * mb - 1) / (32 * mb) * tiles_n;
+    // a stage of 64 kg k: 4 kg KB of x for each row block, 16 KB of weights; the
+    // measured stage times follow (300 rows: 0.59 us for one block, 1.28 for five)
+    const int64_t c = (tiles + cus - 1) / cus * (4 * kg * mb + 16);
+    if (c < cost) { cost = c; best = mb; }
+  }
+  return best;
+}
+
+template <typename T, typename ST, int MB, int KG, int EPI>
+hipError_t mid_launch(const MidArgs& a, int64_t splits, hipStream_t st) {
+  using SH = MidShape<MB, KG>;
+  static const hipError_t attr = hipFuncSetAttribute(
+      reinterpret_cast<const void*>(w8a16_mid_kernel<T, ST, MB, KG, EPI>),
+      hipFuncAttributeMaxDynamicSharedMemorySize, (int)SH::kLds);
+  if (attr != hipSuccess) return attr;
+  const unsigned grid = (unsigned)((int64_t)a.tiles_m * a.tiles_n * splits);
+  hipLaunchKernelGGL((w8a16_mid_kernel<T, ST, MB, KG, EPI>), dim3(grid), dim3(512), SH::kLds, st, a);
+  return hipGetLastError();
+}
+
+template <typename T, typename ST, int EPI>
+hipError_t mid_dispatch(const MidArgs& a, int kg, int mb, int64_t splits, hipStream_t st) {
+  if (kg == 4)
+    return mb == 1 ? mid_launch<T, ST, 1, 4, EPI>(a, splits, st)
+                   : mid_launch<T, ST, 2, 4, EPI>(a, splits, st);
+  switch (mb) {
+    case 1: return mid_launch<T, ST, 1, 2, EPI>(a, splits, st);
+    case 2: return mid_launch<T, ST, 2, 2, EPI>(a, splits, st);
+    case 3: return mid_launch<T, ST, 3, 2, EPI>(a, splits, st);
+    case 4: return mid_launch<T, ST, 4, 2, EPI>(a, splits, st);
+    default: return mid_launch<T, ST, 5, 2, EPI>(a, splits, st);
+  }
+}
+
+template <int EPI>
+hipError_t mid_dtypes(const MidArgs& a, int kg, int mb, int64_t splits, int32_t dtype,
+                      int32_t sdtype, hipStream_t st) {
+  if (dtype == MI_DTYPE_BF16) {
+    if (sdtype == MI_DTYPE_BF16) return mid_dispatch<bf16_t, bf16_t, EPI>(a, kg, mb, splits, st);
+    if (sdtype == MI_DTYPE_F16) return mid_dispatch<bf16_t, f16_t, EPI>(a, kg, mb, splits, st);
+    return mid_dispatch<bf16_t, float, EPI>(a, kg, mb, splits, st);
+  }
+  if (sdtype == MI_DTYPE_BF16) return mid_dispatch<f16_t, bf16_t, EPI>(a, kg, mb, splits, st);
+  if (sdtype == MI_DTYPE_F16) return mid_dispatch<f16_t, f16_t, EPI>(a, kg, mb, splits, st);
+  return mid_dispatch<f16_t, float, EPI>(a, kg, mb, splits, st);
+}
+
+}  // namespace
+
+extern "C" int64_t mi_w8a16_small_gemm_splits(int64_t m, int64_t n, int64_t k) {
+  if (m <= 0 || n <= 0 || k <= 0) return 1;
+  return mid_splits(m, n, k);
+}
+
+extern "C" int32_t mi_w8a16_small_gemm(const void* x, int64_t m, int64_t k, int64_t x_sm,
+                                       int32_t n_mats, const int8_t* const* w,
+                                       const void* const* scales, void* const* y,
+                                       const int64_t* n, const int64_t* w_sn,
+                                       const int64_t* s_sn, const int64_t* y_sm,
+                                       int32_t epilogue, const void* res, int64_t res_sm,
+                                       float* part, int64_t part_elems, int32_t dtype,
+                                       int32_t sdtype, void* stream) {
+  const char* what = "w8a16_small_gemm";
+  if (n_mats < 1 || n_mats > kMidMats || w == nullptr || scales == nullptr || y == nullptr ||
+      n == nullptr || w_sn == nullptr || s_sn == nullptr || y_sm == nullptr) {
+    set_last_error("%s: need 1..%d matrices and non-null argument arrays (n_mats=%d)", what,
+                   kMidMats, (int)n_mats);
+    return MI_ERR_INVALID;
+  }
+  if (!dtypes_ok(dtype, sdtype)) {
+    set_last_error("%s: activations must be bf16 or fp16 (dtype %d, scales %d)", what,
+                   (int)dtype, (int)sdtype);
+    return MI_ERR_UNSUPPORTED;
+  }
+  // epilogue 0: y_i = x w_i^T * s_i;  1: y = res + that (one matrix);
+  // 2: y_0 = silu(x w_0^T * s_0) * (x w_1^T * s_1) (two matrices of one shape)
+  if (epilogue < 0 || epilogue > 2 || (epilogue == 1 && (n_mats != 1 || res == nullptr)) ||
+      (epilogue == 2 && (n_mats != 2 || n[0] != n[1])) || (epilogue != 1 && res != nullptr)) {
+    set_last_error("%s: epilogue %d does not fit %d matrices", what, (int)epilogue, (int)n_mats);
+    return MI_ERR_INVALID;
+  }
+  if (m < 1 || m > 65535) {
+    set_last_error("%s: need 1 <= M <= 65535 (M=%lld)", what, (long long)m);
+    return MI_ERR_INVALID;
+  }
+  const int kg = mid_kg(m), bn = 256 / kg;
+  if (k % mid_bk(kg) != 0) {
+    set_last_error("%s: K must be a multiple of %d (K=%lld)", what, mid_bk(kg), (long long)k);
+    return MI_ERR_UNSUPPORTED;
+  }
+  MidArgs a{};
+  const int cols = epilogue == 2 ? bn / 2 : bn;
+  int64_t tiles_n = 0;
+  for (int i = 0; i < n_mats; ++i) {
+    GemmArgs g;
+    void* yi = epilogue == 2 ? y[0] : y[i];
+    int32_t rc = gemm_setup(what, x, w[i], scales[i], yi, m, n[i], k, x_sm, w_sn[i], s_sn[i],
+                            epilogue == 2 ? y_sm[0] : y_sm[i], g);
+    if (rc != MI_OK) return rc;
+    a.mat[i] = MidMat{g.w, g.scales, yi, g.w_sn, g.s_sn, g.y_sm, g.N, (int32_t)tiles_n, g.y_vec};
+    if (epilogue != 2 || i == 0) tiles_n += (n[i] + cols - 1) / cols;
+  }
+  if (epilogue == 1 && res_sm < n[0]) {
+    set_last_error("%s: residual rows shorter than N", what);
+    return MI_ERR_INVALID;
+  }
+  a.x = static_cast<const unsigned char*>(x);
+  a.res = res;
+  a.x_sm = x_sm;
+  a.res_sm = res_sm;
+  a.res_vec = res != nullptr && (uintptr_t)res % 8 == 0 && res_sm % 4 == 0 ? 1 : 0;
+  a.M = (int32_t)m;
+  a.K = (int32_t)k;
+  a.n_mats = n_mats;
+  const int64_t splits = n_mats == 1 ? mid_splits(m, n[0], k) : 1;
+  if (n_mats > 1) {
+    for (int i = 0; i < n_mats; ++i)
+      if (mid_splits(m, n[i], k) != 1) {
+        set_last_error("%s: a matrix that splits K has no fused form (N=%lld K=%lld)", what,
+                       (long long)n[i], (long long)k);
+        return MI_ERR_UNSUPPORTED;
+      }
+  }
+  const int mb = mid_mb(m, tiles_n * splits, kg);
+  a.tiles_m = (int32_t)((m + 32 * mb - 1) / (32 * mb));
+  a.tiles_n = (int32_t)tiles_n;
+  if (tiles_n * a.tiles_m * splits > INT32_MAX / 64) {
+    set_last_error("%s: too many tiles", what);
+    return MI_ERR_INVALID;
+  }
+  hipStream_t st = (hipStream_t)stream;
+  hipError_t e;
+  if (splits > 1) {
+    if (part == nullptr || part_elems < splits * m * n[0]) {
+      set_last_error("%s: workspace needs %lld fp32 elements (given %lld)", what,
+                     (long long)(splits * m * n[0]), (long long)part_elems);
+      return MI_ERR_INVALID;
+    }
+    const int64_t nk = k / mid_bk(kg);
+    a.part = part;
+    // in stages of the kernel that runs (half as deep above three row blocks)
+    a.split_stages = (int32_t)((nk + splits - 1) / splits) * (mb > 3 ? 2 : 1);
+    a.part_vec = (uintptr_t)part % 16 == 0 && n[0] % 4 == 0 ? 1 : 0;
+    e = mid_dtypes<kMidPartial>(a, kg, mb, splits, dtype, sdtype, st);
+    if (e == hipSuccess) {
+      GemmArgs g;
+      gemm_setup(what, x, w[0], scales[0], y[0], m, n[0], k, x_sm, w_sn[0], s_sn[0], y_sm[0], g);
+      g.part = part;
+      g.part_vec = a.part_vec;
+      g.res = res;
+      g.res_sm = res_sm;
+      launch_reduce(g, (int32_t)splits, dtype, sdtype, st);
+      e = hipGetLastError();
+    }
+  } else {
+    e = epilogue == 2 ? mid_dtypes<kMidSwiglu>(a, kg, mb, 1, dtype, sdtype, st)
+                      : mid_dtypes<kMidStore>(a, kg, mb, 1, dtype, sdtype, st);
+  }
+  if (e != hipSuccess) {
+    set_last_error("%s: launch failed: %s", what, hipGetErrorString(e));
+    return (int32_t)e;
+  }
+  return MI_OK;
 }

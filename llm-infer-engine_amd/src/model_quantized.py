@@ -33,8 +33,9 @@ class QuantizedFeedForward(FeedForward):
     def forward(self, x, *, residual=None):
         """silu(w1(x)) * w3(x) in one launch (the same rounding points, neither
         projection written out): up to 16 rows in the decode projection
-        kernels, prefill-sized inputs in the GEMM when its tiles fill the GPU;
-        otherwise the op chain of src/model.py:23."""
+        kernels, prefill-sized inputs in the large GEMM when its tiles fill the
+        GPU and in the small-M GEMM otherwise; other sizes take the op chain of
+        src/model.py:23."""
         x2 = x.reshape(-1, x.shape[-1])
         w1, w3 = self.w1, self.w3
         if _rows_fusable(x2, w1, swiglu=True) and _rows_fusable(x2, w3):
@@ -43,10 +44,15 @@ class QuantizedFeedForward(FeedForward):
             out = self.down(h.view(*x.shape[:-1], w1.out_features), residual)
             torch.cuda.nvtx.range_pop()
             return out
-        if not quant_linear.swiglu_worth(x2.shape[0], x2.shape[1], w1.out_features, x.device):
+        mats = [(w1.weight, w1.scales), (w3.weight, w3.scales)]
+        if quant_linear.swiglu_worth(x2.shape[0], x2.shape[1], w1.out_features, x.device):
+            torch.cuda.nvtx.range_push("FFN")
+            h = quant_linear.w8a16_gemm_swiglu(x2, *mats[0], *mats[1])
+        elif quant_linear.small_gemm_fuses(x2, mats):
+            torch.cuda.nvtx.range_push("FFN")
+            h = quant_linear.w8a16_small_gemm(x2, mats, swiglu=True)[0]
+        else:
             return super().forward(x, residual=residual)
-        torch.cuda.nvtx.range_push("FFN")
-        h = quant_linear.w8a16_gemm_swiglu(x2, w1.weight, w1.scales, w3.weight, w3.scales)
         out = self.down(h.view(*x.shape[:-1], w1.out_features), residual)
         torch.cuda.nvtx.range_pop()
         return out
@@ -67,15 +73,26 @@ def _project_residual(lin, h, residual):
     (up to 16 rows) or of the GEMM (the same roundings as the separate ops);
     otherwise the two ops."""
     h2 = h.reshape(-1, h.shape[-1])
-    if (residual is not None and residual.dtype == h.dtype
-            and residual.shape == (*h.shape[:-1], lin.out_features) and _rows_fusable(h2, lin)):
+    rows = h2.shape[0]
+    # below GEMM_MIN_ROWS any residual that `residual + out` takes is served: the
+    # fused forms when it has h's dtype and the output's shape, else the two ops
+    plain = (residual is not None and residual.dtype == h.dtype and residual.device == h.device
+             and residual.shape == (*h.shape[:-1], lin.out_features))
+    if plain and _rows_fusable(h2, lin):
         res2 = residual.reshape(-1, lin.out_features)
         if res2.stride(1) == 1:
             return decode_layer.linear_fused(h2, lin, residual=res2).view(residual.shape)
-    if residual is None or not quant_linear.gemm_supported(h2.shape[0], h2.shape[1]):
+    gemm = rows >= quant_linear.GEMM_MIN_ROWS
+    small = quant_linear.small_gemm_worth(h2, lin.weight) and (gemm or plain)
+    if residual is None or not (small or quant_linear.gemm_supported(rows, h2.shape[1])):
         out = lin(h)
         return out if residual is None else residual + out
     res2 = residual.reshape(-1, lin.out_features)
+    if small:
+        if not gemm:
+            res2 = res2.contiguous()
+        y = quant_linear.w8a16_small_gemm(h2, [(lin.weight, lin.scales)], residual=res2)[0]
+        return y.view(*h.shape[:-1], lin.out_features)
     y = quant_linear.w8a16_gemm_residual(h2, lin.weight, lin.scales, res2)
     return y.view(*h.shape[:-1], lin.out_features)
 
@@ -88,15 +105,20 @@ class QuantizedAttention(Attention):
         return _project_residual(self.wo, output, residual)
 
     def qkv(self, x):
-        """Prefill-sized inputs: wq, wk and wv in one GEMM launch (bitwise the
-        three separate GEMMs without a K split) when their tiles together
-        fill the GPU; otherwise one W8A16Linear call each."""
+        """wq, wk and wv in one launch: of the large GEMM (bitwise the three
+        separate GEMMs without a K split) when their tiles together fill the
+        GPU, else of the small-M GEMM; sizes neither takes run one W8A16Linear
+        call each."""
         x2 = x.reshape(-1, x.shape[-1])
         mats = (self.wq, self.wk, self.wv)
-        if not quant_linear.gemm_multi_worth(x2.shape[0], x2.shape[1],
-                                             [m.out_features for m in mats], x.device):
+        pairs = [(m.weight, m.scales) for m in mats]
+        if quant_linear.gemm_multi_worth(x2.shape[0], x2.shape[1],
+                                         [m.out_features for m in mats], x.device):
+            ys = quant_linear.w8a16_gemm_multi(x2, pairs)
+        elif quant_linear.small_gemm_fuses(x2, pairs):
+            ys = quant_linear.w8a16_small_gemm(x2, pairs)
+        else:
             return super().qkv(x)
-        ys = quant_linear.w8a16_gemm_multi(x2, [(m.weight, m.scales) for m in mats])
         return tuple(y.reshape(*x.shape[:-1], m.out_features) for y, m in zip(ys, mats))
 
 

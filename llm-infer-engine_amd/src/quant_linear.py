@@ -8,10 +8,11 @@ the plain store epilogue, every weight load issued before the first MFMA)
 when the shape is one it serves, otherwise through the MFMA GEMV kernel
 mi_w8a16_gemv (any K, strided x, fp32 scales).  Prefill-sized inputs run the
 MFMA GEMM mi_w8a16_gemm (128 x 256 output tiles, int8 weight fragments widened
-in registers), with K split across workgroups (mi_w8a16_gemm_splitk) when the
-tiles alone cannot occupy the GPU.  Between the two, and for K not a multiple
-of 64, the small-M kernels serve the rows in 16-row slices: below
-GEMM_MIN_ROWS rows (two slices) the slices are faster.
+in registers).  Between the two (17 rows and up while that tile grid would leave
+CUs idle: a chat prompt, a large decode batch) mi_w8a16_small_gemm runs smaller
+tiles with a deeper copy pipeline.  K that neither takes (not a multiple of 64;
+below GEMM_MIN_ROWS rows not of 256) goes through the decode kernels in 16-row
+slices.
 """
 from __future__ import annotations
 
@@ -141,6 +142,52 @@ def w8a16_gemm_mfma(x, weight, scales, *, splits: int | None = None):
     return out
 
 
+def w8a16_small_gemm(x, mats, *, residual=None, swiglu: bool = False):
+    """mi_w8a16_small_gemm: x [M, K] times each (weight, scales) of `mats` (1-3
+    pairs) in one launch -> [y_i [M, N_i]]; with ``residual`` [M, N] (one pair)
+    [residual + y]; with ``swiglu`` (two pairs) [silu(y_0) * y_1].  One matrix
+    with a long K splits it and takes a second launch."""
+    import ctypes
+    prepped = [_prep(x, w, s) for w, s in mats]
+    x = prepped[0][0]
+    if x.stride(1) != 1:
+        x = x.contiguous()
+    M, K = x.shape
+    n = len(prepped)
+    if len({s.dtype for _, _, s in prepped}) != 1:
+        raise TypeError("w8a16_small_gemm: all scales must share a dtype")
+    if residual is not None:
+        N = prepped[0][1].shape[0]
+        if residual.shape != (M, N) or residual.dtype != x.dtype or residual.device != x.device:
+            raise ValueError(f"residual must be [{M}, {N}] {x.dtype} on {x.device}, "
+                             f"got {tuple(residual.shape)} {residual.dtype}")
+        if residual.stride(1) != 1:
+            residual = residual.contiguous()
+    outs = [torch.empty((M, w.shape[0]), device=x.device, dtype=x.dtype)
+            for _, w, _ in (prepped[:1] if swiglu else prepped)]
+    lib = _lib.load()
+    part = None
+    if n == 1:
+        S = lib.mi_w8a16_small_gemm_splits(M, prepped[0][1].shape[0], K)
+        if S > 1:
+            part = torch.empty(S * M * prepped[0][1].shape[0], device=x.device, dtype=torch.float32)
+    P = ctypes.c_void_p * n
+    I = ctypes.c_int64 * n
+    ys = outs * n if swiglu else outs
+    arrays = (P(*[w.data_ptr() for _, w, _ in prepped]), P(*[s.data_ptr() for _, _, s in prepped]),
+              P(*[y.data_ptr() for y in ys]), I(*[w.shape[0] for _, w, _ in prepped]),
+              I(*[w.stride(0) for _, w, _ in prepped]), I(*[s.stride(0) for _, _, s in prepped]),
+              I(*[y.stride(0) for y in ys]))
+    st = lib.mi_w8a16_small_gemm(
+        x.data_ptr(), M, K, x.stride(0), n, *map(ctypes.addressof, arrays),
+        2 if swiglu else 0 if residual is None else 1, _lib.ptr(residual),
+        0 if residual is None else residual.stride(0), _lib.ptr(part),
+        0 if part is None else part.numel(), _lib.dtype_code(x.dtype),
+        _lib.dtype_code(prepped[0][2].dtype), _lib.stream_of(x))
+    _lib.check(st, "w8a16_small_gemm")
+    return outs
+
+
 _GEMM_TILE_M, _GEMM_TILE_N = 128, 256
 _CUS: dict = {}
 
@@ -179,6 +226,40 @@ def w8a16_gemm_residual(x, weight, scales, res, *, splits: int | None = None):
         _lib.dtype_code(x.dtype), _lib.dtype_code(s.dtype), _lib.stream_of(x))
     _lib.check(st, "w8a16_gemm_residual")
     return out
+
+
+def _small_gemm_takes(M: int, K: int) -> bool:
+    """Sizes mi_w8a16_small_gemm is built for (and used for: 17 rows and more)."""
+    return _GEMV_MAX_ROWS < M <= 65535 and K % (256 if M <= 64 else 128) == 0
+
+
+def small_gemm_worth(x, weight) -> bool:
+    """Whether w8a16_small_gemm should serve [M, K] rows x through one matrix:
+    more rows than the decode kernels take, and a grid of 128 x 256 tiles that
+    leaves three CUs in ten idle or more.  Measured at both sides: N = 2048, M =
+    2048 (128 tiles of 256 CUs) 26 us against 43 (K = 2048), 79 against 92 (K =
+    8192); N = 3072, M = 2048 (192 tiles) 62 against 54 and 147 against 133."""
+    M, K = x.shape
+    if not _small_gemm_takes(M, K):
+        return False
+    N = weight.shape[0]
+    tiles = -(-M // _GEMM_TILE_M) * -(-N // _GEMM_TILE_N)
+    if tiles * 10 > 7 * _cu_count(x.device):
+        return False
+    # row strides that only the 16-row slices take (they serve such calls below 33 rows)
+    return M >= GEMM_MIN_ROWS or all(K <= t.stride(0) <= (1 << 23) or t.stride(1) != 1
+                                     for t in (x, weight))
+
+
+def small_gemm_fuses(x, mats) -> bool:
+    """Whether one w8a16_small_gemm launch takes several (weight, scales) of the
+    same x: built sizes, no matrix that would split K, one scale dtype."""
+    M, K = x.shape
+    lib = _lib.load()
+    return (_small_gemm_takes(M, K) and len({s.dtype for _, s in mats}) == 1
+            and (M >= GEMM_MIN_ROWS or all(K <= t.stride(0) <= (1 << 23) and t.stride(1) == 1
+                                           for t in (x, *(w for w, _ in mats))))
+            and all(lib.mi_w8a16_small_gemm_splits(M, w.shape[0], K) == 1 for w, _ in mats))
 
 
 def gemm_multi_worth(M: int, K: int, out_features, device) -> bool:
@@ -266,6 +347,8 @@ def w8a16_gemm_launch(x, weight, scales, *, block_m: int = 64, block_n: int = 64
     """Same contract as w8a16_gemv_launch for any M (src/quant_linear.py:191-247).
     block_m/block_n/block_k are accepted for signature compatibility (the
     MFMA tiling is fixed)."""
+    if small_gemm_worth(x, weight):
+        return w8a16_small_gemm(x, [(weight, scales)])[0]
     if gemm_supported(x.shape[0], x.shape[1]):
         return w8a16_gemm_mfma(x, weight, scales)
     return w8a16_rows(x, weight, scales)

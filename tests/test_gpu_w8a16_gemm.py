@@ -343,3 +343,65 @@ def test_gemm_residual_is_the_separate_add(dev, M, K, N, dtype, splits, pad):
     assert torch.equal(y, res + w8a16_gemm_mfma(x, q, s, splits=S))
     with pytest.raises(ValueError):
         w8a16_gemm_residual(x, q, s, res[:, :-1])
+
+
+@pytest.mark.parametrize("M", [17, 33, 64, 65, 97, 129, 161, 300])
+@pytest.mark.parametrize("K,N", [(256, 100), (768, 516), (2048, 2048), (8192, 1027)])
+def test_small_gemm_tile_edges(dev, M, K, N):
+    """mi_w8a16_small_gemm at both tile widths (up to 64 rows and above), with
+    row counts around each number of 32-row blocks, partial columns, rings
+    deeper and shallower than K, and K = 8192 split: against the oracle, and
+    bit-exact where each output is one product (one-hot rows)."""
+    from src.quant_linear import w8a16_small_gemm
+    dtype = torch.bfloat16 if M % 2 else torch.float16
+    q, s = _quantised(N, K, dtype, dev, 200)
+    x = _x(M, K, dtype, dev, 201)
+    res = _x(M, N, dtype, dev, 202)
+    y = w8a16_small_gemm(x, [(q, s)])[0]
+    ref = oq.w8a16(x, q, s)
+    assert _rel(y, ref) < 2e-2
+    assert torch.equal(w8a16_small_gemm(x, [(q, s)], residual=res)[0], res + y)
+    hot = torch.zeros_like(x)
+    k_of = torch.randint(0, K, (M,), generator=torch.Generator().manual_seed(203)).to(dev)
+    hot[torch.arange(M, device=dev), k_of] = 0.5
+    one = w8a16_small_gemm(hot, [(q, s)])[0]
+    assert torch.equal(one, ((q[:, k_of].t().float() * 0.5) * s.float().view(-1)).to(dtype))
+
+
+@pytest.mark.parametrize("M", [24, 64, 96, 300])
+def test_small_gemm_fused_forms(dev, M):
+    """Several matrices in one launch and the SwiGLU epilogue against the same
+    matrices alone (bit for bit up to 64 rows; above, the tile height and with
+    it the fp32 summation order may differ), ragged N, fp32 scales, a strided x."""
+    from src.quant_linear import w8a16_small_gemm
+    K, dtype = 1024, torch.bfloat16
+    x = _x(M, K + 64, dtype, dev, 210)[:, :K]
+    mats = [_quantised(N, K, dtype, dev, 211 + N) for N in (520, 96, 333)]
+    alone = [w8a16_small_gemm(x, [m])[0] for m in mats]
+    for y, a in zip(w8a16_small_gemm(x, mats), alone):
+        assert torch.equal(y, a) if M <= 64 else _rel(y, a) < 1e-2
+    mats = [(q, s.float()) for q, s in (_quantised(777, K, dtype, dev, i) for i in (215, 216))]
+    y1, y3 = (w8a16_small_gemm(x, [m])[0] for m in mats)
+    g = w8a16_small_gemm(x, mats, swiglu=True)[0]
+    assert _rel(g, torch.nn.functional.silu(y1) * y3) < 1e-2
+    with pytest.raises(TypeError):
+        w8a16_small_gemm(x, [mats[0], (mats[1][0], mats[1][1].bfloat16())], swiglu=True)
+    with pytest.raises(ValueError):
+        w8a16_small_gemm(x, mats[:1], residual=y1[:, :-1])
+
+
+@pytest.mark.parametrize("M", [17, 32, 40, 200])
+def test_feed_forward_between_decode_and_prefill_sizes(dev, M):
+    """The feed-forward half at the row counts of the small-M GEMM against its op
+    chain on the same inputs (strided and expanded rows included)."""
+    from src.model import FeedForward
+    from src.model_quantized import QuantizedFeedForward
+    ff = QuantizedFeedForward(1024, 2048).to(dev)
+    for i, lin in enumerate((ff.w1, ff.w2, ff.w3)):
+        q, s = _quantised(lin.out_features, lin.in_features, torch.bfloat16, dev, 220 + i)
+        lin.weight.data.copy_(q)
+        lin.scales.data.copy_(s.view(-1, 1) * 0.03)
+    x = _x(M, 1024, torch.bfloat16, dev, 223)
+    for rows in (x, _x(M, 2048, torch.bfloat16, dev, 224)[:, :1024]) + ((x[:1].expand(M, 1024),) if M < 33 else ()):
+        ref = rows + FeedForward.forward(ff, rows)
+        assert _rel(ff(rows, residual=rows), ref) < 1e-2
