@@ -25,9 +25,13 @@ EPI_RESIDUAL = 1
 EPI_SWIGLU = 2
 
 
-def _w(lin):
-    """int8 weight [N, K], scales [N] of a W8A16Linear."""
-    return lin.weight, lin.scales.reshape(-1)
+def weights_of(lin):
+    """(int8 weight [N, K], contiguous scales of N elements) of a W8A16Linear;
+    such a pair, fetched by the caller once for several uses, is passed through."""
+    if type(lin) is tuple:
+        return lin
+    s = lin.scales
+    return lin.weight, s if s.is_contiguous() else s.reshape(-1)
 
 
 #: reduction lengths the fused GEMV kernels are built for (K = 512 * waves)
@@ -41,12 +45,12 @@ def supported(M: int, K: int, dtype: torch.dtype, lin, norm_weight=None, *,
     be row-aligned (``aligned``).  Otherwise use the op-by-op path."""
     if dtype not in (torch.bfloat16, torch.float16):
         return False
-    w, s = _w(lin)
+    w, s = weights_of(lin)
     if not (1 <= M <= 16 and K in SUPPORTED_K and w.dtype == torch.int8):
         return False
     if not (w.is_contiguous() and w.shape[1] == K and w.data_ptr() % 16 == 0):
         return False
-    if s.dtype != dtype or not s.is_contiguous():
+    if s.dtype != dtype:
         return False
     if swiglu and K > 4096:
         return False
@@ -70,11 +74,11 @@ def linear_fused(x, lin, *, norm_weight=None, eps: float = 0.0, lin_b=None, resi
     residual [M, N]: y = residual + linear;  lin_b: y = silu(lin(x)) * lin_b(x).
     """
     M, K = x.shape
-    w, s = _w(lin)
+    w, s = weights_of(lin)
     N = w.shape[0]
     y = torch.empty((M, N), device=x.device, dtype=x.dtype)
     if lin_b is not None:
-        wb, sb = _w(lin_b)
+        wb, sb = weights_of(lin_b)
         epi = EPI_SWIGLU
     else:
         wb, sb = None, None
@@ -90,19 +94,18 @@ def linear_fused(x, lin, *, norm_weight=None, eps: float = 0.0, lin_b=None, resi
 
 
 def qkv_rope_append(x, attn, norm_weight, eps, rope_cos, rope_sin, rope_row0: int,
-                    pos: torch.Tensor, kv_cache, layer_idx: int):
+                    pos: torch.Tensor, kv_cache, layer_idx: int, *, weights=None):
     """rmsnorm -> wq|wk|wv -> RoPE; writes RoPE(k), v into cache slot pos[0] of
     layer `layer_idx` for rows 0..M-1 and returns q [M, n_heads, 1, head_dim].
+    ``weights``: the three ``weights_of`` pairs, if the caller has them.
 
     rope_cos/rope_sin [rows, head_dim/2]; position p uses row p - rope_row0.
     """
     M, K = x.shape
     Hq, Hkv, D = attn.n_heads, attn.n_kv_heads, attn.head_dim
-    wq, sq = _w(attn.wq)
-    wk, sk = _w(attn.wk)
-    wv, sv = _w(attn.wv)
-    ck = kv_cache.k[layer_idx, :M]
-    cv = kv_cache.v[layer_idx, :M]
+    (wq, sq), (wk, sk), (wv, sv) = weights or map(weights_of, (attn.wq, attn.wk, attn.wv))
+    ck = kv_cache.k[layer_idx]
+    cv = kv_cache.v[layer_idx]
     if ck.dtype != x.dtype or rope_cos.dtype != x.dtype or rope_cos.stride() != rope_sin.stride():
         raise TypeError("fused QKV: cache, rope tables and activations must share a dtype and layout")
     q = torch.empty((M, Hq, 1, D), device=x.device, dtype=x.dtype)

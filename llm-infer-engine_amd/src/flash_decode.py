@@ -70,40 +70,39 @@ def _run_decode(q, k, v, mask, seq_lens, num_splits, return_lse, empty_nan, what
             raise ValueError(f"seq_lens must have shape ({batch_size},), got {tuple(seq_lens.shape)}")
         if seq_lens.device != q.device or seq_lens.dtype != torch.int64:
             seq_lens = seq_lens.to(device=q.device, dtype=torch.int64)
+    lib = _lib.load()
     if num_splits is None:
-        num_splits = default_num_splits(batch_size, n_heads, n_kv_heads, kv_len, head_dim)
+        num_splits = lib.mi_decode_default_splits(batch_size, n_heads, n_kv_heads, kv_len, head_dim)
     num_splits = int(num_splits)
     if num_splits < 1:
         raise ValueError(f"num_splits must be >= 1, got {num_splits}")
     num_splits = min(num_splits, kv_len)
     # too few splits to fill the GPU are subdivided into >= 1024-key ranges
-    num_splits = int(_lib.load().mi_decode_effective_splits(
+    num_splits = int(lib.mi_decode_effective_splits(
         batch_size, n_heads, n_kv_heads, kv_len, head_dim, num_splits))
     k = _kv_ready(k)
     v = _kv_ready(v)
     out = torch.empty_like(q)
     lse = torch.empty((batch_size, n_heads), device=q.device, dtype=torch.float32) if return_lse else None
+    part_m = part_l = part_acc = arrive = None
     if num_splits > 1:
-        part_m = torch.empty((batch_size, n_heads, num_splits), device=q.device, dtype=torch.float32)
-        part_l = torch.empty_like(part_m)
-        part_acc = torch.empty((batch_size, n_heads, num_splits, head_dim),
-                               device=q.device, dtype=torch.float32)
-    else:
-        part_m = part_l = part_acc = None
-    lib = _lib.load()
-    # with several splits the LSE combine runs inside the split launch, on the
-    # library's per-stream arrival counters (batch * n_heads bounds the groups)
-    arrive = _lib.arrive_counters(q, batch_size * n_heads) if num_splits > 1 else None
+        # one workspace: acc [B, Hq, splits, D], then m and l [B, Hq, splits]
+        n = batch_size * n_heads * num_splits
+        part = torch.empty(n * (head_dim + 2), device=q.device, dtype=torch.float32)
+        part_acc = part.data_ptr()
+        part_m = part_acc + 4 * n * head_dim
+        part_l = part_m + 4 * n
+        # with several splits the LSE combine runs inside the split launch, on the
+        # library's per-stream arrival counters (batch * n_heads bounds the groups)
+        arrive = _lib.arrive_counters(q, batch_size * n_heads)
+    qs, ks, vs, os_ = q.stride(), k.stride(), v.stride(), out.stride()
     st = lib.mi_flash_decode(
         q.data_ptr(), k.data_ptr(), v.data_ptr(),
         _lib.ptr(mask), mask_sb, mask_sl, _lib.ptr(seq_lens),
-        _lib.ptr(part_m), _lib.ptr(part_l), _lib.ptr(part_acc), arrive,
+        part_m, part_l, part_acc, arrive,
         out.data_ptr(), _lib.ptr(lse),
         batch_size, n_heads, n_kv_heads, kv_len, head_dim, num_splits,
-        q.stride(0), q.stride(1), q.stride(3),
-        k.stride(0), k.stride(1), k.stride(2),
-        v.stride(0), v.stride(1), v.stride(2),
-        out.stride(0), out.stride(1), out.stride(3),
+        qs[0], qs[1], qs[3], *ks[:3], *vs[:3], os_[0], os_[1], os_[3],
         1.0 / math.sqrt(head_dim), int(empty_nan), _lib.dtype_code(q.dtype), _lib.stream_of(q))
     _lib.check(st, what)
     return (out, lse) if return_lse else out

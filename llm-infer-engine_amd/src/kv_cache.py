@@ -32,6 +32,9 @@ class KVCache:
         # k holds RoPE-applied keys, v the projected values.
         self.k = torch.zeros(shape, device=args.device, dtype=self.dtype)
         self.v = torch.zeros(shape, device=args.device, dtype=self.dtype)
+        # slot numbers, for kernels that take a position from device memory: a
+        # decode step at a host position reads its entry instead of filling a tensor
+        self.positions = torch.arange(self.max_seq_len, device=args.device, dtype=torch.int64)
 
     def reset(self):
         self.k.zero_()

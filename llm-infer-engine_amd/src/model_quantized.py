@@ -38,7 +38,7 @@ class QuantizedFeedForward(FeedForward):
         src/model.py:23."""
         x2 = x.reshape(-1, x.shape[-1])
         w1, w3 = self.w1, self.w3
-        if _rows_fusable(x2, w1, swiglu=True) and _rows_fusable(x2, w3):
+        if x2.shape[0] <= 16 and _rows_fusable(x2, w1, swiglu=True) and _rows_fusable(x2, w3):
             torch.cuda.nvtx.range_push("FFN")
             h = decode_layer.linear_fused(x2, w1, lin_b=w3)
             out = self.down(h.view(*x.shape[:-1], w1.out_features), residual)
@@ -133,44 +133,50 @@ class QuantizedTransformerBlock(TransformerBlock):
     def __init__(self, args, linear=W8A16Linear):
         super().__init__(args, W8A16Linear)
 
-    def _fusable(self, x, rope_cos, kv_cache, layer_idx, positions, rope_by_position) -> bool:
+    def _fused_weights(self, x, rope_cos, kv_cache, layer_idx, positions, rope_by_position):
+        """The block's weights (``decode_layer.weights_of`` pairs of wq, wk, wv, wo,
+        w1, w3, w2) if the fused decode-layer kernels take this call, else None."""
         if not self.fused_decode or kv_cache is None or layer_idx is None or x.shape[1] != 1:
-            return False
+            return None
         if positions is not None and not rope_by_position:
-            return False  # per-step sliced tables at a device position: op chain
+            return None  # per-step sliced tables at a device position: op chain
         attn, ff = self.attention, self.feed_forward
         B, _, dim = x.shape
-        if (B > kv_cache.max_batch_size or kv_cache.k.dtype != x.dtype
-                or rope_cos.dtype != x.dtype or attn.head_dim % 16 != 0 or not x.is_contiguous()):
-            return False
         dt, sup = x.dtype, decode_layer.supported
-        n_o = attn.n_heads * attn.head_dim
-        return (decode_layer.aligned(x.view(B, dim)) and sup(B, dim, dt, attn.wq)
-                and sup(B, dim, dt, attn.wk) and sup(B, dim, dt, attn.wv)
-                and sup(B, n_o, dt, attn.wo)
-                and sup(B, dim, dt, ff.w1, swiglu=True)
-                and sup(B, dim, dt, ff.w3)
-                and sup(B, ff.w1.out_features, dt, ff.w2))
+        if (B > kv_cache.max_batch_size or kv_cache.k.dtype != dt
+                or rope_cos.dtype != dt or attn.head_dim % 16 != 0 or not x.is_contiguous()
+                or not decode_layer.aligned(x.view(B, dim))):
+            return None
+        ws = tuple(map(decode_layer.weights_of,
+                       (attn.wq, attn.wk, attn.wv, attn.wo, ff.w1, ff.w3, ff.w2)))
+        wq, wk, wv, wo, w1, w3, w2 = ws
+        ok = (sup(B, dim, dt, wq) and sup(B, dim, dt, wk) and sup(B, dim, dt, wv)
+              and sup(B, attn.n_heads * attn.head_dim, dt, wo)
+              and sup(B, dim, dt, w1, swiglu=True) and sup(B, dim, dt, w3)
+              and sup(B, w1[0].shape[0], dt, w2))
+        return ws if ok else None
 
     @staticmethod
     def _norm_in(x2, lin, norm, *, swiglu=False):
         """(rows, norm weight) for a projection of the normalised rows: the
         projection's own RMSNorm prologue where it takes these sizes, else the
         rows normalised by a launch of their own and no prologue."""
-        if decode_layer.supported(x2.shape[0], x2.shape[1], x2.dtype, lin, norm.weight, swiglu=swiglu):
-            return x2, norm.weight
+        nw = norm.weight
+        if decode_layer.supported(*x2.shape, x2.dtype, lin, nw, swiglu=swiglu):
+            return x2, nw
         return norm(x2), None
 
     def forward(self, x, rope_cos, rope_sin, layer_idx=None, start_pos=0, kv_cache=None,
                 use_cuda_graph=False, scatter_positions=None, decode_attn_mask=None, **ext):
         positions = scatter_positions if (use_cuda_graph and scatter_positions is not None) else None
         by_pos = bool(ext.get("rope_by_position", False))
-        if not self._fusable(x, rope_cos, kv_cache, layer_idx, positions, by_pos):
+        ws = self._fused_weights(x, rope_cos, kv_cache, layer_idx, positions, by_pos)
+        if ws is None:
             return super().forward(x, rope_cos, rope_sin, layer_idx=layer_idx, start_pos=start_pos,
                                    kv_cache=kv_cache, use_cuda_graph=use_cuda_graph,
                                    scatter_positions=scatter_positions,
                                    decode_attn_mask=decode_attn_mask, **ext)
-        attn, ff = self.attention, self.feed_forward
+        wq, _, _, wo, w1, w3, w2 = ws
         B, _, dim = x.shape
         x2 = x.view(B, dim)
         if positions is not None:  # graph path: device position, full-table RoPE rows
@@ -178,19 +184,26 @@ class QuantizedTransformerBlock(TransformerBlock):
             if pos.dtype != torch.int64:
                 pos = pos.to(torch.int64)
         else:
-            pos = torch.full((1,), int(start_pos), dtype=torch.int64, device=x.device)
-            row0 = 0 if by_pos else int(start_pos)
-        h, nw = self._norm_in(x2, attn.wq, self.attention_norm)
-        q = decode_layer.qkv_rope_append(h, attn, nw, self.attention_norm.eps, rope_cos, rope_sin,
-                                         row0, pos, kv_cache, layer_idx)
+            p = int(start_pos)
+            table = getattr(kv_cache, "positions", None)
+            if table is not None and 0 <= p < table.shape[0] and table.device == x.device:
+                pos = table[p:p + 1]
+            else:
+                pos = torch.full((1,), p, dtype=torch.int64, device=x.device)
+            row0 = 0 if by_pos else p
+        norm = self.attention_norm
+        h, nw = self._norm_in(x2, wq, norm)
+        q = decode_layer.qkv_rope_append(h, self.attention, nw, norm.eps, rope_cos, rope_sin,
+                                         row0, pos, kv_cache, layer_idx, weights=ws[:3])
         ck, cv = kv_cache.k[layer_idx, :B], kv_cache.v[layer_idx, :B]
         if positions is None:
             ck, cv = ck[:, :, :int(start_pos) + 1], cv[:, :, :int(start_pos) + 1]
         o = flash_decode(q, ck, cv, mask=decode_attn_mask, seq_lens=ext.get("seq_lens"))
-        h = decode_layer.linear_fused(o.view(B, -1), attn.wo, residual=x2)
-        n, nw = self._norm_in(h, ff.w1, self.ffn_norm, swiglu=True)
-        g = decode_layer.linear_fused(n, ff.w1, norm_weight=nw, eps=self.ffn_norm.eps, lin_b=ff.w3)
-        y = decode_layer.linear_fused(g, ff.w2, residual=h)
+        h = decode_layer.linear_fused(o.view(B, -1), wo, residual=x2)
+        norm = self.ffn_norm
+        n, nw = self._norm_in(h, w1, norm, swiglu=True)
+        g = decode_layer.linear_fused(n, w1, norm_weight=nw, eps=norm.eps, lin_b=w3)
+        y = decode_layer.linear_fused(g, w2, residual=h)
         return y.view(B, 1, dim)
 
 

@@ -16,6 +16,8 @@ slices.
 """
 from __future__ import annotations
 
+import ctypes
+
 import torch
 import torch.nn as nn
 
@@ -147,7 +149,6 @@ def w8a16_small_gemm(x, mats, *, residual=None, swiglu: bool = False):
     pairs) in one launch -> [y_i [M, N_i]]; with ``residual`` [M, N] (one pair)
     [residual + y]; with ``swiglu`` (two pairs) [silu(y_0) * y_1].  One matrix
     with a long K splits it and takes a second launch."""
-    import ctypes
     prepped = [_prep(x, w, s) for w, s in mats]
     x = prepped[0][0]
     if x.stride(1) != 1:
@@ -171,15 +172,16 @@ def w8a16_small_gemm(x, mats, *, residual=None, swiglu: bool = False):
         S = lib.mi_w8a16_small_gemm_splits(M, prepped[0][1].shape[0], K)
         if S > 1:
             part = torch.empty(S * M * prepped[0][1].shape[0], device=x.device, dtype=torch.float32)
-    P = ctypes.c_void_p * n
-    I = ctypes.c_int64 * n
     ys = outs * n if swiglu else outs
-    arrays = (P(*[w.data_ptr() for _, w, _ in prepped]), P(*[s.data_ptr() for _, _, s in prepped]),
-              P(*[y.data_ptr() for y in ys]), I(*[w.shape[0] for _, w, _ in prepped]),
-              I(*[w.stride(0) for _, w, _ in prepped]), I(*[s.stride(0) for _, _, s in prepped]),
-              I(*[y.stride(0) for y in ys]))
+    # the library's seven host arrays (w, scales, y, N, row and scale strides) in one
+    arrays = (ctypes.c_int64 * (7 * n))(
+        *[w.data_ptr() for _, w, _ in prepped], *[s.data_ptr() for _, _, s in prepped],
+        *[y.data_ptr() for y in ys], *[w.shape[0] for _, w, _ in prepped],
+        *[w.stride(0) for _, w, _ in prepped], *[s.stride(0) for _, _, s in prepped],
+        *[y.stride(0) for y in ys])
+    at = ctypes.addressof(arrays)
     st = lib.mi_w8a16_small_gemm(
-        x.data_ptr(), M, K, x.stride(0), n, *map(ctypes.addressof, arrays),
+        x.data_ptr(), M, K, x.stride(0), n, *range(at, at + 56 * n, 8 * n),
         2 if swiglu else 0 if residual is None else 1, _lib.ptr(residual),
         0 if residual is None else residual.stride(0), _lib.ptr(part),
         0 if part is None else part.numel(), _lib.dtype_code(x.dtype),
@@ -277,7 +279,6 @@ def w8a16_gemm_multi(x, mats):
     """x [M, K] times each (weight [N_i, K] int8, scales [N_i] or [N_i, 1]) of
     `mats` (1-4 pairs) in one launch -> [y_i [M, N_i]]; each y_i is bitwise
     w8a16_gemm_mfma(x, weight_i, scales_i, splits=1)."""
-    import ctypes
     if not 1 <= len(mats) <= 4:
         raise ValueError(f"w8a16_gemm_multi takes 1-4 matrices, got {len(mats)}")
     prepped = [_prep(x, w, s) for w, s in mats]
