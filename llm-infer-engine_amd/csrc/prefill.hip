@@ -1475,9 +1475,8 @@ __global__ __launch_bounds__(256, 2) void prefill_sp2_kernel(PrefillArgs a) {
   }
 }
 
-// Plain VALU flash attention in fp32 arithmetic: every head dim of fp32
-// inputs (no fp32 MFMA tiles), and head dims 16 and 256 of bf16/fp16 inputs
-// (the MFMA kernels cover 32, 64 and 128).  TPR = D/8 lanes per query row, 8
+// Plain VALU flash attention in fp32 arithmetic: head dims 16 and 256 of fp32
+// inputs and 16 of bf16/fp16 (the MFMA kernels cover the others).  TPR = D/8 lanes per query row, 8
 // dims each (32 rows per 256-thread block at D = 64, 16 at D = 128, so a short
 // sequence still gives the GPU hundreds of blocks and a long row's chain of
 // keys is split over many lanes); K/V tiles converted to fp32 and staged in
@@ -1597,6 +1596,187 @@ __global__ __launch_bounds__(256) void prefill_valu_kernel(PrefillArgs a) {
     a.lse[((int64_t)b * a.Hq + head) * a.S + qrow] = (m + __log2f(l)) * kLn2;
 }
 
+// fp32 at head_dim 32, 64 and 128 on the fp32 matrix instruction
+// (v_mfma_f32_32x32x2_f32: fp32 products and sums, twice the rate of plain
+// FMAs).  A block is 32 query rows of one head; its 4 waves take the 32-key tiles
+// in turn and merge their (m, l, O) in LDS at the end, because a prompt of a few
+// hundred rows has too few row blocks to fill the SIMDs any other way and one
+// tile is 2 D x 64 matrix cycles long.
+//  * S^T = K Q^T: each lane then holds 16 scores of one query (its column), and
+//    accumulator i is key 8 (i / 4) + 4 h + i % 4 for lane half h -- exactly a B
+//    operand of O^T += V^T P^T whose two k slots are those two keys, so P needs
+//    no shuffle and V's lanes read 32 consecutive floats of that key's row.
+//  * K and V come straight from global memory (L2): a tile is 2 D x 64 matrix
+//    cycles against 128 D bytes; V of a tile is requested before its QK products
+//    and K of the next tile before its PV products.
+//  * row blocks are dealt heaviest first, then lightest first, so that a CU's two
+//    blocks add up to the same work.
+// Same online softmax in fp32 as prefill_valu_kernel.  MI355X against that kernel,
+// in a graph: one prompt of 512 rows, 32/8 heads, D = 64: 64.3 -> 23.8 us; 1024
+// rows 230 -> 65; 24/8 heads, D = 128, 512 rows 119 -> 37; 33 rows 7.6 -> 5.8.
+template <int D>
+__global__ __launch_bounds__(256) void prefill_f32_kernel(PrefillArgs a) {
+  constexpr int DH = D / 2, NB = D / 32, DP = D < 64 ? D : 64;   // DP: dims per merge pass
+  __shared__ float s_m[4][32], s_l[4][32];
+  __shared__ __align__(16) float s_o[4][32][DP + 4];
+  const int tid = threadIdx.x, lane = tid & 63, r = lane & 31, h = lane >> 5;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int n_rb = (a.S + 31) / 32, n_bh = a.B * a.Hq;
+  const int ri = (int)(blockIdx.x / n_bh), bh = (int)(blockIdx.x % n_bh);
+  const int heavy = (n_rb + 1) / 2;
+  const int rb = ri < heavy ? n_rb - 1 - ri : ri - heavy;
+  const int head = bh % a.Hq, b = bh / a.Hq, kvh = head / a.G;
+  const float* kb = reinterpret_cast<const float*>(a.k) + (int64_t)b * a.k_sb + (int64_t)kvh * a.k_sh;
+  const float* vb = reinterpret_cast<const float*>(a.v) + (int64_t)b * a.v_sb + (int64_t)kvh * a.v_sh;
+  auto key_of = [&](int i) { return 8 * (i >> 2) + 4 * h + (i & 3); };   // of accumulator i
+
+  // ---- q: lane (r, h) holds dims h D/2 .. of query row r
+  const int qr = min(rb * 32 + r, a.S - 1);
+  const float* qp = reinterpret_cast<const float*>(a.q) + (int64_t)b * a.q_sb +
+                    (int64_t)head * a.q_sh + (int64_t)qr * a.q_ss;
+  f32x4 qv[DH / 4];
+#pragma unroll
+  for (int c = 0; c < DH / 4; ++c) qv[c] = *reinterpret_cast<const f32x4*>(qp + h * DH + 4 * c);
+  if (a.rcos != nullptr) {   // rotation partner of dim d: d + D/2 (or d - D/2), the other half's
+    int64_t crow = qr;
+    if (a.rpos != nullptr) crow = min(max(a.rpos[qr], (int64_t)0), a.r_rows - 1);
+    const float* cp = reinterpret_cast<const float*>(a.rcos) + crow * a.r_ss;
+    const float* sp = reinterpret_cast<const float*>(a.rsin) + crow * a.r_ss;
+#pragma unroll
+    for (int c = 0; c < DH / 4; ++c)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int d = 4 * c + e;
+        const float own = qv[c][e], other = qp[(1 - h) * DH + d];
+        float y1, y2;
+        rope_rotate<float, float>(h ? other : own, h ? own : other, cp[d], sp[d], y1, y2);
+        qv[c][e] = h ? y2 : y1;
+      }
+  }
+
+  f32x16 o[NB];
+#pragma unroll
+  for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) o[nb][i] = 0.f;
+  float m = kNegBig, l = 0.f;
+  f32x4 kv[DH / 4];
+  auto load_k = [&](int t) {   // rows past S clamped: their scores are masked
+    const float* p = kb + (int64_t)min(32 * t + r, a.S - 1) * a.k_ss + h * DH;
+#pragma unroll
+    for (int c = 0; c < DH / 4; ++c) kv[c] = *reinterpret_cast<const f32x4*>(p + 4 * c);
+  };
+  if (w <= rb) load_k(w);
+  for (int t = w; t <= rb; t += 4) {
+    float vv[NB][16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const float* p = vb + (int64_t)min(32 * t + key_of(i), a.S - 1) * a.v_ss + r;
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb) vv[nb][i] = p[32 * nb];
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    // four partial sums of the dims, added pairwise: error of the output against 64
+    // bits at 512 x 64 1.6e-7 (one chain of D products 2.4e-7, the VALU form, whose
+    // lanes sum 8 dims each, 2.2e-7), for 5 to 10 % of the time at D = 64
+    f32x16 s4[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) s4[e][i] = 0.f;
+    }
+#pragma unroll
+    for (int c = 0; c < DH / 4; ++c)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        s4[e] = __builtin_amdgcn_mfma_f32_32x32x2f32(kv[c][e], qv[c][e], s4[e], 0, 0, 0);
+    f32x16 s = (s4[0] + s4[1]) + (s4[2] + s4[3]);
+    if (t + 4 <= rb) load_k(t + 4);
+    __builtin_amdgcn_sched_barrier(0);
+    float mx = kNegBig;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      s[i] *= a.scale_log2;
+      if (t == rb && key_of(i) > r) s[i] = -INFINITY;   // the diagonal tile
+      mx = fmaxf(mx, s[i]);
+    }
+    {
+      const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(mx), __float_as_uint(mx),
+                                                       false, false);
+      mx = fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1]));
+    }
+    const float mn = fmaxf(m, mx), alpha = fast_exp2(m - mn);
+    float ps = 0.f;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      s[i] = fast_exp2(s[i] - mn);
+      ps += s[i];
+    }
+    l = l * alpha + ps;   // this lane half's keys; the halves meet at the end
+    m = mn;
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) o[nb][i] *= alpha;
+#pragma unroll
+      for (int i = 0; i < 16; ++i)
+        o[nb] = __builtin_amdgcn_mfma_f32_32x32x2f32(vv[nb][i], s[i], o[nb], 0, 0, 0);
+    }
+  }
+  {
+    const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(l), __float_as_uint(l), false, false);
+    l = __uint_as_float(sw[0]) + __uint_as_float(sw[1]);
+  }
+  if (h == 0) {
+    s_m[w][r] = m;
+    s_l[w][r] = l;
+  }
+
+  // ---- merge the waves: 8 threads per query row, DP dims per pass
+  const int mr = tid >> 3, mp = tid & 7, mrow = rb * 32 + mr;
+  float wt[4], inv = 0.f;
+#pragma unroll
+  for (int pass = 0; pass < D / DP; ++pass) {
+    if (pass > 0) __syncthreads();
+#pragma unroll
+    for (int nb = 0; nb < DP / 32; ++nb)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const f32x16& v = o[pass * (DP / 32) + nb];
+        *reinterpret_cast<f32x4*>(&s_o[w][r][32 * nb + 8 * g + 4 * h]) =
+            f32x4{v[4 * g], v[4 * g + 1], v[4 * g + 2], v[4 * g + 3]};
+      }
+    __syncthreads();
+    if (pass == 0) {
+      float M = s_m[0][mr], L = 0.f;
+#pragma unroll
+      for (int ww = 1; ww < 4; ++ww) M = fmaxf(M, s_m[ww][mr]);
+#pragma unroll
+      for (int ww = 0; ww < 4; ++ww) {
+        wt[ww] = fast_exp2(s_m[ww][mr] - M);
+        L += wt[ww] * s_l[ww][mr];
+      }
+      inv = 1.0f / L;
+      if (a.lse != nullptr && mp == 0 && mrow < a.S)
+        a.lse[((int64_t)b * a.Hq + head) * a.S + mrow] = (M + __log2f(L)) * kLn2;
+    }
+    if (mrow < a.S) {
+      float* op = reinterpret_cast<float*>(a.o) + (int64_t)b * a.o_sb + (int64_t)head * a.o_sh +
+                  (int64_t)mrow * a.o_ss + pass * DP;
+#pragma unroll
+      for (int c = 0; c < DP / 32; ++c) {
+        const int d = 4 * mp + 32 * c;
+        f32x4 t = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int ww = 0; ww < 4; ++ww) t += wt[ww] * *reinterpret_cast<const f32x4*>(&s_o[ww][mr][d]);
+        t *= inv;
+        *reinterpret_cast<float2*>(op + d) = float2{t[0], t[1]};      // rows are 8-byte aligned
+        *reinterpret_cast<float2*>(op + d + 2) = float2{t[2], t[3]};
+      }
+    }
+  }
+}
+
 namespace {
 
 template <typename T, int D>
@@ -1615,6 +1795,14 @@ hipError_t launch(const PrefillArgs& a, int nwaves, hipStream_t stream) {
   return hipGetLastError();
 }
 
+template <int D>
+hipError_t launch_f32(const PrefillArgs& a, hipStream_t st) {
+  const int64_t nblk = (int64_t)a.B * a.Hq * ((a.S + 31) / 32);
+  if (nblk > INT32_MAX) return hipErrorInvalidConfiguration;
+  hipLaunchKernelGGL((prefill_f32_kernel<D>), dim3((unsigned)nblk), dim3(256), 0, st, a);
+  return hipGetLastError();
+}
+
 // VALU kernel: D/8 lanes per query row, 2048/D rows per 256-thread block.
 template <typename T>
 hipError_t launch_valu(const PrefillArgs& a, int64_t head_dim, hipStream_t st) {
@@ -1622,12 +1810,10 @@ hipError_t launch_valu(const PrefillArgs& a, int64_t head_dim, hipStream_t st) {
   const int64_t nblk = (int64_t)a.B * a.Hq * ((a.S + rows - 1) / rows);
   if (nblk > INT32_MAX) return hipErrorInvalidConfiguration;
   const dim3 grid((unsigned)nblk), block(256);
-  switch (head_dim) {
-    case 16: hipLaunchKernelGGL((prefill_valu_kernel<T, 16>), grid, block, 0, st, a); break;
-    case 32: hipLaunchKernelGGL((prefill_valu_kernel<T, 32>), grid, block, 0, st, a); break;
-    case 64: hipLaunchKernelGGL((prefill_valu_kernel<T, 64>), grid, block, 0, st, a); break;
-    case 128: hipLaunchKernelGGL((prefill_valu_kernel<T, 128>), grid, block, 0, st, a); break;
-    default: hipLaunchKernelGGL((prefill_valu_kernel<T, 256>), grid, block, 0, st, a); break;
+  if (head_dim == 16) {
+    hipLaunchKernelGGL((prefill_valu_kernel<T, 16>), grid, block, 0, st, a);
+  } else if constexpr (sizeof(T) == 4) {   // fp32 at 256: 32 to 128 run prefill_f32_kernel
+    hipLaunchKernelGGL((prefill_valu_kernel<T, 256>), grid, block, 0, st, a);
   }
   return hipGetLastError();
 }
@@ -1752,7 +1938,11 @@ int32_t attn_prefill(const void* q, const void* k, const void* v, void* o, float
   hipError_t e;
   hipStream_t st = (hipStream_t)stream;
   if (dtype == MI_DTYPE_F32 || head_dim == 16) {
-    e = dtype == MI_DTYPE_F32   ? launch_valu<float>(a, head_dim, st)
+    e = dtype == MI_DTYPE_F32
+            ? (head_dim == 32    ? launch_f32<32>(a, st)
+               : head_dim == 64  ? launch_f32<64>(a, st)
+               : head_dim == 128 ? launch_f32<128>(a, st)
+                                 : launch_valu<float>(a, head_dim, st))
         : dtype == MI_DTYPE_BF16 ? launch_valu<bf16_t>(a, head_dim, st)
                                  : launch_valu<f16_t>(a, head_dim, st);
   } else if (dtype == MI_DTYPE_BF16) {
