@@ -368,9 +368,16 @@ extern "C" int64_t mi_decode_default_splits(int64_t batch, int64_t n_heads,
   // B8 Hkv8 D64 at 4097 of 8192 keys, 4 splits 22.9 us vs 8 splits 25.0 us).
   const int64_t row_bytes = 2LL * 2 * head_dim;                            // bf16 K + V
   const int64_t s_bytes = (kv_len * row_bytes + (512 << 10) - 1) / (512 << 10);
-  const int64_t s_cover = (cus + units - 1) / units;                       // one block per CU
+  // one block per CU, but no second split where half the CUs have a block already
+  // (B16 Hkv8 at 1024 keys, D64: 12.0 -> 10.8 us with one split, D128 13.0 -> 11.7)
+  const int64_t s_cover = 2 * units >= cus ? 1 : (cus + units - 1) / units;
   if (s > s_bytes) s = s_bytes > s_cover ? s_bytes : s_cover;
-  const int64_t s_keys = (kv_len + 63) / 64;                               // >= 64 keys a split
+  // >= 128 keys a split, and none up to 256 keys: short splits cost more (partials,
+  // combine) than their parallelism gains.  B1 Hkv8 D64, per call in a graph:
+  // 128 keys 9.3 -> 5.9 us (2 splits -> 1), 256 keys 9.5 -> 7.4 (4 -> 1), 1024
+  // keys 10.6 -> 8.3 (16 -> 8), 2048 keys 10.0 -> 9.1 (32 -> 16); with 64 splits'
+  // worth of keys or more nothing changes
+  const int64_t s_keys = kv_len <= 256 ? 1 : (kv_len + 127) / 128;
   if (s > s_keys) s = s_keys;
   if (s < 1) s = 1;
   if (s > kMaxSplits) s = kMaxSplits;
