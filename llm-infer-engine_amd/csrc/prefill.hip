@@ -59,6 +59,7 @@ struct PrefillArgs {
   int32_t head_chunks;      // G / GH
   int32_t pj;               // 32-row slices per head per block
   int32_t n_pb;             // position blocks (of 32*pj rows)
+  int32_t cus;              // compute units of the device
   float scale_log2;         // sm_scale * log2(e)
   // Optional RoPE of q in the Q prologue (rcos == nullptr: q is used as
   // given).  Rotate-half with the table row rpos[s] (or s when rpos is null)
@@ -69,6 +70,31 @@ struct PrefillArgs {
   int64_t r_ss, r_rows;     // positions are clamped into the table's rows
   int32_t o_line;           // out and its rows are 16-byte aligned (whole-row epilogue)
 };
+
+// Block -> (pair = (batch, kv head, head chunk), position block): all blocks of a
+// pair on one XCD (ids are dealt to the XCDs round-robin) where the pairs divide
+// by 8, heaviest position first.  PAIR (the D = 64 kernel, two blocks per CU): with
+// fewer than three blocks per CU the second one of a CU goes out lightest first,
+// so that the two add up to the same work and stay resident together to the end
+// (a CU with one block left runs at 0.8 of its rate with two); the few past two
+// per CU are the lightest and fill the first free slots.  With more blocks the
+// dispatch itself balances heaviest-first order.  MI355X, 32/8 heads, D = 64: B1
+// S4534 103.9 -> 94.2 us, B2 S2295 56.5 -> 51.6, B4 S1024 27.9 -> 26.4; at D = 128
+// the longest block decides and the order changes nothing (-4 to +1.5 %).
+template <bool PAIR>
+__device__ inline void block_of_grid(const PrefillArgs& a, int& pair, int& pb) {
+  const int n_pairs = a.B * a.Hkv * a.head_chunks, bid = blockIdx.x;
+  const bool by_xcd = (n_pairs & 7) == 0;
+  const int xcd = by_xcd ? bid & 7 : 0, per = by_xcd ? n_pairs >> 3 : n_pairs;
+  const int cus = by_xcd ? a.cus >> 3 : a.cus, n = per * a.n_pb;
+  int s = by_xcd ? bid >> 3 : bid;
+  if (PAIR && n < 3 * cus && s >= cus) {
+    const int end = min(n, 2 * cus);
+    if (s < end) s = cus + end - 1 - s;
+  }
+  pair = xcd * per + s % per;
+  pb = a.n_pb - 1 - s / per;
+}
 
 // RoPE of the Q fragments a lane holds for one 32-row block: chunk c (dims
 // 16c + 8hh .. +7) pairs with chunk c + DC/2 (the same dims + D/2), so every
@@ -191,18 +217,8 @@ __global__ __launch_bounds__(256, prefill_min_blocks<D>()) void prefill_kernel(P
 
   // ---- block -> (batch, kv head, head chunk, position block), heavy first,
   //      all blocks of one (b, kvh, chunk) on one XCD
-  const int n_pairs = a.B * a.Hkv * a.head_chunks;
-  const int bid = blockIdx.x;
-  int pair, pb_rank;
-  if ((n_pairs & 7) == 0) {
-    const int xcd = bid & 7, slot = bid >> 3, ppx = n_pairs >> 3;
-    pair = xcd * ppx + slot % ppx;
-    pb_rank = slot / ppx;
-  } else {
-    pair = bid % n_pairs;
-    pb_rank = bid / n_pairs;
-  }
-  const int pb = a.n_pb - 1 - pb_rank;
+  int pair, pb;
+  block_of_grid<false>(a, pair, pb);
   const int hc = pair % a.head_chunks;
   const int kvh = (pair / a.head_chunks) % a.Hkv;
   const int b = pair / (a.head_chunks * a.Hkv);
@@ -557,18 +573,8 @@ __global__ __launch_bounds__(256, 2) void prefill_sp_kernel(PrefillArgs a) {
 
   // ---- block -> (batch, kv head, head chunk, position block), heavy first,
   //      all blocks of one (b, kvh, chunk) on one XCD
-  const int n_pairs = a.B * a.Hkv * a.head_chunks;
-  const int bid = blockIdx.x;
-  int pair, pb_rank;
-  if ((n_pairs & 7) == 0) {
-    const int xcd = bid & 7, slot = bid >> 3, ppx = n_pairs >> 3;
-    pair = xcd * ppx + slot % ppx;
-    pb_rank = slot / ppx;
-  } else {
-    pair = bid % n_pairs;
-    pb_rank = bid / n_pairs;
-  }
-  const int pb = a.n_pb - 1 - pb_rank;
+  int pair, pb;
+  block_of_grid<true>(a, pair, pb);
   const int hc = pair % a.head_chunks;
   const int kvh = (pair / a.head_chunks) % a.Hkv;
   const int b = pair / (a.head_chunks * a.Hkv);
@@ -1026,18 +1032,8 @@ __global__ __launch_bounds__(256, 2) void prefill_sp2_kernel(PrefillArgs a) {
 
   // ---- block -> (batch, kv head, head chunk, position block), heavy first,
   //      all blocks of one (b, kvh, chunk) on one XCD
-  const int n_pairs = a.B * a.Hkv * a.head_chunks;
-  const int bid = blockIdx.x;
-  int pair, pb_rank;
-  if ((n_pairs & 7) == 0) {
-    const int xcd = bid & 7, slot = bid >> 3, ppx = n_pairs >> 3;
-    pair = xcd * ppx + slot % ppx;
-    pb_rank = slot / ppx;
-  } else {
-    pair = bid % n_pairs;
-    pb_rank = bid / n_pairs;
-  }
-  const int pb = a.n_pb - 1 - pb_rank;
+  int pair, pb;
+  block_of_grid<false>(a, pair, pb);
   const int hc = pair % a.head_chunks;
   const int kvh = (pair / a.head_chunks) % a.Hkv;
   const int b = pair / (a.head_chunks * a.Hkv);
@@ -1925,6 +1921,7 @@ int32_t attn_prefill(const void* q, const void* k, const void* v, void* o, float
   const bool sp = head_dim == 64 && dtype != MI_DTYPE_F32;
   const int rows_per_block = sp ? 64 * pj : 32 * prefill_row_blocks<128>() * pj;
   a.n_pb = (int32_t)((seq_len + rows_per_block - 1) / rows_per_block);
+  a.cus = device_cu_count();
   a.scale_log2 = sm_scale * kLog2e;
   a.rcos = rq.cos; a.rsin = rq.sin; a.rpos = rq.pos;
   a.r_ss = rq.row_stride; a.r_rows = rq.rows;
