@@ -26,7 +26,7 @@ EPI_SWIGLU = 2
 
 
 def weights_of(lin):
-    """(int8 weight [N, K], contiguous scales of N elements) of a W8A16Linear;
+    """(int8 weight [N, K], scales of N elements, as they are stored) of a W8A16Linear;
     such a pair, fetched by the caller once for several uses, is passed through."""
     if type(lin) is tuple:
         return lin
@@ -50,7 +50,9 @@ def supported(M: int, K: int, dtype: torch.dtype, lin, norm_weight=None, *,
         return False
     if not (w.is_contiguous() and w.shape[1] == K and w.data_ptr() % 16 == 0):
         return False
-    if s.dtype != dtype:
+    if s.dtype != dtype or not s.is_contiguous() or s.numel() != w.shape[0]:
+        return False
+    if not (w.is_cuda and s.is_cuda):
         return False
     if swiglu and K > 4096:
         return False
@@ -79,6 +81,8 @@ def linear_fused(x, lin, *, norm_weight=None, eps: float = 0.0, lin_b=None, resi
     y = torch.empty((M, N), device=x.device, dtype=x.dtype)
     if lin_b is not None:
         wb, sb = weights_of(lin_b)
+        if wb.shape != w.shape:
+            raise ValueError(f"SwiGLU weights differ in shape: {tuple(w.shape)} and {tuple(wb.shape)}")
         epi = EPI_SWIGLU
     else:
         wb, sb = None, None

@@ -38,7 +38,8 @@ class QuantizedFeedForward(FeedForward):
         src/model.py:23."""
         x2 = x.reshape(-1, x.shape[-1])
         w1, w3 = self.w1, self.w3
-        if x2.shape[0] <= 16 and _rows_fusable(x2, w1, swiglu=True) and _rows_fusable(x2, w3):
+        if (x2.shape[0] <= 16 and w1.weight.shape == w3.weight.shape
+                and _rows_fusable(x2, w1, swiglu=True) and _rows_fusable(x2, w3)):
             torch.cuda.nvtx.range_push("FFN")
             h = decode_layer.linear_fused(x2, w1, lin_b=w3)
             out = self.down(h.view(*x.shape[:-1], w1.out_features), residual)

@@ -197,6 +197,28 @@ def test_block_of_9_to_16_rows_matches_op_chain(dev, M, dim, Hq, Hkv, D):
     _close(kv[0].v, kv[1].v, 1e-2)
 
 
+@pytest.mark.parametrize("M", [3, 11])
+def test_feed_forward_with_strided_scales(dev, M):
+    """Scales that are a column of a wider tensor (every second element): the
+    fused projections read N consecutive scales, so such a layer is not theirs."""
+    from src import decode_layer
+    from src.model_quantized import QuantizedFeedForward
+    from src.quant_linear import W8A16Linear
+    ff = QuantizedFeedForward(512, 1024, W8A16Linear).to(dev)
+    for i, name in enumerate(("w1", "w2", "w3")):
+        lin = getattr(ff, name)
+        setattr(ff, name, _linear(dev, lin.in_features, lin.out_features, torch.bfloat16, 70 + i))
+    x = randn((M, 512), 73, torch.bfloat16, dev)
+    with torch.no_grad():
+        want = ff(x, residual=x)
+        for lin in (ff.w1, ff.w2, ff.w3):
+            wide = torch.full((lin.out_features, 2), 7.0, device=dev, dtype=torch.bfloat16)
+            wide[:, :1] = lin.scales
+            lin.scales.data = wide[:, :1]
+            assert not decode_layer.supported(M, lin.in_features, torch.bfloat16, lin)
+        _close(ff(x, residual=x), want, 1e-2)
+
+
 def test_unsupported_shapes_are_rejected(dev):
     """K outside the built set, M > 16: the C side refuses (nothing launched)
     and the model-level predicate routes such calls to the op chain."""
