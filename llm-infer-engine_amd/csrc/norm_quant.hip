@@ -8,8 +8,9 @@
 //   amax = max(max_k |w[n,k]|, 1e-12)          (fp32)
 //   s    = round_to_dtype(amax / 127)            (IEEE fp32 divide, RNE)
 //   q    = clamp(rne(w / s), -128, 127) -> int8  (IEEE fp32 divide)
-// Bit-exact with the reference recipe: every step is a correctly rounded IEEE
-// operation (no reciprocal approximations, no contraction).
+// Bit-exact with the reference recipe: every result is that of correctly rounded
+// IEEE operations (quantize_vec_kernel multiplies by 1/s only where that provably
+// rounds to the same integer).
 #include <math.h>
 
 #include "common.hpp"

@@ -572,8 +572,8 @@ __global__ __launch_bounds__(256) void w8a16_splitk_reduce_kernel(GemmArgs a, in
 //  * the two operands use the widening of the large GEMM; their 16-byte chunks are
 //    XOR-swizzled by the row so that an LDS read of 8 rows covers all banks.
 //  * a stage's operands are read from LDS one step ahead of their MFMAs.
-// What bounds it: per 128 k a CU spends about 0.4 us (widening, 24 VALU ops per 16 k
-// of 32 columns, and the barrier) plus 0.17 us per 32-row block (its MFMAs and LDS
+// What bounds it: per 128 k a CU spends about 0.4 us (widening, 12 VALU ops of a wave
+// per 16 k of 32 columns, and the barrier) plus 0.17 us per 32-row block (its MFMAs and LDS
 // reads).  MI355X, per call in a graph over rotating weights, against split K and
 // separate silu and product launches: 300 rows SwiGLU 2 x [8192, 2048] 73.3 -> 30.7 us
 // (655 TFLOP/s), [2048, 8192] + residual 31.9 -> 25.6, [2048, 2048] 21.4 -> 10.6; 48

@@ -5,8 +5,8 @@ src/quant_utils.py:7-36), run by one HIP launch (mi_quantize_int8):
     scale = (amax / 127) rounded to w's dtype        [N, 1]
     q     = clamp(round_half_even(w / scale), -128, 127) as int8
 
-Each step is a correctly rounded IEEE operation, so q and scale are bit-exact
-with the reference's torch recipe.
+Each result is that of correctly rounded IEEE operations, so q and scale are
+bit-exact with the reference's torch recipe.
 """
 from __future__ import annotations
 
