@@ -368,16 +368,21 @@ extern "C" int64_t mi_decode_default_splits(int64_t batch, int64_t n_heads,
   // B8 Hkv8 D64 at 4097 of 8192 keys, 4 splits 22.9 us vs 8 splits 25.0 us).
   const int64_t row_bytes = 2LL * 2 * head_dim;                            // bf16 K + V
   const int64_t s_bytes = (kv_len * row_bytes + (512 << 10) - 1) / (512 << 10);
-  // one block per CU, but no second split where half the CUs have a block already
-  // (B16 Hkv8 at 1024 keys, D64: 12.0 -> 10.8 us with one split, D128 13.0 -> 11.7)
-  const int64_t s_cover = 2 * units >= cus ? 1 : (cus + units - 1) / units;
+  // One block per CU; up to 1024 keys no second split where half the CUs have a block
+  // already (B16 Hkv8 D64, 512 keys 11.4 -> 10.2 us, 1024 keys 12.0 -> 10.8 with one
+  // split; at 1500 keys two splits 15.9 us, one 16.6)
+  const int64_t s_cover =
+      kv_len <= 1024 && 2 * units >= cus ? 1 : (cus + units - 1) / units;
   if (s > s_bytes) s = s_bytes > s_cover ? s_bytes : s_cover;
-  // >= 128 keys a split, and none up to 256 keys: short splits cost more (partials,
-  // combine) than their parallelism gains.  B1 Hkv8 D64, per call in a graph:
-  // 128 keys 9.3 -> 5.9 us (2 splits -> 1), 256 keys 9.5 -> 7.4 (4 -> 1), 1024
-  // keys 10.6 -> 8.3 (16 -> 8), 2048 keys 10.0 -> 9.1 (32 -> 16); with 64 splits'
-  // worth of keys or more nothing changes
-  const int64_t s_keys = kv_len <= 256 ? 1 : (kv_len + 127) / 128;
+  // >= 64 keys a split.  Up to 1024 keys fewer, because short splits cost more there
+  // (partials, combine) than their parallelism gains: one up to 256 keys, 4 up to 512,
+  // 8 up to 1024 (powers of two: 7 splits of 777 keys are slower than 8).  B1 Hkv8 D64,
+  // per call in a graph, against one split per 64 keys: 128 keys 9.9 -> 6.6 us, 256 keys
+  // 10.0 -> 8.3, 300 keys 13.7 -> 10.3, 512 keys 10.4 -> 8.9, 777 keys 15.2 -> 11.0, 1024
+  // keys 11.5 -> 9.1.  Above, half as many lose: 1500 keys 10.9 us with 24 splits, 11.9
+  // with 12; D128, 2048 keys 10.4 us with 32, 11.3 with 16.
+  const int64_t s_keys =
+      kv_len <= 256 ? 1 : kv_len <= 512 ? 4 : kv_len <= 1024 ? 8 : (kv_len + 63) / 64;
   if (s > s_keys) s = s_keys;
   if (s < 1) s = 1;
   if (s > kMaxSplits) s = kMaxSplits;

@@ -100,6 +100,23 @@ def test_split_rules_at_any_head_dim(head_dim):
     assert "head_dim" in _lib.last_error() or "positive" in _lib.last_error()
 
 
+@pytest.mark.parametrize("batch,head_dim,keys,splits", [
+    (1, 64, 128, 1), (1, 64, 256, 1),                    # no split
+    (1, 64, 257, 4), (8, 64, 300, 4), (1, 128, 512, 4),
+    (1, 64, 513, 8), (4, 64, 777, 8), (1, 128, 1024, 8),
+    (1, 64, 1025, 17), (1, 64, 1500, 24), (1, 64, 2048, 32), (1, 128, 2048, 32),   # 64 keys a split
+    (1, 64, 4096, 32), (1, 128, 8192, 32),               # one block per CU
+    (16, 64, 1024, 1), (16, 64, 1500, 2), (16, 64, 2048, 2),   # half the CUs have a block
+])
+def test_default_split_counts(batch, head_dim, keys, splits):
+    """Default splits of 8 KV heads on 256 CUs: few of them up to 1024 keys, one per
+    64 keys above (fewer were slower there: a decode step at 2048 slots keeps the
+    split count, and with it the bits, that it had before the short contexts' rule)."""
+    from src import _lib
+    lib = _lib.load()
+    assert lib.mi_decode_default_splits(batch, 32 if head_dim == 64 else 24, 8, keys, head_dim) == splits
+
+
 def test_rope_kv_append_rejects_out_of_capacity():
     from src import _lib
     lib = _lib.load()
