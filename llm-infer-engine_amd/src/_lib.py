@@ -259,8 +259,13 @@ def ptr(t: torch.Tensor | None) -> int | None:
 
 def stream_of(t: torch.Tensor) -> int:
     """hipStream_t of torch's current stream on t's device (graph-capture aware);
-    the raw handle, without the Stream object around it (4 us less per call)."""
-    return torch._C._cuda_getCurrentRawStream(t.get_device())
+    the raw handle, without the Stream object around it (4 us less per call).  A
+    host tensor has no stream: its index -1 would ask for the current device's, and
+    a kernel would get its host pointer."""
+    index = t.get_device()
+    if index < 0:
+        raise ValueError(f"needs a CUDA tensor, got one on {t.device}")
+    return torch._C._cuda_getCurrentRawStream(index)
 
 
 _ARRIVE: dict[tuple[int, int], int | None] = {}

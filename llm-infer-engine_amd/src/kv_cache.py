@@ -50,6 +50,8 @@ class KVCache:
                              f"[{self.max_batch_size}, {self.n_kv_heads}, *, {self.head_dim}]")
         ck = self.k[layer_idx, :B]
         cv = self.v[layer_idx, :B]
+        for t in (ck, cv, k_val, v_val):
+            _lib.require_device(t, "KVCache write")
         k_val = k_val.to(self.dtype)
         v_val = v_val.to(self.dtype)
         lib = _lib.load()

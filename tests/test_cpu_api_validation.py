@@ -59,6 +59,28 @@ def test_kv_cache_position_errors():
         kv.update_positions(0, torch.zeros(2, dtype=torch.long), _t(1, 1, 1, 32), _t(1, 1, 1, 32))
 
 
+def test_host_tensors_never_reach_a_kernel(monkeypatch):
+    """A host tensor has no stream, and a cache built on the host refuses writes,
+    both before the library is called (it would launch on host pointers)."""
+    from src import _lib
+    from src.config import ModelArgs
+    from src.kv_cache import KVCache
+    kv = KVCache(ModelArgs(dim=64, n_layers=1, n_heads=2, n_kv_heads=1, max_seq_len=8,
+                           device="cpu"), dtype=torch.bfloat16)
+
+    class NoLibrary:
+        def __getattr__(self, name):
+            raise AssertionError(f"{name} called with host pointers")
+
+    monkeypatch.setattr(_lib, "load", NoLibrary)
+    with pytest.raises(ValueError, match="CUDA tensor"):
+        _lib.stream_of(kv.k)
+    with pytest.raises(ValueError, match="requires CUDA tensors"):
+        kv.update(0, 0, _t(1, 1, 2, 32), _t(1, 1, 2, 32))
+    with pytest.raises(ValueError, match="requires CUDA tensors"):
+        kv.update_positions(0, torch.zeros(2, dtype=torch.long), _t(1, 1, 2, 32), _t(1, 1, 2, 32))
+
+
 def test_model_args_defaults_are_llama_3_2_1b():
     from src.config import ModelArgs
     a = ModelArgs()
