@@ -36,6 +36,8 @@ def weights_of(lin):
 
 #: reduction lengths the fused GEMV kernels are built for (K = 512 * waves)
 SUPPORTED_K = (512, 1024, 1536, 2048, 3072, 4096, 6144, 8192)
+#: bytes that x, and a weight matrix, must stay below (the kernels' 32-bit offsets)
+_SPAN = 1 << 31
 
 
 def supported(M: int, K: int, dtype: torch.dtype, lin, norm_weight=None, *,
@@ -48,7 +50,8 @@ def supported(M: int, K: int, dtype: torch.dtype, lin, norm_weight=None, *,
     w, s = weights_of(lin)
     if not (1 <= M <= 16 and K in SUPPORTED_K and w.dtype == torch.int8):
         return False
-    if not (w.is_contiguous() and w.shape[1] == K and w.data_ptr() % 16 == 0):
+    if not (w.is_contiguous() and w.shape[1] == K and w.data_ptr() % 16 == 0
+            and w.numel() < _SPAN):
         return False
     if s.dtype != dtype or not s.is_contiguous() or s.numel() != w.shape[0]:
         return False
@@ -65,9 +68,10 @@ def supported(M: int, K: int, dtype: torch.dtype, lin, norm_weight=None, *,
 
 
 def aligned(x: torch.Tensor) -> bool:
-    """Rows of x [M, K] are unit-stride and 16-byte aligned."""
-    return (x.is_cuda and x.stride(1) == 1 and x.data_ptr() % 16 == 0
-            and (x.stride(0) * x.element_size()) % 16 == 0)
+    """Rows of x [M, K] are unit-stride, 16-byte aligned and span less than 2 GB."""
+    row, size = x.stride(0), x.element_size()
+    return (x.is_cuda and x.stride(1) == 1 and x.data_ptr() % 16 == 0 and (row * size) % 16 == 0
+            and ((x.shape[0] - 1) * row + x.shape[1]) * size < _SPAN)
 
 
 def linear_fused(x, lin, *, norm_weight=None, eps: float = 0.0, lin_b=None, residual=None):

@@ -219,6 +219,29 @@ def test_feed_forward_with_strided_scales(dev, M):
         _close(ff(x, residual=x), want, 1e-2)
 
 
+def test_feed_forward_rows_2gb_apart(dev):
+    """Rows of x (the last position of long sequences, say) or weights that span 2 GB
+    and more: past the fused projections' 32-bit offsets, so not theirs, but served."""
+    from src import decode_layer
+    from src.model_quantized import QuantizedFeedForward
+    from src.quant_linear import W8A16Linear
+    M, K, row = 9, 512, 1 << 27                       # (M - 1) * row * 2 bytes = 2 GiB
+    ff = QuantizedFeedForward(K, 1024, W8A16Linear).to(dev)
+    for i, name in enumerate(("w1", "w2", "w3")):
+        lin = getattr(ff, name)
+        setattr(ff, name, _linear(dev, lin.in_features, lin.out_features, torch.bfloat16, 80 + i))
+    near = randn((M, K), 83, torch.bfloat16, dev)
+    far = torch.empty((M - 1) * row + K, device=dev, dtype=torch.bfloat16).as_strided((M, K), (row, 1))
+    far.copy_(near)
+    assert decode_layer.aligned(near) and decode_layer.aligned(far[:-1]) and not decode_layer.aligned(far)
+    with torch.no_grad():
+        _close(ff(far, residual=far), ff(near, residual=near), 1e-2)
+    scales = torch.ones((1 << 20), device=dev, dtype=torch.bfloat16)
+    weight = torch.empty((1 << 20, 2048), device=dev, dtype=torch.int8)
+    assert not decode_layer.supported(M, 2048, torch.bfloat16, (weight, scales))
+    assert decode_layer.supported(M, 2048, torch.bfloat16, (weight[:-1], scales[:-1]))
+
+
 def test_unsupported_shapes_are_rejected(dev):
     """K outside the built set, M > 16: the C side refuses (nothing launched)
     and the model-level predicate routes such calls to the op chain."""
