@@ -34,7 +34,8 @@ class KVCache:
         self.v = torch.zeros(shape, device=args.device, dtype=self.dtype)
         # slot numbers, for kernels that take a position from device memory: a
         # decode step at a host position reads its entry instead of filling a tensor
-        self.positions = torch.arange(self.max_seq_len, device=args.device, dtype=torch.int64)
+        # (private: the kernels write where its entries say)
+        self._slot_numbers = torch.arange(self.max_seq_len, device=args.device, dtype=torch.int64)
 
     def reset(self):
         self.k.zero_()

@@ -186,8 +186,9 @@ class QuantizedTransformerBlock(TransformerBlock):
                 pos = pos.to(torch.int64)
         else:
             p = int(start_pos)
-            table = getattr(kv_cache, "positions", None)
-            if table is not None and 0 <= p < table.shape[0] and table.device == x.device:
+            table = getattr(kv_cache, "_slot_numbers", None)
+            if (isinstance(table, torch.Tensor) and table.dtype == torch.int64 and table.dim() == 1
+                    and 0 <= p < table.shape[0] and table.device == x.device):
                 pos = table[p:p + 1]
             else:
                 pos = torch.full((1,), p, dtype=torch.int64, device=x.device)

@@ -281,6 +281,33 @@ def test_qkv_position_outside_cache_writes_nothing(dev, Hq, Hkv):
     assert torch.equal(cache.k, k0) and torch.equal(cache.v, v0)
 
 
+def test_decode_at_a_host_position_trusts_no_attribute_of_the_cache(dev):
+    """A cache that keeps something of its own under the name ``positions`` (or no
+    table of slot numbers): the fused block still writes slot start_pos."""
+    from src.config import ModelArgs
+    from src.kv_cache import KVCache
+    from src.model_quantized import build_random_quantized
+    args = ModelArgs(dim=512, n_layers=1, n_heads=8, n_kv_heads=2, vocab_size=1000, hidden_dim=1024,
+                     max_batch_size=2, max_seq_len=32, device=str(dev))
+    model = build_random_quantized(args, seed=3, device=str(dev))
+    toks = torch.randint(0, args.vocab_size, (2, 1), generator=torch.Generator().manual_seed(6)).to(dev)
+    seen = []
+    for change in (None, "positions", "no table", "int32 table"):
+        kv = KVCache(args, dtype=torch.bfloat16)
+        if change == "positions":       # the next free slot of each sequence, say
+            kv.positions = torch.zeros(32, dtype=torch.int64, device=dev)
+        elif change == "no table":
+            del kv._slot_numbers
+        elif change == "int32 table":
+            kv._slot_numbers = kv._slot_numbers.int()
+        with torch.no_grad():
+            logits = model(toks, start_pos=5, kv_cache=kv)
+        assert kv.k[:, :, :, 5].any() and not kv.k[:, :, :, :5].any() and not kv.k[:, :, :, 6:].any()
+        seen.append((logits, kv.k, kv.v))
+    for other in seen[1:]:
+        assert all(torch.equal(a, b) for a, b in zip(seen[0], other))
+
+
 def test_fused_decode_step_matches_unfused(dev):
     """The quantized block's fused single-token path against the op-by-op
     composition of the same model (eager, three decode steps)."""
