@@ -59,12 +59,14 @@ def supported(M: int, K: int, dtype: torch.dtype, lin, norm_weight=None, *,
         return False
     if swiglu and K > 4096:
         return False
-    if norm_weight is not None:
-        if (norm_weight.dtype != dtype or not norm_weight.is_contiguous()
-                or norm_weight.data_ptr() % 16 != 0 or M * K * 2 > 64 * 1024
-                or (M > 8 and K > 2048)):
-            return False
-    return True
+    return norm_weight is None or norm_supported(M, K, dtype, norm_weight)
+
+
+def norm_supported(M: int, K: int, dtype: torch.dtype, norm_weight) -> bool:
+    """Whether the projections' RMSNorm prologue takes [M, K] rows and this weight."""
+    return (norm_weight.dtype == dtype and norm_weight.is_contiguous()
+            and norm_weight.data_ptr() % 16 == 0 and M * K * 2 <= 64 * 1024
+            and (M <= 8 or K <= 2048))
 
 
 def aligned(x: torch.Tensor) -> bool:

@@ -18,12 +18,29 @@ from __future__ import annotations
 
 import torch
 import torch.nn as nn
+from torch.nn.modules import module as _hooks
 
 from . import decode_layer, quant_linear
 from .flash_decode import flash_decode
 from .model import Attention, FeedForward, Llama3, TransformerBlock
 from .quant_linear import W8A16Linear
 from .quant_utils import quantize_weight_symmetric_per_channel
+
+
+def _no_hooks(*modules) -> bool:
+    """Whether a call of these modules is only their class's forward: no forward
+    (pre-)hook, their own or a global one, and no forward set on the instance."""
+    if _hooks._global_forward_hooks or _hooks._global_forward_pre_hooks:
+        return False
+    return not any(m._forward_hooks or m._forward_pre_hooks or "forward" in m.__dict__
+                   for m in modules)
+
+
+def _plain(*lins) -> bool:
+    """Whether projections up to chat-prompt size may run on their weights in one launch:
+    W8A16Linear modules whose call nothing observes or replaces.  (The decode step of
+    the block and prefill-sized GEMMs take the weights without this look.)"""
+    return _no_hooks(*lins) and all(type(m).forward is W8A16Linear.forward for m in lins)
 
 
 class QuantizedFeedForward(FeedForward):
@@ -34,22 +51,23 @@ class QuantizedFeedForward(FeedForward):
         """silu(w1(x)) * w3(x) in one launch (the same rounding points, neither
         projection written out): up to 16 rows in the decode projection
         kernels, prefill-sized inputs in the large GEMM when its tiles fill the
-        GPU and in the small-M GEMM otherwise; other sizes take the op chain of
+        GPU and in the small-M GEMM otherwise; other sizes, and below the large
+        GEMM's sizes projections that are not ``_plain``, take the op chain of
         src/model.py:23."""
         x2 = x.reshape(-1, x.shape[-1])
         w1, w3 = self.w1, self.w3
-        if (x2.shape[0] <= 16 and w1.weight.shape == w3.weight.shape
+        plain = _plain(w1, w3)
+        if (plain and x2.shape[0] <= 16 and w1.weight.shape == w3.weight.shape
                 and _rows_fusable(x2, w1, swiglu=True) and _rows_fusable(x2, w3)):
             torch.cuda.nvtx.range_push("FFN")
             h = decode_layer.linear_fused(x2, w1, lin_b=w3)
             out = self.down(h.view(*x.shape[:-1], w1.out_features), residual)
             torch.cuda.nvtx.range_pop()
             return out
-        mats = [(w1.weight, w1.scales), (w3.weight, w3.scales)]
         if quant_linear.swiglu_worth(x2.shape[0], x2.shape[1], w1.out_features, x.device):
             torch.cuda.nvtx.range_push("FFN")
-            h = quant_linear.w8a16_gemm_swiglu(x2, *mats[0], *mats[1])
-        elif quant_linear.small_gemm_fuses(x2, mats):
+            h = quant_linear.w8a16_gemm_swiglu(x2, w1.weight, w1.scales, w3.weight, w3.scales)
+        elif plain and quant_linear.small_gemm_fuses(x2, mats := _pairs(w1, w3)):
             torch.cuda.nvtx.range_push("FFN")
             h = quant_linear.w8a16_small_gemm(x2, mats, swiglu=True)[0]
         else:
@@ -60,6 +78,10 @@ class QuantizedFeedForward(FeedForward):
 
     def down(self, h, residual=None):
         return _project_residual(self.w2, h, residual)
+
+
+def _pairs(*lins):
+    return [(m.weight, m.scales) for m in lins]
 
 
 def _rows_fusable(x2, lin, *, swiglu=False) -> bool:
@@ -73,21 +95,23 @@ def _project_residual(lin, h, residual):
     """lin(h) + residual with the add in the epilogue of the decode projection
     (up to 16 rows) or of the GEMM (the same roundings as the separate ops);
     otherwise the two ops."""
+    if residual is None:
+        return lin(h)
     h2 = h.reshape(-1, h.shape[-1])
     rows = h2.shape[0]
-    # below GEMM_MIN_ROWS any residual that `residual + out` takes is served: the
-    # fused forms when it has h's dtype and the output's shape, else the two ops
-    plain = (residual is not None and residual.dtype == h.dtype and residual.device == h.device
+    # below GEMM_MIN_ROWS any projection and any residual that `residual + out` takes are
+    # served: the fused forms when the residual has h's dtype and the output's shape,
+    # else the two ops
+    plain = (residual.dtype == h.dtype and residual.device == h.device and _plain(lin)
              and residual.shape == (*h.shape[:-1], lin.out_features))
     if plain and _rows_fusable(h2, lin):
         res2 = residual.reshape(-1, lin.out_features)
         if res2.stride(1) == 1:
             return decode_layer.linear_fused(h2, lin, residual=res2).view(residual.shape)
     gemm = rows >= quant_linear.GEMM_MIN_ROWS
-    small = quant_linear.small_gemm_worth(h2, lin.weight) and (gemm or plain)
-    if residual is None or not (small or quant_linear.gemm_supported(rows, h2.shape[1])):
-        out = lin(h)
-        return out if residual is None else residual + out
+    small = (gemm or plain) and quant_linear.small_gemm_worth(h2, lin.weight)
+    if not (small or quant_linear.gemm_supported(rows, h2.shape[1])):
+        return residual + lin(h)
     res2 = residual.reshape(-1, lin.out_features)
     if small:
         if not gemm:
@@ -108,15 +132,14 @@ class QuantizedAttention(Attention):
     def qkv(self, x):
         """wq, wk and wv in one launch: of the large GEMM (bitwise the three
         separate GEMMs without a K split) when their tiles together fill the
-        GPU, else of the small-M GEMM; sizes neither takes run one W8A16Linear
-        call each."""
+        GPU, else of the small-M GEMM; sizes neither takes, and modules that are
+        not ``_plain`` at the small-M GEMM's, run one W8A16Linear call each."""
         x2 = x.reshape(-1, x.shape[-1])
         mats = (self.wq, self.wk, self.wv)
-        pairs = [(m.weight, m.scales) for m in mats]
         if quant_linear.gemm_multi_worth(x2.shape[0], x2.shape[1],
                                          [m.out_features for m in mats], x.device):
-            ys = quant_linear.w8a16_gemm_multi(x2, pairs)
-        elif quant_linear.small_gemm_fuses(x2, pairs):
+            ys = quant_linear.w8a16_gemm_multi(x2, _pairs(*mats))
+        elif _plain(*mats) and quant_linear.small_gemm_fuses(x2, pairs := _pairs(*mats)):
             ys = quant_linear.w8a16_small_gemm(x2, pairs)
         else:
             return super().qkv(x)
@@ -136,7 +159,10 @@ class QuantizedTransformerBlock(TransformerBlock):
 
     def _fused_weights(self, x, rope_cos, kv_cache, layer_idx, positions, rope_by_position):
         """The block's weights (``decode_layer.weights_of`` pairs of wq, wk, wv, wo,
-        w1, w3, w2) if the fused decode-layer kernels take this call, else None."""
+        w1, w3, w2) and whether the QKV and the SwiGLU projection normalise their rows
+        themselves, if the fused decode-layer kernels take this call, else None.  Rows
+        that need a launch of their own for a norm are taken only where no module's
+        call is observed or replaced."""
         if not self.fused_decode or kv_cache is None or layer_idx is None or x.shape[1] != 1:
             return None
         if positions is not None and not rope_by_position:
@@ -155,29 +181,28 @@ class QuantizedTransformerBlock(TransformerBlock):
               and sup(B, attn.n_heads * attn.head_dim, dt, wo)
               and sup(B, dim, dt, w1, swiglu=True) and sup(B, dim, dt, w3)
               and sup(B, w1[0].shape[0], dt, w2))
-        return ws if ok else None
-
-    @staticmethod
-    def _norm_in(x2, lin, norm, *, swiglu=False):
-        """(rows, norm weight) for a projection of the normalised rows: the
-        projection's own RMSNorm prologue where it takes these sizes, else the
-        rows normalised by a launch of their own and no prologue."""
-        nw = norm.weight
-        if decode_layer.supported(*x2.shape, x2.dtype, lin, nw, swiglu=swiglu):
-            return x2, nw
-        return norm(x2), None
+        if not ok:
+            return None
+        prologue = tuple(decode_layer.norm_supported(B, dim, dt, norm.weight)
+                         for norm in (self.attention_norm, self.ffn_norm))
+        if not all(prologue) and not (
+                _plain(attn.wq, attn.wk, attn.wv, attn.wo, ff.w1, ff.w3, ff.w2)
+                and _no_hooks(attn, ff, self.attention_norm, self.ffn_norm)):
+            return None
+        return ws, prologue
 
     def forward(self, x, rope_cos, rope_sin, layer_idx=None, start_pos=0, kv_cache=None,
                 use_cuda_graph=False, scatter_positions=None, decode_attn_mask=None, **ext):
         positions = scatter_positions if (use_cuda_graph and scatter_positions is not None) else None
         by_pos = bool(ext.get("rope_by_position", False))
-        ws = self._fused_weights(x, rope_cos, kv_cache, layer_idx, positions, by_pos)
-        if ws is None:
+        fused = self._fused_weights(x, rope_cos, kv_cache, layer_idx, positions, by_pos)
+        if fused is None:
             return super().forward(x, rope_cos, rope_sin, layer_idx=layer_idx, start_pos=start_pos,
                                    kv_cache=kv_cache, use_cuda_graph=use_cuda_graph,
                                    scatter_positions=scatter_positions,
                                    decode_attn_mask=decode_attn_mask, **ext)
-        wq, _, _, wo, w1, w3, w2 = ws
+        ws, (qkv_norms, ffn_norms) = fused
+        wo, w1, w3, w2 = ws[3:]
         B, _, dim = x.shape
         x2 = x.view(B, dim)
         if positions is not None:  # graph path: device position, full-table RoPE rows
@@ -194,7 +219,7 @@ class QuantizedTransformerBlock(TransformerBlock):
                 pos = torch.full((1,), p, dtype=torch.int64, device=x.device)
             row0 = 0 if by_pos else p
         norm = self.attention_norm
-        h, nw = self._norm_in(x2, wq, norm)
+        h, nw = (x2, norm.weight) if qkv_norms else (norm(x2), None)
         q = decode_layer.qkv_rope_append(h, self.attention, nw, norm.eps, rope_cos, rope_sin,
                                          row0, pos, kv_cache, layer_idx, weights=ws[:3])
         ck, cv = kv_cache.k[layer_idx, :B], kv_cache.v[layer_idx, :B]
@@ -203,7 +228,7 @@ class QuantizedTransformerBlock(TransformerBlock):
         o = flash_decode(q, ck, cv, mask=decode_attn_mask, seq_lens=ext.get("seq_lens"))
         h = decode_layer.linear_fused(o.view(B, -1), wo, residual=x2)
         norm = self.ffn_norm
-        n, nw = self._norm_in(h, w1, norm, swiglu=True)
+        n, nw = (h, norm.weight) if ffn_norms else (norm(h), None)
         g = decode_layer.linear_fused(n, w1, norm_weight=nw, eps=norm.eps, lin_b=w3)
         y = decode_layer.linear_fused(g, w2, residual=h)
         return y.view(B, 1, dim)

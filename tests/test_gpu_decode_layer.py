@@ -242,6 +242,75 @@ def test_feed_forward_rows_2gb_apart(dev):
     assert decode_layer.supported(M, 2048, torch.bfloat16, (weight[:-1], scales[:-1]))
 
 
+def _watched_block(dev, dim, M, S):
+    """A quantized block, its rope rows, a cache and x [M, S, dim]."""
+    from src.config import ModelArgs
+    from src.kv_cache import KVCache
+    from src.model_quantized import build_random_quantized
+    from src.rope import DeviceRopeTable
+    args = ModelArgs(dim=dim, n_layers=1, n_heads=dim // 128, n_kv_heads=2, vocab_size=64,
+                     hidden_dim=1024, max_batch_size=M, max_seq_len=64, device=str(dev))
+    block = build_random_quantized(args, seed=3, device=str(dev)).layers[0]
+    rope = DeviceRopeTable(orope.freqs_cis(128, 64, 500000.0), torch.bfloat16, dev).rows(0, S)
+    x = randn((M, S, dim), 90, torch.bfloat16, dev)
+    return block, rope, KVCache(args, dtype=torch.bfloat16), x
+
+
+# chat prompts and feed-forwards of up to 16 rows, decode past the RMSNorm prologue
+@pytest.mark.parametrize("dim,M,S", [(1024, 2, 4), (1024, 1, 24), (1024, 3, 40), (3072, 9, 1)])
+def test_hooks_of_the_projections_fire(dev, dim, M, S):
+    """Every projection and norm of a block called at these sizes is called as a
+    module where a hook watches it; hooked and plain calls agree.  (From 33 rows wo
+    and w2 add the residual in the GEMM, hook or not.)"""
+    block, rope, kv, x = _watched_block(dev, dim, M, S)
+    names = ("attention.wq", "attention.wk", "attention.wv", "attention.wo", "feed_forward.w1",
+             "feed_forward.w2", "feed_forward.w3", "attention_norm", "ffn_norm")
+    if M * S >= 33:
+        names = tuple(n for n in names if not n.endswith(("wo", "w2")))
+    with torch.no_grad():
+        want = block(x, *rope, layer_idx=0, start_pos=0, kv_cache=kv)
+        fired = []
+        handles = [block.get_submodule(n).register_forward_hook(lambda m, i, o, n=n: fired.append(n))
+                   for n in names]
+        got = block(x, *rope, layer_idx=0, start_pos=0, kv_cache=kv)
+        for h in handles:
+            h.remove()
+        assert sorted(fired) == sorted(names)
+        _close(got, want, 1e-2)
+        again = block(x, *rope, layer_idx=0, start_pos=0, kv_cache=kv)
+        assert torch.equal(again, want) and len(fired) == len(names)
+
+
+@pytest.mark.parametrize("rows", [3, 12, 24])
+def test_replaced_projections_are_called(dev, rows):
+    """A projection swapped for another module (one without int8 weights), or with its
+    forward replaced on the instance, is called: its weights are not read around it."""
+    block, _, _, _ = _watched_block(dev, 1024, 1, 1)
+    ff, attn = block.feed_forward, block.attention
+    x = randn((rows, 1024), 91, torch.bfloat16, dev)
+
+    class Dense(torch.nn.Module):            # no weight, scales or out_features of its own
+        def __init__(self, lin):
+            super().__init__()
+            self.dense = (lin.weight.float() * lin.scales.float()).to(torch.bfloat16)
+
+        def forward(self, x):
+            return x @ self.dense.t()
+
+    with torch.no_grad():
+        want = ff(x, residual=x), attn.out_proj(x, x)
+        for name in ("w1", "w2", "w3"):
+            lin = getattr(ff, name)
+            lin.forward = Dense(lin).forward
+        attn.wo = Dense(attn.wo)
+        ff.w2 = Dense(ff.w2)
+        got = ff(x, residual=x), attn.out_proj(x, x)
+        for a, b in zip(got, want):
+            _close(a, b, 2e-2)
+        ff.w1.forward = lambda x: torch.zeros((rows, 1024), device=dev, dtype=x.dtype)
+        assert torch.equal(ff(x, residual=x), x)         # silu(0) * w3(x) = 0
+
+
 def test_unsupported_shapes_are_rejected(dev):
     """K outside the built set, M > 16: the C side refuses (nothing launched)
     and the model-level predicate routes such calls to the op chain."""
