@@ -157,12 +157,13 @@ class QuantizedTransformerBlock(TransformerBlock):
     def __init__(self, args, linear=W8A16Linear):
         super().__init__(args, W8A16Linear)
 
-    def _fused_weights(self, x, rope_cos, kv_cache, layer_idx, positions, rope_by_position):
+    def _fused_weights(self, x, rope_cos, rope_sin, kv_cache, layer_idx, positions,
+                       rope_by_position, start_pos):
         """The block's weights (``decode_layer.weights_of`` pairs of wq, wk, wv, wo,
         w1, w3, w2) and whether the QKV and the SwiGLU projection normalise their rows
         themselves, if the fused decode-layer kernels take this call, else None.  Rows
-        that need a launch of their own for a norm are taken only where no module's
-        call is observed or replaced."""
+        that need a launch of their own for a norm are taken only at a position inside
+        the cache and where no module's call is observed or replaced."""
         if not self.fused_decode or kv_cache is None or layer_idx is None or x.shape[1] != 1:
             return None
         if positions is not None and not rope_by_position:
@@ -174,19 +175,31 @@ class QuantizedTransformerBlock(TransformerBlock):
                 or rope_cos.dtype != dt or attn.head_dim % 16 != 0 or not x.is_contiguous()
                 or not decode_layer.aligned(x.view(B, dim))):
             return None
+        if (rope_cos.stride(1) != 1 or rope_cos.stride() != rope_sin.stride()
+                or rope_sin.dtype != dt or rope_sin.shape[0] != rope_cos.shape[0]
+                or kv_cache.v.dtype != dt or kv_cache.k.stride(4) != 1
+                or kv_cache.k.stride() != kv_cache.v.stride()):
+            return None  # the kernels take one set of strides for each pair
         ws = tuple(map(decode_layer.weights_of,
                        (attn.wq, attn.wk, attn.wv, attn.wo, ff.w1, ff.w3, ff.w2)))
         wq, wk, wv, wo, w1, w3, w2 = ws
-        ok = (sup(B, dim, dt, wq) and sup(B, dim, dt, wk) and sup(B, dim, dt, wv)
-              and sup(B, attn.n_heads * attn.head_dim, dt, wo)
+        n_q, n_kv = attn.n_heads * attn.head_dim, attn.n_kv_heads * attn.head_dim
+        # (rows first: the kernels read as many as the heads and the residual have)
+        ok = (wq[0].shape[0] == n_q and wk[0].shape[0] == wv[0].shape[0] == n_kv
+              and wo[0].shape[0] == w2[0].shape[0] == dim
+              and sup(B, dim, dt, wq) and sup(B, dim, dt, wk) and sup(B, dim, dt, wv)
+              and sup(B, n_q, dt, wo)
               and sup(B, dim, dt, w1, swiglu=True) and sup(B, dim, dt, w3)
               and sup(B, w1[0].shape[0], dt, w2))
         if not ok:
             return None
         prologue = tuple(decode_layer.norm_supported(B, dim, dt, norm.weight)
                          for norm in (self.attention_norm, self.ffn_norm))
+        # past the prologue the op chain served (and at a position outside the cache
+        # refused) these rows: it still does where a module's call is observed
         if not all(prologue) and not (
-                _plain(attn.wq, attn.wk, attn.wv, attn.wo, ff.w1, ff.w3, ff.w2)
+                (positions is not None or 0 <= int(start_pos) < kv_cache.k.shape[3])
+                and _plain(attn.wq, attn.wk, attn.wv, attn.wo, ff.w1, ff.w3, ff.w2)
                 and _no_hooks(attn, ff, self.attention_norm, self.ffn_norm)):
             return None
         return ws, prologue
@@ -195,7 +208,8 @@ class QuantizedTransformerBlock(TransformerBlock):
                 use_cuda_graph=False, scatter_positions=None, decode_attn_mask=None, **ext):
         positions = scatter_positions if (use_cuda_graph and scatter_positions is not None) else None
         by_pos = bool(ext.get("rope_by_position", False))
-        fused = self._fused_weights(x, rope_cos, kv_cache, layer_idx, positions, by_pos)
+        fused = self._fused_weights(x, rope_cos, rope_sin, kv_cache, layer_idx, positions,
+                                    by_pos, start_pos)
         if fused is None:
             return super().forward(x, rope_cos, rope_sin, layer_idx=layer_idx, start_pos=start_pos,
                                    kv_cache=kv_cache, use_cuda_graph=use_cuda_graph,
@@ -207,8 +221,8 @@ class QuantizedTransformerBlock(TransformerBlock):
         x2 = x.view(B, dim)
         if positions is not None:  # graph path: device position, full-table RoPE rows
             pos, row0 = positions, 0
-            if pos.dtype != torch.int64:
-                pos = pos.to(torch.int64)
+            if pos.dtype != torch.int64 or pos.device != x.device:
+                pos = pos.to(device=x.device, dtype=torch.int64)
         else:
             p = int(start_pos)
             table = getattr(kv_cache, "_slot_numbers", None)

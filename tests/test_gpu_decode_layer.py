@@ -311,6 +311,53 @@ def test_replaced_projections_are_called(dev, rows):
         assert torch.equal(ff(x, residual=x), x)         # silu(0) * w3(x) = 0
 
 
+# rows of the RMSNorm prologue and past it
+@pytest.mark.parametrize("dim,M", [(1024, 3), (3072, 9)])
+def test_decode_tables_and_caches_of_other_layouts(dev, dim, M):
+    """RoPE tables that are every second column of a wider one, a cache whose V has
+    other strides than its K, and a position tensor on the host: the same step."""
+    block, (cos, sin), kv, x = _watched_block(dev, dim, M, 1)
+    other = _watched_block(dev, dim, M, 1)[2]
+    other.v = torch.zeros([other.v.shape[i] for i in (0, 1, 3, 2, 4)], device=dev,
+                          dtype=torch.bfloat16).transpose(2, 3)
+    wide = [torch.full((1, 128), 9.0, device=dev, dtype=torch.bfloat16) for _ in range(2)]
+    for w, t in zip(wide, (cos, sin)):
+        w[:, ::2] = t
+    full = [t.repeat(64, 1) for t in (cos, sin)]
+    with torch.no_grad():
+        want = block(x, cos, sin, layer_idx=0, start_pos=7, kv_cache=kv)
+        kv.reset()
+        got = block(x, wide[0][:, ::2], wide[1][:, ::2], layer_idx=0, start_pos=7, kv_cache=kv)
+        _close(got, want, 1e-2)
+        _close(block(x, cos, sin, layer_idx=0, start_pos=7, kv_cache=other), want, 1e-2)
+        _close(other.k, kv.k, 1e-2)
+        _close(other.v, kv.v, 1e-2)
+        kv.reset()
+        lens = torch.full((M,), 8, dtype=torch.int64, device=dev)
+        got = block(x, *full, layer_idx=0, kv_cache=kv, use_cuda_graph=True, rope_by_position=True,
+                    scatter_positions=torch.tensor([7]), seq_lens=lens)
+        _close(got, want, 1e-2)
+
+
+def test_decode_past_the_cache_is_refused_past_the_prologue(dev):
+    """9 rows of 3072: a host position outside the cache raises, as the op chain does."""
+    block, rope, kv, x = _watched_block(dev, 3072, 9, 1)
+    with torch.no_grad(), pytest.raises(ValueError, match="capacity"):
+        block(x, *rope, layer_idx=0, start_pos=64, kv_cache=kv)
+    assert not kv.k.any() and not kv.v.any()
+
+
+def test_decode_weights_of_other_heads_are_refused(dev):
+    """Projections with fewer rows than the heads, or than the residual: refused, not read past."""
+    for name, rows in (("wk", 128), ("wo", 512)):
+        block, rope, kv, x = _watched_block(dev, 1024, 3, 1)
+        lin = getattr(block.attention, name)
+        lin.weight.data, lin.scales.data = lin.weight[:rows].clone(), lin.scales[:rows].clone()
+        lin.out_features = rows
+        with torch.no_grad(), pytest.raises((RuntimeError, ValueError)):
+            block(x, *rope, layer_idx=0, start_pos=7, kv_cache=kv)
+
+
 def test_unsupported_shapes_are_rejected(dev):
     """K outside the built set, M > 16: the C side refuses (nothing launched)
     and the model-level predicate routes such calls to the op chain."""
