@@ -240,7 +240,10 @@ def small_gemm_worth(x, weight) -> bool:
     more rows than the decode kernels take, and a grid of 128 x 256 tiles that
     leaves three CUs in ten idle or more.  Measured at both sides: N = 2048, M =
     2048 (128 tiles of 256 CUs) 26 us against 43 (K = 2048), 79 against 92 (K =
-    8192); N = 3072, M = 2048 (192 tiles) 62 against 54 and 147 against 133."""
+    8192); N = 3072, M = 2048 (192 tiles) 62 against 54 and 147 against 133.
+    Operands that ``_prep`` refuses (host tensors, other ranks) are left to it."""
+    if not x.is_cuda or x.dim() != 2 or weight.dim() != 2:
+        return False
     M, K = x.shape
     if not _small_gemm_takes(M, K):
         return False

@@ -107,6 +107,17 @@ def test_small_m_w8a16_routing_rule():
     assert not _fused_gemv_ok(torch.zeros(2048, 8, dtype=torch.bfloat16).t(), w, s)  # k stride
 
 
+@pytest.mark.parametrize("rows", [4, 12, 20, 40, 3000])
+def test_w8a16_linear_refuses_host_tensors_and_ranks(rows):
+    """An AssertionError at every row count, with or without a GPU in the machine."""
+    from src.quant_linear import W8A16Linear, w8a16_gemm_launch
+    lin = W8A16Linear(2048, 512)
+    with pytest.raises(AssertionError):
+        lin(_t(rows, 2048))
+    with pytest.raises(AssertionError):
+        w8a16_gemm_launch(_t(2, rows, 2048), lin.weight, lin.scales)
+
+
 @pytest.mark.parametrize("shape,layer,msg", [
     ((3, 2, 1, 16), 0, "does not fit the cache"),     # batch above max_batch_size
     ((2, 3, 1, 16), 0, "does not fit the cache"),     # more kv heads than the cache
