@@ -1592,6 +1592,49 @@ __global__ __launch_bounds__(256) void prefill_valu_kernel(PrefillArgs a) {
     a.lse[((int64_t)b * a.Hq + head) * a.S + qrow] = (m + __log2f(l)) * kLn2;
 }
 
+// Whether x is an infinity or a NaN, from its bits: this file is built as if no float
+// were a NaN, and a test of the float itself would be folded accordingly.
+__device__ inline bool not_finite(float x) {
+  uint32_t bits = __float_as_uint(x);
+  asm("" : "+v"(bits));
+  return (bits & 0x7f800000u) == 0x7f800000u;
+}
+
+// sum over keys 0..row of exp2(score - M) V[key][d .. d+3] in plain fp32 FMAs (before
+// the division by the row's sum), for an output whose V holds infinities or NaNs.
+template <int D>
+__device__ inline f32x4 visible_keys_f32(const PrefillArgs& a, int b, int head,
+                                         int kvh, int row, int d, float M) {
+  const float* qp = reinterpret_cast<const float*>(a.q) + (int64_t)b * a.q_sb +
+                    (int64_t)head * a.q_sh + (int64_t)row * a.q_ss;
+  const float* kb = reinterpret_cast<const float*>(a.k) + (int64_t)b * a.k_sb + (int64_t)kvh * a.k_sh;
+  const float* vb = reinterpret_cast<const float*>(a.v) + (int64_t)b * a.v_sb +
+                    (int64_t)kvh * a.v_sh + d;
+  int64_t crow = row;
+  if (a.rcos != nullptr && a.rpos != nullptr) crow = min(max(a.rpos[row], (int64_t)0), a.r_rows - 1);
+  f32x4 t = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+  for (int key = 0; key <= row; ++key) {
+    const float* kr = kb + (int64_t)key * a.k_ss;
+    float s1 = 0.f, s2 = 0.f;
+#pragma unroll 1
+    for (int i = 0; i < D / 2; ++i) {
+      float y1 = qp[i], y2 = qp[i + D / 2];
+      if (a.rcos != nullptr)
+        rope_rotate<float, float>(qp[i], qp[i + D / 2],
+                                  reinterpret_cast<const float*>(a.rcos)[crow * a.r_ss + i],
+                                  reinterpret_cast<const float*>(a.rsin)[crow * a.r_ss + i], y1, y2);
+      s1 = fmaf(y1, kr[i], s1);
+      s2 = fmaf(y2, kr[i + D / 2], s2);
+    }
+    const float p = fast_exp2((s1 + s2) * a.scale_log2 - M);
+    const f32x4 v = *reinterpret_cast<const f32x4*>(vb + (int64_t)key * a.v_ss);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) t[e] = fmaf(p, v[e], t[e]);
+  }
+  return t;
+}
+
 // fp32 at head_dim 32, 64 and 128 on the fp32 matrix instruction
 // (v_mfma_f32_32x32x2_f32: fp32 products and sums, twice the rate of plain
 // FMAs).  A block is 32 query rows of one head; its 4 waves take the 32-key tiles
@@ -1730,7 +1773,7 @@ __global__ __launch_bounds__(256) void prefill_f32_kernel(PrefillArgs a) {
 
   // ---- merge the waves: 8 threads per query row, DP dims per pass
   const int mr = tid >> 3, mp = tid & 7, mrow = rb * 32 + mr;
-  float wt[4], inv = 0.f;
+  float wt[4], M = 0.f, inv = 0.f, chk = 0.f;
 #pragma unroll
   for (int pass = 0; pass < D / DP; ++pass) {
     if (pass > 0) __syncthreads();
@@ -1744,7 +1787,8 @@ __global__ __launch_bounds__(256) void prefill_f32_kernel(PrefillArgs a) {
       }
     __syncthreads();
     if (pass == 0) {
-      float M = s_m[0][mr], L = 0.f;
+      float L = 0.f;
+      M = s_m[0][mr];
 #pragma unroll
       for (int ww = 1; ww < 4; ++ww) M = fmaxf(M, s_m[ww][mr]);
 #pragma unroll
@@ -1766,9 +1810,24 @@ __global__ __launch_bounds__(256) void prefill_f32_kernel(PrefillArgs a) {
 #pragma unroll
         for (int ww = 0; ww < 4; ++ww) t += wt[ww] * *reinterpret_cast<const f32x4*>(&s_o[ww][mr][d]);
         t *= inv;
+        chk += (t[0] + t[1]) + (t[2] + t[3]);
         *reinterpret_cast<float2*>(op + d) = float2{t[0], t[1]};      // rows are 8-byte aligned
         *reinterpret_cast<float2*>(op + d + 2) = float2{t[2], t[3]};
       }
+    }
+  }
+  // The diagonal tile multiplies hidden keys by 0, and 0 times an infinity or a NaN in
+  // V is a NaN: outputs that came out so (with sound weights) are added up once more,
+  // over their visible keys alone.
+  if (not_finite(chk) && !not_finite(inv)) {
+    float* op = reinterpret_cast<float*>(a.o) + (int64_t)b * a.o_sb + (int64_t)head * a.o_sh +
+                (int64_t)mrow * a.o_ss;
+#pragma unroll 1
+    for (int d = 4 * mp; d < D; d += 32) {
+      const f32x4 t = visible_keys_f32<D>(a, b, head, kvh, mrow, d, M);
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (not_finite(op[d + e])) op[d + e] = t[e] * inv;
     }
   }
 }

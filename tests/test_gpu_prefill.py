@@ -115,6 +115,38 @@ def test_config1_rope_prefill_fp32(dev):
     assert max_abs(lse, ref_lse) < 1e-3
 
 
+@pytest.mark.parametrize("D", [32, 64, 128])
+def test_fp32_prefill_with_non_finite_values(dev, D):
+    """An infinity or a NaN in V reaches the rows that see its key and no earlier one
+    (their weights are 0 for it, and 0 x inf is NaN), in every place of a 32-key tile
+    and in the last row, which stands in for the keys past it."""
+    Hq, Hkv, S = 4, 2, 201
+    q = randn((1, Hq, S, D), 60, torch.float32)
+    k = randn((1, Hkv, S, D), 61, torch.float32)
+    v = randn((1, Hkv, S, D), 62, torch.float32)
+    bad = {(0, 40, 5): math.inf, (0, 95, 9): -math.inf, (0, S - 1, 0): math.nan,
+           (1, 160, 7): math.nan, (1, 191, 7): math.inf, (1, S - 1, D - 1): math.inf}
+    ref, ref_lse = ora.prefill(q, k, v)
+    for (h, key, d), value in bad.items():
+        v[0, h, key, d] = value
+        for qh in range(h * Hq // Hkv, (h + 1) * Hq // Hkv):
+            ref[0, qh, key:, d] = math.nan if ref[0, qh, -1, d].isnan() else value
+    out, lse = _fa()(q.to(dev), k.to(dev), v.to(dev), return_lse=True)
+    out = out.cpu()
+    assert torch.equal(out.isnan(), ref.isnan()) and torch.equal(out.isinf(), ref.isinf())
+    finite = ref.isfinite()
+    assert max_abs(out[finite], ref[finite]) < TOL[torch.float32]
+    assert torch.equal(out[ref.isinf()], ref[ref.isinf()].float()) and max_abs(lse, ref_lse) < 1e-3
+    # with q's RoPE fused: the same as rotating by hand
+    from src.rope import apply_rotary
+    cos, sin = _rope_tables(D, S, torch.float32, dev)
+    args = k.to(dev), v.to(dev)
+    fused = _fa()(q.to(dev), *args, rope_cos=cos, rope_sin=sin)
+    assert torch.equal(fused.isfinite().cpu(), finite)
+    hand = _fa()(apply_rotary(q.to(dev), cos, sin), *args)
+    assert torch.equal(fused.nan_to_num(), hand.nan_to_num())
+
+
 def test_config2_full_size(dev):
     """bf16 B4 S2048 32/8 D64, seed 0, Q pre-scaled by 1/8
     and sm_scale=1 (the softmax scale folded into Q; exact for D=64)."""
