@@ -1472,7 +1472,8 @@ __global__ __launch_bounds__(256, 2) void prefill_sp2_kernel(PrefillArgs a) {
 }
 
 // Plain VALU flash attention in fp32 arithmetic: head dims 16 and 256 of fp32
-// inputs and 16 of bf16/fp16 (the MFMA kernels cover the others).  TPR = D/8 lanes per query row, 8
+// inputs, 16 of bf16/fp16 and short fp32 prompts at 64 and 128 (f32_matrix_kernel);
+// the MFMA kernels cover the others.  TPR = D/8 lanes per query row, 8
 // dims each (32 rows per 256-thread block at D = 64, 16 at D = 128, so a short
 // sequence still gives the GPU hundreds of blocks and a long row's chain of
 // keys is split over many lanes); K/V tiles converted to fp32 and staged in
@@ -1858,6 +1859,23 @@ hipError_t launch_f32(const PrefillArgs& a, hipStream_t st) {
   return hipGetLastError();
 }
 
+// Whether fp32 prompts of these sizes run prefill_f32_kernel; else the VALU kernel.
+// A block of the former pads its rows to 32 and has a CU to itself, so a short prompt
+// pays for rows that are not there, and twice once its blocks outnumber the CUs; the
+// VALU kernel packs 32 (D = 64) or 16 (D = 128) rows a block, several to a CU.
+// MI355X, VALU against matrix kernel, per call in a graph: D = 128, 24 heads, 16 rows
+// 5.4 / 9.3 us, 48 rows 9.1 / 10.3, 64 rows 10.5 / 10.8, 65 rows 12.7 / 10.8; 4 prompts
+// of 80 rows (288 blocks) 15.2 / 18.8, of 96 rows 20.3 / 18.9.  D = 64, 32 heads, 32
+// rows 6.2 / 6.6, 33 rows 8.4 / 6.6; 12 and 16 prompts of 48 rows (768, 1024 blocks) 17
+// to 20 % less, of 65 rows 6 % more.  D = 32: the matrix kernel at any length.
+bool f32_matrix_kernel(const PrefillArgs& a, int64_t head_dim) {
+  if (head_dim == 32) return true;
+  const bool many = (int64_t)a.B * a.Hq * ((a.S + 31) / 32) > a.cus;
+  if (head_dim == 64) return a.S > (many ? 64 : 32);
+  if (head_dim == 128) return a.S > 48 && !(many && a.S > 64 && a.S <= 80);
+  return false;
+}
+
 // VALU kernel: D/8 lanes per query row, 2048/D rows per 256-thread block.
 template <typename T>
 hipError_t launch_valu(const PrefillArgs& a, int64_t head_dim, hipStream_t st) {
@@ -1867,8 +1885,12 @@ hipError_t launch_valu(const PrefillArgs& a, int64_t head_dim, hipStream_t st) {
   const dim3 grid((unsigned)nblk), block(256);
   if (head_dim == 16) {
     hipLaunchKernelGGL((prefill_valu_kernel<T, 16>), grid, block, 0, st, a);
-  } else if constexpr (sizeof(T) == 4) {   // fp32 at 256: 32 to 128 run prefill_f32_kernel
-    hipLaunchKernelGGL((prefill_valu_kernel<T, 256>), grid, block, 0, st, a);
+  } else if constexpr (sizeof(T) == 4) {   // the other head dims of fp32 that come here
+    switch (head_dim) {
+      case 64: hipLaunchKernelGGL((prefill_valu_kernel<T, 64>), grid, block, 0, st, a); break;
+      case 128: hipLaunchKernelGGL((prefill_valu_kernel<T, 128>), grid, block, 0, st, a); break;
+      default: hipLaunchKernelGGL((prefill_valu_kernel<T, 256>), grid, block, 0, st, a); break;
+    }
   }
   return hipGetLastError();
 }
@@ -1995,10 +2017,10 @@ int32_t attn_prefill(const void* q, const void* k, const void* v, void* o, float
   hipStream_t st = (hipStream_t)stream;
   if (dtype == MI_DTYPE_F32 || head_dim == 16) {
     e = dtype == MI_DTYPE_F32
-            ? (head_dim == 32    ? launch_f32<32>(a, st)
-               : head_dim == 64  ? launch_f32<64>(a, st)
-               : head_dim == 128 ? launch_f32<128>(a, st)
-                                 : launch_valu<float>(a, head_dim, st))
+            ? (!f32_matrix_kernel(a, head_dim) ? launch_valu<float>(a, head_dim, st)
+               : head_dim == 32                ? launch_f32<32>(a, st)
+               : head_dim == 64                ? launch_f32<64>(a, st)
+                                               : launch_f32<128>(a, st))
         : dtype == MI_DTYPE_BF16 ? launch_valu<bf16_t>(a, head_dim, st)
                                  : launch_valu<f16_t>(a, head_dim, st);
   } else if (dtype == MI_DTYPE_BF16) {

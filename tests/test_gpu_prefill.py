@@ -115,6 +115,20 @@ def test_config1_rope_prefill_fp32(dev):
     assert max_abs(lse, ref_lse) < 1e-3
 
 
+# both kernels at the lines between them; the last column: more 32-row blocks than CUs
+@pytest.mark.parametrize("D,S,B,Hq", [
+    (64, 1, 1, 4), (64, 32, 1, 4), (64, 33, 1, 4), (64, 64, 5, 32), (64, 65, 5, 32),
+    (128, 16, 1, 4), (128, 17, 1, 4), (128, 48, 1, 4), (128, 49, 1, 4), (128, 65, 1, 4),
+    (128, 64, 6, 24), (128, 65, 6, 24), (128, 80, 6, 24), (128, 81, 6, 24)])
+def test_fp32_short_prompts(dev, D, S, B, Hq):
+    q = randn((B, Hq, S, D), 63, torch.float32, dev)
+    k = randn((B, Hq // 4, S, D), 64, torch.float32, dev)
+    v = randn((B, Hq // 4, S, D), 65, torch.float32, dev)
+    out, lse = _fa()(q, k, v, return_lse=True)
+    ref, ref_lse = ora.prefill(q, k, v)
+    assert max_abs(out, ref) < TOL[torch.float32] and max_abs(lse, ref_lse) < 1e-3
+
+
 @pytest.mark.parametrize("D", [32, 64, 128])
 def test_fp32_prefill_with_non_finite_values(dev, D):
     """An infinity or a NaN in V reaches the rows that see its key and no earlier one
