@@ -444,13 +444,13 @@ __device__ inline u32x4 rows_hi(const u32x4& a, const u32x4& b) {
 // [3072, 3072] 10.8 -> 6.3 us, [3072, 8192] 25.2 -> 14.6, SwiGLU 2 x [8192, 3072]
 // 17.9 -> 13.0 (3.9 TB/s), SwiGLU 2 x [8192, 2048] 11.7 -> 9.5, [3072, 2048] 6.9 -> 4.9.
 // What is left is x: the same calls with all 16 rows at one address take 1 to 3 us less.
-template <typename T, int NW, int SC, bool NORM, int EPI, int TPB>
+template <typename T, int NW, int SC, bool NORM, int EPI, int TPB, int RT>
 __global__ __launch_bounds__(64 * NW) void rows_gemv_kernel(LayerGemvArgs a) {
   using MM = LMfma<T>;
   typedef typename MM::v8 v8;
   constexpr int NMAT = EPI == kEpiSwiglu ? 2 : 1;
-  constexpr int NT = NMAT * TPB;                       // 16-row A tiles per block
-  constexpr int NOUT = 256 * TPB;                      // outputs of a block
+  constexpr int NT = NMAT * TPB;                       // A tiles (RT rows) per block
+  constexpr int NOUT = 16 * RT * TPB;                  // outputs of a block
   constexpr int NO = (NOUT + 64 * NW - 1) / (64 * NW); // outputs of a thread
   __shared__ __align__(16) float red[NW][NT][16][16];  // [wave][tile][token][row]
   __shared__ float ssq[NORM ? NW : 1][16];             // per-wave sums of squares
@@ -465,7 +465,7 @@ __global__ __launch_bounds__(64 * NW) void rows_gemv_kernel(LayerGemvArgs a) {
   // ---- the block's tiles.  QKV: tiles of wq, then wk, then wv in one list,
   //      each 8 rotation pairs of a head (rows 0..7 dims d, rows 8..15 d + D/2)
   const int half = a.D >> 1, tph = EPI == kEpiQkvRope ? half >> 3 : 1;
-  const int n_tiles = EPI == kEpiQkvRope ? a.n_tiles0 + 2 * a.n_tiles1 : (a.N + 15) >> 4;
+  const int n_tiles = EPI == kEpiQkvRope ? a.n_tiles0 + 2 * a.n_tiles1 : (a.N + RT - 1) / RT;
   auto mat_of = [&](int tile) -> int {
     if constexpr (EPI != kEpiQkvRope) return 0;
     return tile < a.n_tiles0 ? 0 : tile < a.n_tiles0 + a.n_tiles1 ? 1 : 2;
@@ -476,7 +476,7 @@ __global__ __launch_bounds__(64 * NW) void rows_gemv_kernel(LayerGemvArgs a) {
       const int head = tim / tph, j = tim - head * tph;
       return head * a.D + 8 * j + (row & 7) + ((row >> 3) ? half : 0);
     } else {
-      return tile * 16 + row;
+      return tile * RT + row;
     }
   };
   // weight rows through buffer resources (host-checked: each matrix spans < 2^31
@@ -492,7 +492,7 @@ __global__ __launch_bounds__(64 * NW) void rows_gemv_kernel(LayerGemvArgs a) {
     const int rows = EPI == kEpiQkvRope && mat != 0 ? a.Hkv * a.D : a.N;
     wr[t] = make_rsrc(wm, (uint32_t)((int64_t)(rows - 1) * sn + a.K));
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
+    for (int h = 0; h < RT / 8; ++h) {
       const int n = w_row(tile, mat, 8 * h + (r & 7));
       woff[t][h] = (tile < n_tiles && n < rows ? (uint32_t)((int64_t)n * sn) : kOobOffset) +
                    (r >> 3) * 64 + 16 * g;
@@ -523,7 +523,8 @@ __global__ __launch_bounds__(64 * NW) void rows_gemv_kernel(LayerGemvArgs a) {
   for (int s = 0; s < SC; ++s)
 #pragma unroll
     for (int t = 0; t < NT; ++t)
-      wq[t][s] = buf_load16_nt(wr[t], woff[t][s & 1] + (uint32_t)(kw + (s >> 1) * 128));
+      if (RT == 16 || s % 2 == 0)
+        wq[t][s] = buf_load16_nt(wr[t], woff[t][s & 1] + (uint32_t)(kw + (s >> 1) * 128));
 
   // ---- epilogue operands behind the weights, from clamped indices
   T e_s0[NO], e_s1[NO], e_res[NO], e_cos[NO], e_sin[NO];
@@ -531,8 +532,8 @@ __global__ __launch_bounds__(64 * NW) void rows_gemv_kernel(LayerGemvArgs a) {
 #pragma unroll
   for (int o = 0; o < NO; ++o) {
     const int i = min(tid + o * 64 * NW, NOUT - 1);
-    const int tile = min((int)blockIdx.x * TPB + (i >> 8), n_tiles - 1);
-    const int row = i & 15, m = min((i >> 4) & 15, a.M - 1);
+    const int tile = min((int)blockIdx.x * TPB + i / (16 * RT), n_tiles - 1);
+    const int row = i % RT, m = min(i / RT % 16, a.M - 1);
     if constexpr (EPI == kEpiQkvRope) {
       const int mat = mat_of(tile), n = w_row(tile, mat, row);
       const T* sc = reinterpret_cast<const T*>(mat == 0 ? a.s0 : mat == 1 ? a.s1 : a.s2);
@@ -543,7 +544,7 @@ __global__ __launch_bounds__(64 * NW) void rows_gemv_kernel(LayerGemvArgs a) {
       e_cos[o] = reinterpret_cast<const T*>(a.cos)[crow * a.c_ss + ii];
       e_sin[o] = reinterpret_cast<const T*>(a.sin)[crow * a.c_ss + ii];
     } else {
-      const int n = min(tile * 16 + row, a.N - 1);
+      const int n = min(tile * RT + row, a.N - 1);
       e_s0[o] = reinterpret_cast<const T*>(a.s0)[n];
       if constexpr (EPI == kEpiSwiglu) e_s1[o] = reinterpret_cast<const T*>(a.s1)[n];
       if constexpr (EPI == kEpiResidual)
@@ -598,7 +599,12 @@ __global__ __launch_bounds__(64 * NW) void rows_gemv_kernel(LayerGemvArgs a) {
     const v8 xb1 = __builtin_bit_cast(v8, xr[s][1]);
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
-      const u32x4 wv = s & 1 ? rows_hi(wq[t][s - 1], wq[t][s]) : rows_lo(wq[t][s], wq[t][s + 1]);
+      // (8-row tiles: A rows 8..15 are left as they come, nobody reads their sums)
+      u32x4 wv;
+      if constexpr (RT == 16)
+        wv = s & 1 ? rows_hi(wq[t][s - 1], wq[t][s]) : rows_lo(wq[t][s], wq[t][s + 1]);
+      else
+        wv = s & 1 ? rows_hi(wq[t][s - 1], wq[t][s - 1]) : wq[t][s];
       acc[t] = MM::mma(i8x8_cvt<T, v8>(wv.x, wv.y), xb0, acc[t]);
       acc[t] = MM::mma(i8x8_cvt<T, v8>(wv.z, wv.w), xb1, acc[t]);
     }
@@ -618,7 +624,7 @@ __global__ __launch_bounds__(64 * NW) void rows_gemv_kernel(LayerGemvArgs a) {
 #pragma unroll
   for (int o = 0; o < NO; ++o) {
     const int i = tid + o * 64 * NW;
-    const int t = i >> 8, tile = blockIdx.x * TPB + t, row = i & 15, m = (i >> 4) & 15;
+    const int t = i / (16 * RT), tile = blockIdx.x * TPB + t, row = i % RT, m = i / RT % 16;
     if (i >= NOUT || tile >= n_tiles || m >= a.M) continue;
     if constexpr (EPI == kEpiQkvRope) {
       const int mat = mat_of(tile), n = w_row(tile, mat, row);
@@ -641,7 +647,7 @@ __global__ __launch_bounds__(64 * NW) void rows_gemv_kernel(LayerGemvArgs a) {
         c[(int64_t)m * a.c_sb + (int64_t)head * a.c_sh + pos * a.c_st + d] = out;
       }
     } else {
-      const int n = tile * 16 + row;
+      const int n = tile * RT + row;
       if (n >= a.N) continue;
       float v = rnd(wsum(t, m, row) * f32_of(e_s0[o]));
       if constexpr (EPI == kEpiResidual) {
@@ -657,34 +663,35 @@ __global__ __launch_bounds__(64 * NW) void rows_gemv_kernel(LayerGemvArgs a) {
 
 namespace {
 
-template <typename T, bool NORM, int EPI, int TPB, int NW, int SC>
+template <typename T, bool NORM, int EPI, int TPB, int NW, int SC, int RT>
 hipError_t launch_rows(const LayerGemvArgs& a, int n_tiles, hipStream_t st) {
-  hipLaunchKernelGGL((rows_gemv_kernel<T, NW, SC, NORM, EPI, TPB>),
+  hipLaunchKernelGGL((rows_gemv_kernel<T, NW, SC, NORM, EPI, TPB, RT>),
                      dim3((unsigned)((n_tiles + TPB - 1) / TPB)), dim3(64 * NW), 0, st, a);
   return hipGetLastError();
 }
 
 // Waves and chunks per wave from K = 64 * NW * SC, at most 16 waves.
-template <typename T, bool NORM, int EPI, int TPB>
+template <typename T, bool NORM, int EPI, int TPB, int RT>
 hipError_t dispatch_rows_k(const LayerGemvArgs& a, int n_tiles, hipStream_t st) {
   switch (a.K) {
-    case 512: return launch_rows<T, NORM, EPI, TPB, 4, 2>(a, n_tiles, st);
-    case 1024: return launch_rows<T, NORM, EPI, TPB, 8, 2>(a, n_tiles, st);
-    case 1536: return launch_rows<T, NORM, EPI, TPB, 12, 2>(a, n_tiles, st);
-    case 2048: return launch_rows<T, NORM, EPI, TPB, 8, 4>(a, n_tiles, st);
+    case 512: return launch_rows<T, NORM, EPI, TPB, 4, 2, RT>(a, n_tiles, st);
+    case 1024: return launch_rows<T, NORM, EPI, TPB, 8, 2, RT>(a, n_tiles, st);
+    case 1536: return launch_rows<T, NORM, EPI, TPB, 12, 2, RT>(a, n_tiles, st);
+    case 2048: return launch_rows<T, NORM, EPI, TPB, 8, 4, RT>(a, n_tiles, st);
     default: break;
   }
   if constexpr (!NORM) {   // the prologue serves K <= 2048 (host-checked)
     switch (a.K) {
-      case 3072: return launch_rows<T, NORM, EPI, TPB, 12, 4>(a, n_tiles, st);
+      case 3072: return launch_rows<T, NORM, EPI, TPB, 12, 4, RT>(a, n_tiles, st);
       // 16 waves have 128 registers each: one tile of two matrices at a time
-      case 4096: return launch_rows<T, NORM, EPI, EPI == kEpiSwiglu ? 1 : TPB, 16, 4>(a, n_tiles, st);
+      case 4096:
+        return launch_rows<T, NORM, EPI, EPI == kEpiSwiglu ? 1 : TPB, 16, 4, RT>(a, n_tiles, st);
       default: break;
     }
     if constexpr (EPI != kEpiSwiglu) {  // two weight streams: K <= 4096 (host-checked)
       switch (a.K) {
-        case 6144: return launch_rows<T, NORM, EPI, 1, 16, 6>(a, n_tiles, st);
-        case 8192: return launch_rows<T, NORM, EPI, 1, 16, 8>(a, n_tiles, st);
+        case 6144: return launch_rows<T, NORM, EPI, 1, 16, 6, RT>(a, n_tiles, st);
+        case 8192: return launch_rows<T, NORM, EPI, 1, 16, 8, RT>(a, n_tiles, st);
         default: break;
       }
     }
@@ -692,15 +699,25 @@ hipError_t dispatch_rows_k(const LayerGemvArgs& a, int n_tiles, hipStream_t st) 
   return hipErrorInvalidValue;
 }
 
-// 9..16 rows: two tiles per block when one per block is more than a block per CU.
+template <typename T, int EPI, int TPB, int RT>
+hipError_t dispatch_rows_norm(const LayerGemvArgs& a, int n_tiles, hipStream_t st) {
+  return a.norm_w != nullptr ? dispatch_rows_k<T, true, EPI, TPB, RT>(a, n_tiles, st)
+                             : dispatch_rows_k<T, false, EPI, TPB, RT>(a, n_tiles, st);
+}
+
+// 9..16 rows: two tiles per block when one per block is more than a block per CU, and
+// tiles of 8 rows where tiles of 16 leave half the CUs without a block (twice the
+// blocks and twice the reads of x, but half the weights and sums per block).  MI355X,
+// 16 rows, 16- against 8-row tiles, per call in a graph: [2048, 8192] 12.9 -> 11.5 us,
+// [1024, 6144] 10.1 -> 8.9, [512, 2048] 4.7 -> 4.4, [2048, 512] 3.0 -> 2.8; [2080, 8192],
+// the first N past the line, 12.9 with 16-row tiles.
 template <typename T, int EPI>
 hipError_t dispatch_rows(const LayerGemvArgs& a, int n_tiles, hipStream_t st) {
-  const bool two = n_tiles > device_cu_count();
-  if (a.norm_w != nullptr)
-    return two ? dispatch_rows_k<T, true, EPI, 2>(a, n_tiles, st)
-               : dispatch_rows_k<T, true, EPI, 1>(a, n_tiles, st);
-  return two ? dispatch_rows_k<T, false, EPI, 2>(a, n_tiles, st)
-             : dispatch_rows_k<T, false, EPI, 1>(a, n_tiles, st);
+  const int cus = device_cu_count();
+  if constexpr (EPI != kEpiQkvRope)
+    if (2 * n_tiles <= cus) return dispatch_rows_norm<T, EPI, 1, 8>(a, (a.N + 7) / 8, st);
+  return n_tiles > cus ? dispatch_rows_norm<T, EPI, 2, 16>(a, n_tiles, st)
+                       : dispatch_rows_norm<T, EPI, 1, 16>(a, n_tiles, st);
 }
 
 // Diagonal-packed kernel (M <= 8): waves and superchunks per wave from K =

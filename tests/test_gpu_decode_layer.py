@@ -34,7 +34,10 @@ def _close(a, b, tol):
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("M,K,N", [(1, 512, 384), (3, 2048, 512), (8, 2048, 2048), (16, 1024, 256),
                                    (8, 8192, 2048), (12, 2048, 4096), (5, 3072, 600),
-                                   (7, 1024, 100), (2, 4096, 36)])
+                                   (7, 1024, 100), (2, 4096, 36),
+                                   # 9..16 rows: 8-row tiles up to 128 tiles of 16, then 16-row
+                                   (9, 512, 7), (11, 2048, 100), (16, 1536, 2041), (13, 1024, 2048),
+                                   (10, 4096, 2049), (9, 6144, 1020), (16, 8192, 2048)])
 @pytest.mark.parametrize("norm", [False, True])
 def test_linear_store_and_residual(dev, dtype, M, K, N, norm):
     if norm and (M * K * 2 > 64 * 1024 or (M > 8 and K > 2048)):
