@@ -423,6 +423,9 @@ int32_t mi_w8a16_gemm_multi(const void* x, int64_t m, int64_t k, int64_t x_sm,
  * w8a16_gemm_launch at these sizes  src/quant_linear.py:123-188, :191-247.
  */
 int64_t mi_w8a16_small_gemm_splits(int64_t m, int64_t n, int64_t k);
+/* Rows of a tile (32 to 160) that such a call runs with (0: no such call). */
+int64_t mi_w8a16_small_gemm_tile_rows(int64_t m, int32_t n_mats, const int64_t* n, int64_t k,
+                                      int32_t epilogue);
 int32_t mi_w8a16_small_gemm(const void* x, int64_t m, int64_t k, int64_t x_sm,
                             int32_t n_mats, const int8_t* const* w,
                             const void* const* scales, void* const* y,

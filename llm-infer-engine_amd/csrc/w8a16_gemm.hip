@@ -566,7 +566,7 @@ __global__ __launch_bounds__(256) void w8a16_splitk_reduce_kernel(GemmArgs a, in
 //    BM = 32 MB rows; the tile is 32 MB x 32 NG and its k groups meet in LDS at
 //    the end, in k-group order.
 //  * x and the int8 weights both come by LDS DMA into a ring of S stages of
-//    64 KG k (96 to 144 KB, one workgroup per CU), S - 1 of them in flight; the
+//    64 KG k (120 to 144 KB, one workgroup per CU), S - 1 of them in flight; the
 //    wait counts this wave's own copies (vmcnt), one barrier per stage publishes
 //    them and frees the slot that the next copy overwrites.
 //  * the two operands use the widening of the large GEMM; their 16-byte chunks are
@@ -1256,6 +1256,14 @@ int mid_mb(int64_t m, int64_t tiles_n, int kg) {
   return best;
 }
 
+// Tile columns of a call: of all its matrices, or of the gated product (SwiGLU).
+int64_t mid_tiles_n(int kg, int32_t n_mats, const int64_t* n, int32_t epilogue) {
+  const int64_t cols = epilogue == 2 ? 128 / kg : 256 / kg;
+  int64_t t = 0;
+  for (int i = 0; i < (epilogue == 2 ? 1 : n_mats); ++i) t += (n[i] + cols - 1) / cols;
+  return t;
+}
+
 template <typename T, typename ST, int MB, int KG, int EPI>
 hipError_t mid_launch(const MidArgs& a, int64_t splits, hipStream_t st) {
   using SH = MidShape<MB, KG>;
@@ -1302,6 +1310,14 @@ extern "C" int64_t mi_w8a16_small_gemm_splits(int64_t m, int64_t n, int64_t k) {
   return mid_splits(m, n, k);
 }
 
+extern "C" int64_t mi_w8a16_small_gemm_tile_rows(int64_t m, int32_t n_mats, const int64_t* n,
+                                                 int64_t k, int32_t epilogue) {
+  if (m <= 0 || n_mats < 1 || n_mats > kMidMats || n == nullptr || k <= 0) return 0;
+  const int kg = mid_kg(m);
+  const int64_t splits = n_mats == 1 ? mid_splits(m, n[0], k) : 1;
+  return 32 * mid_mb(m, mid_tiles_n(kg, n_mats, n, epilogue) * splits, kg);
+}
+
 extern "C" int32_t mi_w8a16_small_gemm(const void* x, int64_t m, int64_t k, int64_t x_sm,
                                        int32_t n_mats, const int8_t* const* w,
                                        const void* const* scales, void* const* y,
@@ -1333,22 +1349,21 @@ extern "C" int32_t mi_w8a16_small_gemm(const void* x, int64_t m, int64_t k, int6
     set_last_error("%s: need 1 <= M <= 65535 (M=%lld)", what, (long long)m);
     return MI_ERR_INVALID;
   }
-  const int kg = mid_kg(m), bn = 256 / kg;
+  const int kg = mid_kg(m);
   if (k % mid_bk(kg) != 0) {
     set_last_error("%s: K must be a multiple of %d (K=%lld)", what, mid_bk(kg), (long long)k);
     return MI_ERR_UNSUPPORTED;
   }
   MidArgs a{};
-  const int cols = epilogue == 2 ? bn / 2 : bn;
-  int64_t tiles_n = 0;
+  const int64_t tiles_n = mid_tiles_n(kg, n_mats, n, epilogue);
   for (int i = 0; i < n_mats; ++i) {
     GemmArgs g;
     void* yi = epilogue == 2 ? y[0] : y[i];
     int32_t rc = gemm_setup(what, x, w[i], scales[i], yi, m, n[i], k, x_sm, w_sn[i], s_sn[i],
                             epilogue == 2 ? y_sm[0] : y_sm[i], g);
     if (rc != MI_OK) return rc;
-    a.mat[i] = MidMat{g.w, g.scales, yi, g.w_sn, g.s_sn, g.y_sm, g.N, (int32_t)tiles_n, g.y_vec};
-    if (epilogue != 2 || i == 0) tiles_n += (n[i] + cols - 1) / cols;
+    a.mat[i] = MidMat{g.w, g.scales, yi, g.w_sn, g.s_sn, g.y_sm, g.N,
+                      (int32_t)mid_tiles_n(kg, i, n, 0), g.y_vec};
   }
   if (epilogue == 1 && res_sm < n[0]) {
     set_last_error("%s: residual rows shorter than N", what);
@@ -1371,7 +1386,7 @@ extern "C" int32_t mi_w8a16_small_gemm(const void* x, int64_t m, int64_t k, int6
         return MI_ERR_UNSUPPORTED;
       }
   }
-  const int mb = mid_mb(m, tiles_n * splits, kg);
+  const int mb = (int)(mi_w8a16_small_gemm_tile_rows(m, n_mats, n, k, epilogue) / 32);
   a.tiles_m = (int32_t)((m + 32 * mb - 1) / (32 * mb));
   a.tiles_n = (int32_t)tiles_n;
   if (tiles_n * a.tiles_m * splits > INT32_MAX / 64) {

@@ -170,6 +170,7 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
         _i32, _i32, _ptr,                      # dtype sdtype stream
     ]),
     "mi_w8a16_small_gemm_splits": (_i64, [_i64, _i64, _i64]),
+    "mi_w8a16_small_gemm_tile_rows": (_i64, [_i64, _i32, _ptr, _i64, _i32]),
     "mi_w8a16_small_gemm": (_i32, [
         _ptr, _i64, _i64, _i64, _i32,          # x M K x_sm n_mats
         _ptr, _ptr, _ptr,                      # w[] scales[] y[] (host arrays)

@@ -11,6 +11,8 @@ ragged M / N that leave partial 128 x 256 tiles.  Bars:
     (oracle.quant.w8a16, the reference test's reference), and within 1e-2 of
     the GEMV kernel's result on the same rows (two fp32 summation orders).
 """
+import ctypes
+
 import pytest
 import torch
 
@@ -349,7 +351,7 @@ def test_gemm_residual_is_the_separate_add(dev, M, K, N, dtype, splits, pad):
 @pytest.mark.parametrize("K,N", [(256, 100), (768, 516), (2048, 2048), (8192, 1027)])
 def test_small_gemm_tile_edges(dev, M, K, N):
     """mi_w8a16_small_gemm at both tile widths (up to 64 rows and above), with
-    row counts around each number of 32-row blocks, partial columns, rings
+    row counts around multiples of 32, partial columns, rings
     deeper and shallower than K, and K = 8192 split: against the oracle, and
     bit-exact where each output is one product (one-hot rows)."""
     from src.quant_linear import w8a16_small_gemm
@@ -366,6 +368,77 @@ def test_small_gemm_tile_edges(dev, M, K, N):
     hot[torch.arange(M, device=dev), k_of] = 0.5
     one = w8a16_small_gemm(hot, [(q, s)])[0]
     assert torch.equal(one, ((q[:, k_of].t().float() * 0.5) * s.float().view(-1)).to(dtype))
+
+
+def _tile_rows(M, ns, K, epilogue):
+    from src import _lib
+    n = (ctypes.c_int64 * len(ns))(*ns)
+    return _lib.load().mi_w8a16_small_gemm_tile_rows(M, len(ns), ctypes.addressof(n), K, epilogue)
+
+
+def _one_hot(M, K, dtype, dev, seed):
+    """Rows of one 0.5 each: x, and the exact output for (q, s) from it."""
+    k_of = torch.randint(0, K, (M,), generator=torch.Generator().manual_seed(seed)).to(dev)
+    hot = torch.zeros((M, K), device=dev, dtype=dtype)
+    hot[torch.arange(M, device=dev), k_of] = 0.5
+    return hot, lambda q, s: ((q[:, k_of].t().float() * 0.5) * s.float().view(-1)).to(dtype)
+
+
+# every tile height of both widths (64 columns up to 64 rows, 128 above), with and without
+# a K split, ragged in rows and columns; rows and splits are those that 256 CUs lead to
+@pytest.mark.parametrize("M,N,K,rows,splits", [
+    (60, 16382, 256, 64, 1), (48, 3070, 8192, 64, 4), (61, 8190, 4096, 64, 2),
+    (200, 8190, 512, 64, 1), (300, 8190, 512, 96, 1), (453, 8190, 384, 128, 1), (550, 8190, 512, 160, 1),
+    (200, 2045, 8192, 64, 4), (300, 2045, 8192, 96, 4), (453, 2045, 8192, 128, 4),
+    (550, 2045, 8192, 160, 4), (701, 2045, 8192, 160, 3)])
+def test_small_gemm_tile_heights(dev, M, N, K, rows, splits):
+    from src import _lib
+    from src.quant_linear import w8a16_small_gemm
+    assert _tile_rows(M, [N], K, 0) == rows
+    assert _lib.load().mi_w8a16_small_gemm_splits(M, N, K) == splits
+    dtype = torch.bfloat16 if M % 2 else torch.float16
+    q, s = _quantised(N, K, dtype, dev, 230)
+    x, res = _x(M, K, dtype, dev, 231), _x(M, N, dtype, dev, 232)
+    y = w8a16_small_gemm(x, [(q, s)])[0]
+    assert _rel(y, oq.w8a16(x, q, s)) < 2e-2
+    assert torch.equal(w8a16_small_gemm(x, [(q, s)], residual=res)[0], res + y)
+    hot, exact = _one_hot(M, K, dtype, dev, 233)
+    assert torch.equal(w8a16_small_gemm(hot, [(q, s)])[0], exact(q, s))
+
+
+@pytest.mark.parametrize("M,rows", [(40, 64), (100, 64), (130, 96), (250, 128), (301, 160)])
+def test_small_gemm_swiglu_tile_heights(dev, M, rows):
+    """The gated form at each tile height: against the oracle, and on one-hot rows
+    against silu and product of the exact projections (silu one ulp off at most)."""
+    from src.quant_linear import w8a16_small_gemm
+    N, K = 8190, 256
+    assert _tile_rows(M, [N, N], K, 2) == rows
+    dtype = torch.bfloat16 if M % 2 else torch.float16
+    mats = [_quantised(N, K, dtype, dev, i) for i in (240, 241)]
+    x = _x(M, K, dtype, dev, 242)
+    y1, y3 = (oq.w8a16(x, *m).float() for m in mats)
+    assert _rel(w8a16_small_gemm(x, mats, swiglu=True)[0], torch.nn.functional.silu(y1) * y3) < 3e-2
+    hot, exact = _one_hot(M, K, dtype, dev, 243)
+    g, want = w8a16_small_gemm(hot, mats, swiglu=True)[0], torch.nn.functional.silu(exact(*mats[0])) * exact(*mats[1])
+    # two roundings to dtype from values one ulp apart: two ulps of the result
+    ulp = torch.finfo(dtype).eps
+    assert ((g.float() - want.float()).abs() <= 2 * ulp * want.float().abs() + 1e-7).all()
+
+
+@pytest.mark.parametrize("M,rows", [(400, 64), (700, 96), (1001, 128), (1400, 160)])
+def test_small_gemm_multi_tile_heights(dev, M, rows):
+    """Three matrices in one launch at each tile height above 64 rows: bit-exact on
+    one-hot rows, which pins each matrix's tile columns and scales."""
+    from src.quant_linear import w8a16_small_gemm
+    ns, K, dtype = (2046, 512, 509), 256, torch.bfloat16
+    assert _tile_rows(M, ns, K, 0) == rows
+    mats = [_quantised(n, K, dtype, dev, 250 + i) for i, n in enumerate(ns)]
+    x = _x(M, K, dtype, dev, 253)
+    for y, m in zip(w8a16_small_gemm(x, mats), mats):
+        assert _rel(y, oq.w8a16(x, *m)) < 2e-2
+    hot, exact = _one_hot(M, K, dtype, dev, 254)
+    for y, m in zip(w8a16_small_gemm(hot, mats), mats):
+        assert torch.equal(y, exact(*m))
 
 
 @pytest.mark.parametrize("M", [24, 64, 96, 300])
