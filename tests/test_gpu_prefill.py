@@ -77,6 +77,23 @@ def test_reference_selftest_shape(dev):
     assert torch.allclose(out.cpu(), ref, atol=1e-3, rtol=1e-3)
 
 
+# grids (per XCD, 32 CUs, at 8 x 8 KV heads; all together, 256 CUs, at 3 x 5) of just over
+# one, of two, of just over two and of nearly three blocks per CU; the last is not reordered
+@pytest.mark.parametrize("B,Hq,Hkv,S", [(8, 32, 8, 317), (8, 32, 8, 512), (8, 32, 8, 575), (8, 32, 8, 703),
+                                        (8, 32, 8, 768), (3, 20, 5, 1150), (3, 20, 5, 2239)])
+def test_prefill_d64_paired_block_order(dev, B, Hq, Hkv, S):
+    """D = 64 with one to three blocks per CU, where the second block of a CU goes out
+    lightest first: every block is there, once."""
+    q = randn((B, Hq, S, 64), 66, torch.bfloat16, dev)
+    k = randn((B, Hkv, S, 64), 67, torch.bfloat16, dev)
+    v = randn((B, Hkv, S, 64), 68, torch.bfloat16, dev)
+    out, lse = _fa()(q, k, v, return_lse=True)
+    for b in range(B):      # the oracle one prompt at a time to bound host memory
+        ref, ref_lse = ora.prefill(q[b:b + 1], k[b:b + 1], v[b:b + 1])
+        assert max_abs(out[b:b + 1], ref) < TOL[torch.bfloat16]
+        assert max_abs(lse[b:b + 1], ref_lse) < 1e-3
+
+
 def test_model_layout_and_cache_views(dev):
     """q is a [B,H,S,D] view of [B,S,H,D] memory; k/v are cache views with a
     larger capacity T (strides (Hkv*T*D, T*D, D, 1)), as in src/model.py:57-79."""
