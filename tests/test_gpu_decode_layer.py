@@ -79,6 +79,31 @@ def test_swiglu_with_norm(dev, dtype, M):
     _close(y, torch.nn.functional.silu(w1(xn)) * w3(xn), 1e-2)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M,K,N", [(9, 2048, 8192), (16, 2048, 8192), (11, 1024, 4250), (16, 512, 4100)])
+def test_rows_gemv_norm_with_two_tiles(dev, dtype, M, K, N):
+    """9..16 rows with the RMSNorm prologue and two tiles per block (more than 256
+    tiles), an odd last tile among them: every epilogue."""
+    from src import decode_layer
+    from src.quant_linear import w8a16_gemv_launch
+    from src.rms_norm import rmsnorm_triton
+    w1, w3 = _linear(dev, K, N, dtype, 55), _linear(dev, K, N, dtype, 56)
+    x, res = randn((M, K), 57, dtype, dev, scale=3.0), randn((M, N), 58, dtype, dev)
+    nw = (1.0 + 0.1 * randn((K,), 59, torch.float32)).to(dtype).to(dev)
+    a, xn = oq.rmsnorm(x, nw, 1e-5), rmsnorm_triton(x, nw, 1e-5)
+    ref = oq.w8a16(a, w1.weight, w1.scales)
+    un, un3 = (w8a16_gemv_launch(xn, w.weight, w.scales) for w in (w1, w3))
+    y = decode_layer.linear_fused(x, w1, norm_weight=nw, eps=1e-5)
+    _close(y, ref, 2e-2)
+    _close(y, un, 1e-2)
+    yr = decode_layer.linear_fused(x, w1, norm_weight=nw, eps=1e-5, residual=res)
+    _close(yr, (res.cpu().float() + ref.float()).to(dtype), 2e-2)
+    _close(yr, res + un, 1e-2)
+    g = decode_layer.linear_fused(x, w1, norm_weight=nw, eps=1e-5, lin_b=w3)
+    _close(g, torch.nn.functional.silu(ref.float()) * oq.w8a16(a, w3.weight, w3.scales).float(), 2e-2)
+    _close(g, torch.nn.functional.silu(un) * un3, 1e-2)
+
+
 class _Attn:
     def __init__(self, dev, dim, Hq, Hkv, D, dtype):
         self.n_heads, self.n_kv_heads, self.head_dim = Hq, Hkv, D
@@ -157,9 +182,10 @@ def test_rows_gemv_widths_and_tile_edges(dev, M, K, N):
 
 @pytest.mark.parametrize("M,dim,Hq,Hkv,D", [(16, 3072, 24, 8, 128), (9, 2048, 32, 8, 64),
                                             (11, 1024, 3, 1, 48)])
-def test_block_of_9_to_16_rows_matches_op_chain(dev, M, dim, Hq, Hkv, D):
+def test_block_of_9_to_16_rows_matches_op_chain(dev, M, dim, Hq, Hkv, D, monkeypatch):
     """The fused block at batches above 8 (RMSNorm as its own launch where the
     prologue does not take the size) against its op-by-op form."""
+    from src import model_quantized
     from src.config import ModelArgs
     from src.kv_cache import KVCache
     from src.model_quantized import QuantizedTransformerBlock, build_random_quantized
@@ -190,11 +216,10 @@ def test_block_of_9_to_16_rows_matches_op_chain(dev, M, dim, Hq, Hkv, D):
     ys = []
     with torch.no_grad():
         for c, fused in zip(kv, (True, False)):
-            QuantizedTransformerBlock.fused_decode = fused
-            try:
-                ys.append(block(x, cos.to(dev), sin.to(dev), layer_idx=0, start_pos=40, kv_cache=c))
-            finally:
-                QuantizedTransformerBlock.fused_decode = True
+            monkeypatch.setattr(QuantizedTransformerBlock, "fused_decode", fused)
+            if not fused:      # nor the feed-forward's and the residual's fused forms
+                monkeypatch.setattr(model_quantized, "_plain", lambda *lins: False)
+            ys.append(block(x, cos.to(dev), sin.to(dev), layer_idx=0, start_pos=40, kv_cache=c))
     _close(ys[0], ys[1], 1e-2)
     _close(kv[0].k, kv[1].k, 1e-2)
     _close(kv[0].v, kv[1].v, 1e-2)
@@ -427,9 +452,10 @@ def test_decode_at_a_host_position_trusts_no_attribute_of_the_cache(dev):
         assert all(torch.equal(a, b) for a, b in zip(seen[0], other))
 
 
-def test_fused_decode_step_matches_unfused(dev):
+def test_fused_decode_step_matches_unfused(dev, monkeypatch):
     """The quantized block's fused single-token path against the op-by-op
     composition of the same model (eager, three decode steps)."""
+    from src import model_quantized
     from src.config import ModelArgs
     from src.kv_cache import KVCache
     from src.model_quantized import QuantizedTransformerBlock, build_random_quantized
@@ -444,13 +470,11 @@ def test_fused_decode_step_matches_unfused(dev):
         kv_b.v.copy_(kv_a.v)
         for step in range(3):
             tok = toks[:, step:step + 1]
-            QuantizedTransformerBlock.fused_decode = True
             la = model(tok, start_pos=20 + step, kv_cache=kv_a)
-            QuantizedTransformerBlock.fused_decode = False
-            try:
+            with monkeypatch.context() as m:
+                m.setattr(QuantizedTransformerBlock, "fused_decode", False)
+                m.setattr(model_quantized, "_plain", lambda *lins: False)   # the sub-blocks' fused forms
                 lb = model(tok, start_pos=20 + step, kv_cache=kv_b)
-            finally:
-                QuantizedTransformerBlock.fused_decode = True
             _close(la, lb, 1e-2)
             _close(kv_a.k, kv_b.k, 1e-2)
             _close(kv_a.v, kv_b.v, 1e-2)

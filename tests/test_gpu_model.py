@@ -73,6 +73,7 @@ def test_w8a16_prefill_with_one_launch_projections(dev, monkeypatch):
     block runs q|k|v as one GEMM launch and silu(w1)*w3 as one launch: the
     prefill's logits and KV cache match the per-projection op chain within
     the output bar, and the decode step that follows matches the oracle."""
+    from src import model as plain_model
     from src import quant_linear
     from src.kv_cache import KVCache
     args = _small_args(dev, dim=2048, n_layers=1, n_heads=32, n_kv_heads=8, hidden_dim=8192,
@@ -82,15 +83,20 @@ def test_w8a16_prefill_with_one_launch_projections(dev, monkeypatch):
     assert quant_linear.gemm_multi_worth(B * S, args.dim, [2048, 512, 512], dev)
     assert quant_linear.swiglu_worth(B * S, args.dim, args.hidden_dim, dev)
     tokens = torch.randint(0, args.vocab_size, (B, S), generator=torch.Generator().manual_seed(3)).to(dev)
-    runs = []
+    runs, chain = [], []
     for fused in (True, False):
         if not fused:
             monkeypatch.setattr(quant_linear, "gemm_multi_worth", lambda *a: False)
             monkeypatch.setattr(quant_linear, "swiglu_worth", lambda *a: False)
+            monkeypatch.setattr(quant_linear, "small_gemm_fuses", lambda *a: False)
+            for cls, name in ((plain_model.Attention, "qkv"), (plain_model.FeedForward, "forward")):
+                monkeypatch.setattr(cls, name, lambda self, *a, _f=getattr(cls, name), _n=name, **k:
+                                    (chain.append(_n), _f(self, *a, **k))[1])
         kv = KVCache(args, dtype=torch.bfloat16)
         logits = model(tokens, start_pos=0, kv_cache=kv)
         runs.append((logits, kv))
     (lf, kvf), (lc, kvc) = runs
+    assert chain == ["qkv", "forward"]      # the second run's block went through the op chain
     _logit_check(lf[:, -1], lc[:, -1])
     for a, b in ((kvf.k[:, :B, :, :S], kvc.k[:, :B, :, :S]), (kvf.v[:, :B, :, :S], kvc.v[:, :B, :, :S])):
         assert max_abs(a, b) < 2e-2 * float(b.abs().max())
