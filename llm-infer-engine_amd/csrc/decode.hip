@@ -368,21 +368,23 @@ extern "C" int64_t mi_decode_default_splits(int64_t batch, int64_t n_heads,
   // B8 Hkv8 D64 at 4097 of 8192 keys, 4 splits 22.9 us vs 8 splits 25.0 us).
   const int64_t row_bytes = 2LL * 2 * head_dim;                            // bf16 K + V
   const int64_t s_bytes = (kv_len * row_bytes + (512 << 10) - 1) / (512 << 10);
-  // One block per CU; up to 1024 keys no second split where half the CUs have a block
-  // already (B16 Hkv8 D64, 512 keys 11.4 -> 10.2 us, 1024 keys 12.0 -> 10.8 with one
-  // split; at 1500 keys two splits 15.9 us, one 16.6)
-  const int64_t s_cover =
-      kv_len <= 1024 && 2 * units >= cus ? 1 : (cus + units - 1) / units;
+  // One block per CU; but no second split where half the CUs have a block already, up
+  // to 1024 keys or head_dim 32 (B16 Hkv8 D64, 512 keys 11.4 -> 10.2 us, 1024 keys 12.0 ->
+  // 10.8 with one split, D32 1100 keys 10.1 -> 8.4; D64 at 1500 keys two splits 15.9, one 16.6)
+  const int64_t s_cover = 2 * units >= cus && (kv_len <= 1024 || head_dim <= 32)
+                              ? 1 : (cus + units - 1) / units;
   if (s > s_bytes) s = s_bytes > s_cover ? s_bytes : s_cover;
-  // >= 64 keys a split.  Up to 1024 keys fewer, because short splits cost more there
-  // (partials, combine) than their parallelism gains: one up to 256 keys, 4 up to 512,
-  // 8 up to 1024 (powers of two: 7 splits of 777 keys are slower than 8).  B1 Hkv8 D64,
-  // per call in a graph, against one split per 64 keys: 128 keys 9.9 -> 6.6 us, 256 keys
-  // 10.0 -> 8.3, 300 keys 13.7 -> 10.3, 512 keys 10.4 -> 8.9, 777 keys 15.2 -> 11.0, 1024
-  // keys 11.5 -> 9.1.  Above, half as many lose: 1500 keys 10.9 us with 24 splits, 11.9
-  // with 12; D128, 2048 keys 10.4 us with 32, 11.3 with 16.
-  const int64_t s_keys =
-      kv_len <= 256 ? 1 : kv_len <= 512 ? 4 : kv_len <= 1024 ? 8 : (kv_len + 63) / 64;
+  // One split up to 256 keys.  Above, splits whose keys are a full pass of 4 waves (128 at
+  // D64, 64 at D128) at least: one key fewer halves a block's waves (make_plan), so 12
+  // splits of 1500 keys (125 each) are slower than 11 (137); and 128 at least up to 1024
+  // keys, where partials and combine cost more than the parallelism gains.  B1 Hkv8 D64,
+  // per call in a graph, against one split per 64 keys: 128 keys 9.9 -> 6.6 us, 300 keys
+  // 13.7 -> 9.3, 777 keys 15.2 -> 9.5, 1024 keys 11.5 -> 9.1, 1500 keys 10.9 -> 9.9; D128,
+  // 777 keys 12.2 -> 9.8, 2048 keys 10.4 at 32 splits, 11.3 at 16.
+  const HostGeom geo = host_geom(MI_DTYPE_BF16, head_dim);
+  const int64_t full = std::clamp(4 * geo.rpw * geo.u, 64, 128);
+  int64_t s_keys = kv_len <= 256 ? 1 : (kv_len - 1) / (full - 1);   // ceil(kv_len / s) >= full
+  if (kv_len <= 1024) s_keys = std::min(s_keys, (kv_len + 127) / 128);
   if (s > s_keys) s = s_keys;
   if (s < 1) s = 1;
   if (s > kMaxSplits) s = kMaxSplits;

@@ -101,20 +101,23 @@ def test_split_rules_at_any_head_dim(head_dim):
 
 
 @pytest.mark.parametrize("batch,head_dim,keys,splits", [
-    (1, 64, 128, 1), (1, 64, 256, 1),                    # no split
-    (1, 64, 257, 4), (8, 64, 300, 4), (1, 128, 512, 4),
-    (1, 64, 513, 8), (4, 64, 777, 8), (1, 128, 1024, 8),
-    (1, 64, 1025, 17), (1, 64, 1500, 24), (1, 64, 2048, 32), (1, 128, 2048, 32),   # 64 keys a split
-    (1, 64, 4096, 32), (1, 128, 8192, 32),               # one block per CU
-    (16, 64, 1024, 1), (16, 64, 1500, 2), (16, 64, 2048, 2),   # half the CUs have a block
+    (1, 64, 128, 1), (1, 64, 256, 1), (1, 128, 256, 1),          # no split
+    # 128 keys a split at least, also for the last keys below a multiple
+    (1, 64, 257, 2), (8, 64, 300, 2), (1, 64, 511, 4), (1, 64, 512, 4), (4, 64, 777, 6),
+    (1, 64, 1024, 8), (1, 64, 1025, 8), (1, 64, 1500, 11), (1, 64, 2047, 16), (1, 64, 2048, 16),
+    (1, 128, 300, 3), (1, 128, 512, 4), (1, 128, 1024, 8),       # D128 up to 1024 keys as well,
+    (1, 128, 1025, 16), (1, 128, 1500, 23), (1, 128, 2048, 32),  # 64 above
+    (1, 64, 4096, 32), (1, 128, 8192, 32),                       # one block per CU
+    (16, 64, 1024, 1), (16, 64, 1500, 2), (16, 64, 2048, 2), (16, 32, 2048, 1),   # half the CUs have one
 ])
 def test_default_split_counts(batch, head_dim, keys, splits):
-    """Default splits of 8 KV heads on 256 CUs: few of them up to 1024 keys, one per
-    64 keys above (fewer were slower there: a decode step at 2048 slots keeps the
-    split count, and with it the bits, that it had before the short contexts' rule)."""
+    """Default splits of 8 KV heads on 256 CUs: no split so short that its block runs
+    fewer than 4 waves (a full pass of them is 128 keys at D64, 64 at D128)."""
     from src import _lib
     lib = _lib.load()
-    assert lib.mi_decode_default_splits(batch, 32 if head_dim == 64 else 24, 8, keys, head_dim) == splits
+    s = lib.mi_decode_default_splits(batch, 24 if head_dim == 128 else 32, 8, keys, head_dim)
+    assert s == splits
+    assert s == 1 or -(-keys // s) >= (64 if head_dim == 128 else 128)
 
 
 def test_rope_kv_append_rejects_out_of_capacity():
