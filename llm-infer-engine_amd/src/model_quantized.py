@@ -32,15 +32,20 @@ def _no_hooks(*modules) -> bool:
     (pre-)hook, their own or a global one, and no forward set on the instance."""
     if _hooks._global_forward_hooks or _hooks._global_forward_pre_hooks:
         return False
-    return not any(m._forward_hooks or m._forward_pre_hooks or "forward" in m.__dict__
-                   for m in modules)
+    for m in modules:
+        if m._forward_hooks or m._forward_pre_hooks or "forward" in m.__dict__:
+            return False
+    return True
 
 
 def _plain(*lins) -> bool:
     """Whether projections up to chat-prompt size may run on their weights in one launch:
     W8A16Linear modules whose call nothing observes or replaces.  (The decode step of
     the block and prefill-sized GEMMs take the weights without this look.)"""
-    return _no_hooks(*lins) and all(type(m).forward is W8A16Linear.forward for m in lins)
+    for m in lins:
+        if type(m).forward is not W8A16Linear.forward:
+            return False
+    return _no_hooks(*lins)
 
 
 class QuantizedFeedForward(FeedForward):
@@ -81,7 +86,13 @@ class QuantizedFeedForward(FeedForward):
 
 
 def _pairs(*lins):
-    return [(m.weight, m.scales) for m in lins]
+    return [decode_layer.raw_weights(m) for m in lins]
+
+
+def _children(module, *names):
+    """Submodules by name, from the module's own table where they are in it."""
+    own = module._modules
+    return [own[n] if n in own else getattr(module, n) for n in names]
 
 
 def _rows_fusable(x2, lin, *, swiglu=False) -> bool:
@@ -108,17 +119,18 @@ def _project_residual(lin, h, residual):
         res2 = residual.reshape(-1, lin.out_features)
         if res2.stride(1) == 1:
             return decode_layer.linear_fused(h2, lin, residual=res2).view(residual.shape)
-    gemm = rows >= quant_linear.GEMM_MIN_ROWS
-    small = (gemm or plain) and quant_linear.small_gemm_worth(h2, lin.weight)
-    if not (small or quant_linear.gemm_supported(rows, h2.shape[1])):
+    gemm = quant_linear.gemm_supported(rows, h2.shape[1])
+    pair = decode_layer.raw_weights(lin) if gemm or plain else None
+    small = pair is not None and quant_linear.small_gemm_worth(h2, pair[0])
+    if not (small or gemm):
         return residual + lin(h)
     res2 = residual.reshape(-1, lin.out_features)
     if small:
         if not gemm:
             res2 = res2.contiguous()
-        y = quant_linear.w8a16_small_gemm(h2, [(lin.weight, lin.scales)], residual=res2)[0]
+        y = quant_linear.w8a16_small_gemm(h2, [pair], residual=res2)[0]
         return y.view(*h.shape[:-1], lin.out_features)
-    y = quant_linear.w8a16_gemm_residual(h2, lin.weight, lin.scales, res2)
+    y = quant_linear.w8a16_gemm_residual(h2, *pair, res2)
     return y.view(*h.shape[:-1], lin.out_features)
 
 
@@ -160,8 +172,8 @@ class QuantizedTransformerBlock(TransformerBlock):
     def _fused_weights(self, x, rope_cos, rope_sin, kv_cache, layer_idx, positions,
                        rope_by_position, start_pos):
         """The block's weights (``decode_layer.weights_of`` pairs of wq, wk, wv, wo,
-        w1, w3, w2) and whether the QKV and the SwiGLU projection normalise their rows
-        themselves, if the fused decode-layer kernels take this call, else None.  Rows
+        w1, w3, w2), its two norms, and whether the QKV and the SwiGLU projection
+        normalise their rows themselves, if the fused decode-layer kernels take this call, else None.  Rows
         that need a launch of their own for a norm are taken only at a position inside
         the cache and where no module's call is observed or replaced."""
         if not self.fused_decode or kv_cache is None or layer_idx is None or x.shape[1] != 1:
@@ -180,29 +192,28 @@ class QuantizedTransformerBlock(TransformerBlock):
                 or kv_cache.v.dtype != dt or kv_cache.k.stride(4) != 1
                 or kv_cache.k.stride() != kv_cache.v.stride()):
             return None  # the kernels take one set of strides for each pair
-        ws = tuple(map(decode_layer.weights_of,
-                       (attn.wq, attn.wk, attn.wv, attn.wo, ff.w1, ff.w3, ff.w2)))
-        wq, wk, wv, wo, w1, w3, w2 = ws
+        lins = (*_children(attn, "wq", "wk", "wv", "wo"), *_children(ff, "w1", "w3", "w2"))
+        norms = _children(self, "attention_norm", "ffn_norm")
+        wq, wk, wv, wo, w1, w3, w2 = ws = tuple(map(decode_layer.weights_of, lins))
         n_q, n_kv = attn.n_heads * attn.head_dim, attn.n_kv_heads * attn.head_dim
         # (rows first: the kernels read as many as the heads and the residual have)
-        ok = (wq[0].shape[0] == n_q and wk[0].shape[0] == wv[0].shape[0] == n_kv
-              and wo[0].shape[0] == w2[0].shape[0] == dim
+        ok = (wq[0].size(0) == n_q and wk[0].size(0) == wv[0].size(0) == n_kv
+              and wo[0].size(0) == w2[0].size(0) == dim
               and sup(B, dim, dt, wq) and sup(B, dim, dt, wk) and sup(B, dim, dt, wv)
               and sup(B, n_q, dt, wo)
               and sup(B, dim, dt, w1, swiglu=True) and sup(B, dim, dt, w3)
-              and sup(B, w1[0].shape[0], dt, w2))
+              and sup(B, w1[0].size(0), dt, w2))
         if not ok:
             return None
         prologue = tuple(decode_layer.norm_supported(B, dim, dt, norm.weight)
-                         for norm in (self.attention_norm, self.ffn_norm))
+                         for norm in norms)
         # past the prologue the op chain served (and at a position outside the cache
         # refused) these rows: it still does where a module's call is observed
         if not all(prologue) and not (
                 (positions is not None or 0 <= int(start_pos) < kv_cache.k.shape[3])
-                and _plain(attn.wq, attn.wk, attn.wv, attn.wo, ff.w1, ff.w3, ff.w2)
-                and _no_hooks(attn, ff, self.attention_norm, self.ffn_norm)):
+                and _plain(*lins) and _no_hooks(attn, ff, *norms)):
             return None
-        return ws, prologue
+        return ws, norms, prologue
 
     def forward(self, x, rope_cos, rope_sin, layer_idx=None, start_pos=0, kv_cache=None,
                 use_cuda_graph=False, scatter_positions=None, decode_attn_mask=None, **ext):
@@ -215,7 +226,7 @@ class QuantizedTransformerBlock(TransformerBlock):
                                    kv_cache=kv_cache, use_cuda_graph=use_cuda_graph,
                                    scatter_positions=scatter_positions,
                                    decode_attn_mask=decode_attn_mask, **ext)
-        ws, (qkv_norms, ffn_norms) = fused
+        ws, (norm, ffn_norm), (qkv_norms, ffn_norms) = fused
         wo, w1, w3, w2 = ws[3:]
         B, _, dim = x.shape
         x2 = x.view(B, dim)
@@ -232,7 +243,6 @@ class QuantizedTransformerBlock(TransformerBlock):
             else:
                 pos = torch.full((1,), p, dtype=torch.int64, device=x.device)
             row0 = 0 if by_pos else p
-        norm = self.attention_norm
         h, nw = (x2, norm.weight) if qkv_norms else (norm(x2), None)
         q = decode_layer.qkv_rope_append(h, self.attention, nw, norm.eps, rope_cos, rope_sin,
                                          row0, pos, kv_cache, layer_idx, weights=ws[:3])
@@ -241,9 +251,8 @@ class QuantizedTransformerBlock(TransformerBlock):
             ck, cv = ck[:, :, :int(start_pos) + 1], cv[:, :, :int(start_pos) + 1]
         o = flash_decode(q, ck, cv, mask=decode_attn_mask, seq_lens=ext.get("seq_lens"))
         h = decode_layer.linear_fused(o.view(B, -1), wo, residual=x2)
-        norm = self.ffn_norm
-        n, nw = (h, norm.weight) if ffn_norms else (norm(h), None)
-        g = decode_layer.linear_fused(n, w1, norm_weight=nw, eps=norm.eps, lin_b=w3)
+        n, nw = (h, ffn_norm.weight) if ffn_norms else (ffn_norm(h), None)
+        g = decode_layer.linear_fused(n, w1, norm_weight=nw, eps=ffn_norm.eps, lin_b=w3)
         y = decode_layer.linear_fused(g, w2, residual=h)
         return y.view(B, 1, dim)
 
