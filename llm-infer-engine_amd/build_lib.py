@@ -2,8 +2,8 @@
 
 Usage: python build_lib.py [--report]     (--report prints per-kernel VGPR/LDS use)
 
-The library is built in-tree (next to this file) so it travels with the repo
-snapshot to the GPU box; it is never pip-installed.
+The library is built in-tree (next to this file) and travels with the source
+tree; it is never pip-installed.
 """
 from __future__ import annotations
 
@@ -23,7 +23,8 @@ INCLUDE = HERE.parent / "include"
 
 ARCH = "gfx950"
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
-# Packed-FP32 VALU ops are disabled for all device code.
+# Packed-FP32 VALU ops are disabled for all device code: some of their forms have
+# given wrong results now and then.
 COMMON = [
     f"--offload-arch={ARCH}",
     "-O3",

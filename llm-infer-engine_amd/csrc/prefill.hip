@@ -78,9 +78,10 @@ struct PrefillArgs {
 // so that the two add up to the same work and stay resident together to the end
 // (a CU with one block left runs at 0.8 of its rate with two); the few past two
 // per CU are the lightest and fill the first free slots.  With more blocks the
-// dispatch itself balances heaviest-first order.  MI355X, 32/8 heads, D = 64: B1
-// S4534 103.9 -> 94.2 us, B2 S2295 56.5 -> 51.6, B4 S1024 27.9 -> 26.4; at D = 128
-// the longest block decides and the order changes nothing (-4 to +1.5 %).
+// dispatch itself balances heaviest-first order.  MI355X, 32/8 heads, D = 64, per call
+// in a graph, heaviest first throughout -> this: B1 S4534 103.4 -> 93.4 us, B2 S2295
+// 56.7 -> 51.6, B4 S1024 28.7 -> 27.1; at D = 128 the longest block decides and the
+// order changes nothing (-4 to +1.5 %).
 template <bool PAIR>
 __device__ inline void block_of_grid(const PrefillArgs& a, int& pair, int& pb) {
   const int n_pairs = a.B * a.Hkv * a.head_chunks, bid = blockIdx.x;
@@ -1641,19 +1642,22 @@ __device__ inline f32x4 visible_keys_f32(const PrefillArgs& a, int b, int head,
 // FMAs).  A block is 32 query rows of one head; its 4 waves take the 32-key tiles
 // in turn and merge their (m, l, O) in LDS at the end, because a prompt of a few
 // hundred rows has too few row blocks to fill the SIMDs any other way and one
-// tile is 2 D x 64 matrix cycles long.
+// tile is D x 64 matrix cycles long (D products of 64 cycles).
 //  * S^T = K Q^T: each lane then holds 16 scores of one query (its column), and
 //    accumulator i is key 8 (i / 4) + 4 h + i % 4 for lane half h -- exactly a B
 //    operand of O^T += V^T P^T whose two k slots are those two keys, so P needs
 //    no shuffle and V's lanes read 32 consecutive floats of that key's row.
-//  * K and V come straight from global memory (L2): a tile is 2 D x 64 matrix
-//    cycles against 128 D bytes; V of a tile is requested before its QK products
-//    and K of the next tile before its PV products.
-//  * row blocks are dealt heaviest first, then lightest first, so that a CU's two
-//    blocks add up to the same work.
+//  * K and V come straight from global memory (L2): a tile is D x 64 matrix cycles
+//    against 256 D bytes; V of a tile is requested before its QK products and K of
+//    the next tile before its PV products.
+//  * the heavier half of the row blocks goes out first, heaviest first, then the
+//    lighter half, lightest first.  At D = 64 and 128 a wave holds 270 and 398
+//    registers, so a CU has one block at a time (two at D = 32) and a wave's own
+//    requests ahead are all that covers its load and softmax latency: that, and the
+//    second round that the 512 blocks of the call below take, is what bounds it.
 // Same online softmax in fp32 as prefill_valu_kernel.  MI355X against that kernel,
-// in a graph: one prompt of 512 rows, 32/8 heads, D = 64: 64.3 -> 23.8 us; 1024
-// rows 230 -> 65; 24/8 heads, D = 128, 512 rows 119 -> 37; 33 rows 7.6 -> 5.8.
+// in a graph: one prompt of 512 rows, 32/8 heads, D = 64: 65.6 -> 24.7 us; 1024
+// rows 232 -> 66; 33 rows 8.4 -> 6.7; 24/8 heads, D = 128, 512 rows 118 -> 37.4.
 template <int D>
 __global__ __launch_bounds__(256) void prefill_f32_kernel(PrefillArgs a) {
   constexpr int DH = D / 2, NB = D / 32, DP = D < 64 ? D : 64;   // DP: dims per merge pass

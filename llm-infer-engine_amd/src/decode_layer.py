@@ -42,7 +42,8 @@ def raw_weights(lin):
     return (lin.weight if w is None else w), (lin.scales if s is None else s)
 
 
-#: reduction lengths the fused GEMV kernels are built for (K = 512 * waves)
+#: reduction lengths the fused GEMV kernels are built for (K split over a block's waves,
+#: 1 to 4 chunks of 128 each up to 8 rows, 2 to 8 of 64 above)
 SUPPORTED_K = (512, 1024, 1536, 2048, 3072, 4096, 6144, 8192)
 #: bytes that x, and a weight matrix, must stay below (the kernels' 32-bit offsets)
 _SPAN = 1 << 31
