@@ -96,9 +96,14 @@ def _children(module, *names):
 
 
 def _rows_fusable(x2, lin, *, swiglu=False) -> bool:
-    """Whether the decode projection kernels take rows x2 [M <= 16, K] through `lin`."""
-    return (1 <= x2.shape[0] <= 16
-            and decode_layer.supported(x2.shape[0], x2.shape[1], x2.dtype, lin, swiglu=swiglu)
+    """Whether the decode projection kernels take rows x2 [M <= 16, K] through `lin`
+    (whose weight has the rows it names: outputs and residual are sized by them)."""
+    M, K = x2.shape
+    if not 1 <= M <= 16:
+        return False
+    pair = decode_layer.weights_of(lin)
+    return (pair[0].size(0) == lin.out_features
+            and decode_layer.supported(M, K, x2.dtype, pair, swiglu=swiglu)
             and decode_layer.aligned(x2))
 
 

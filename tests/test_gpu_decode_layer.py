@@ -386,6 +386,21 @@ def test_decode_weights_of_other_heads_are_refused(dev):
             block(x, *rope, layer_idx=0, start_pos=7, kv_cache=kv)
 
 
+def test_feed_forward_weights_of_other_sizes_are_refused(dev):
+    """A w2 or w1 / w3 with other rows than the module names: refused, and the residual
+    is not read by the weight's rows."""
+    for names, rows in ((("w2",), 2048), (("w1", "w3"), 512)):
+        block, _, _, _ = _watched_block(dev, 1024, 1, 1)
+        ff = block.feed_forward
+        for name in names:
+            lin = getattr(ff, name)
+            lin.weight.data = lin.weight.repeat(2, 1)[:rows].clone()
+            lin.scales.data = lin.scales.repeat(2, 1)[:rows].clone()
+        x = randn((3, 1024), 92, torch.bfloat16, dev)
+        with torch.no_grad(), pytest.raises((RuntimeError, ValueError)):
+            ff(x, residual=x)
+
+
 def test_unsupported_shapes_are_rejected(dev):
     """K outside the built set, M > 16: the C side refuses (nothing launched)
     and the model-level predicate routes such calls to the op chain."""
