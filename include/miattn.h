@@ -189,8 +189,13 @@ int64_t mi_decode_effective_splits(int64_t batch, int64_t n_heads, int64_t n_kv_
 
 /*
  * Split count the library would pick for a decode of this shape on the
- * current device (used when the caller passes no explicit num_splits).
+ * current device (used when the caller passes no explicit num_splits):
+ * mi_decode_call_splits for a dtype code and for a call with a mask
+ * (masked != 0) or without, mi_decode_default_splits for bf16 without one.
  */
+int64_t mi_decode_call_splits(int64_t batch, int64_t n_heads, int64_t n_kv_heads,
+                              int64_t kv_len, int64_t head_dim, int32_t dtype,
+                              int32_t masked);
 int64_t mi_decode_default_splits(int64_t batch, int64_t n_heads,
                                  int64_t n_kv_heads, int64_t kv_len,
                                  int64_t head_dim);

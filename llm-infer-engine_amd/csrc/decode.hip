@@ -353,6 +353,12 @@ extern "C" int32_t mi_decode_arrive_counters(void* stream, uint64_t** counters) 
 extern "C" int64_t mi_decode_default_splits(int64_t batch, int64_t n_heads,
                                             int64_t n_kv_heads, int64_t kv_len,
                                             int64_t head_dim) {
+  return mi_decode_call_splits(batch, n_heads, n_kv_heads, kv_len, head_dim, MI_DTYPE_BF16, 0);
+}
+
+extern "C" int64_t mi_decode_call_splits(int64_t batch, int64_t n_heads, int64_t n_kv_heads,
+                                         int64_t kv_len, int64_t head_dim, int32_t dtype,
+                                         int32_t masked) {
   if (batch <= 0 || n_heads <= 0 || n_kv_heads <= 0 || kv_len <= 0) return 1;
   if (!supported_head_dim(head_dim)) head_dim = 128;
   const int64_t G = n_heads / n_kv_heads;
@@ -368,13 +374,18 @@ extern "C" int64_t mi_decode_default_splits(int64_t batch, int64_t n_heads,
   // B8 Hkv8 D64 at 4097 of 8192 keys, 4 splits 22.9 us vs 8 splits 25.0 us).
   const int64_t row_bytes = 2LL * 2 * head_dim;                            // bf16 K + V
   const int64_t s_bytes = (kv_len * row_bytes + (512 << 10) - 1) / (512 << 10);
-  // One block per CU; but no second split where half the CUs have a block already, up
-  // to 1024 keys or head_dim 32 (B16 Hkv8 D64, 512 keys 11.4 -> 10.2 us, 1024 keys 12.0 ->
-  // 10.8 with one split, D32 1100 keys 10.1 -> 8.4; D64 at 1500 keys two splits 15.9, one 16.6)
-  const int64_t s_cover = 2 * units >= cus && (kv_len <= 1024 || head_dim <= 32)
-                              ? 1 : (cus + units - 1) / units;
+  // One block per CU; but no second split where half the CUs have a block already and the
+  // context is short: without a mask up to 1024 keys or head_dim 32 (B16 Hkv8 D64, 512 keys
+  // 11.4 -> 10.2 us, 1024 keys 12.0 -> 10.8 with one split, D128 777 keys 15.2 -> 14.6, D32
+  // 1100 keys 10.1 -> 8.4; D64 at 1500 keys two splits 15.9, one 16.6), with one up to
+  // 256 KB of K + V a sequence (D128 at 1024 keys two splits 19.3, one 21.2), not for fp32
+  // (D64 at 777 keys two splits 16.0, one 17.4)
+  const bool small = dtype != MI_DTYPE_F32 &&
+                     (masked != 0 ? kv_len * row_bytes <= (256 << 10)
+                                  : kv_len <= 1024 || head_dim <= 32);
+  const int64_t s_cover = 2 * units >= cus && small ? 1 : (cus + units - 1) / units;
   if (s > s_bytes) s = s_bytes > s_cover ? s_bytes : s_cover;
-  // One split up to 256 keys.  Above, splits whose keys are a full pass of 4 waves (128 at
+  // One split up to 256 keys (128 KB).  Above, splits whose keys are a full pass of 4 waves (128 at
   // D64, 64 at D128) at least: one key fewer halves a block's waves (make_plan), so 12
   // splits of 1500 keys (125 each) are slower than 11 (137); and 128 at least up to 1024
   // keys, where partials and combine cost more than the parallelism gains.  B1 Hkv8 D64,
@@ -383,8 +394,21 @@ extern "C" int64_t mi_decode_default_splits(int64_t batch, int64_t n_heads,
   // 777 keys 12.2 -> 9.8, 2048 keys 10.4 at 32 splits, 11.3 at 16.
   const HostGeom geo = host_geom(MI_DTYPE_BF16, head_dim);
   const int64_t full = std::clamp(4 * geo.rpw * geo.u, 64, 128);
-  int64_t s_keys = kv_len <= 256 ? 1 : (kv_len - 1) / (full - 1);   // ceil(kv_len / s) >= full
-  if (kv_len <= 1024) s_keys = std::min(s_keys, (kv_len + 127) / 128);
+  int64_t s_keys;
+  if (kv_len <= 256 && kv_len * row_bytes <= (128 << 10)) {
+    s_keys = 1;
+  } else if (dtype != MI_DTYPE_F32 && head_dim <= (masked != 0 ? 64 : 128)) {
+    s_keys = (kv_len - 1) / (full - 1);   // ceil(kv_len / s) >= full
+    if (kv_len <= 1024) s_keys = std::min(s_keys, (kv_len + 127) / 128);
+  } else {
+    // The single-buffered kernels (a mask past head_dim 64, fp32) and 1 KB rows pay a round
+    // trip per few keys: 64 keys a split, 8 splits at most up to 1024 keys.  B1 D128 with a mask, 511
+    // keys 11.8 us with 8 splits, 12.7 with 4; B3, 1024 keys 16.4 with 11, 14.1 with 8;
+    // fp32 B1 D64, 511 keys 8.5 with 8, 9.3 with 4; B2 D256, 300 keys 8.1 with 5, 8.7 with 3.
+    s_keys = (kv_len + 63) / 64;
+    if (kv_len <= 1024 && !(dtype == MI_DTYPE_F32 && masked != 0))   // B1 D64: 16 11.3 us, 8 12.4
+      s_keys = std::min<int64_t>(s_keys, 8);
+  }
   if (s > s_keys) s = s_keys;
   if (s < 1) s = 1;
   if (s > kMaxSplits) s = kMaxSplits;

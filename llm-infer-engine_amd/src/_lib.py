@@ -83,6 +83,7 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
     ]),
     "mi_decode_arrive_counters": (_i32, [_ptr, _ptr]),      # stream, uint64_t** out
     "mi_decode_default_splits": (_i64, [_i64, _i64, _i64, _i64, _i64]),
+    "mi_decode_call_splits": (_i64, [_i64, _i64, _i64, _i64, _i64, _i32, _i32]),
     "mi_decode_effective_splits": (_i64, [_i64, _i64, _i64, _i64, _i64, _i64]),
     "mi_attn_prefill": (_i32, [
         _ptr, _ptr, _ptr, _ptr, _ptr,          # q k v out lse

@@ -72,7 +72,8 @@ def _run_decode(q, k, v, mask, seq_lens, num_splits, return_lse, empty_nan, what
             seq_lens = seq_lens.to(device=q.device, dtype=torch.int64)
     lib = _lib.load()
     if num_splits is None:
-        num_splits = lib.mi_decode_default_splits(batch_size, n_heads, n_kv_heads, kv_len, head_dim)
+        num_splits = lib.mi_decode_call_splits(batch_size, n_heads, n_kv_heads, kv_len, head_dim,
+                                               _lib.dtype_code(q.dtype), int(mask is not None))
     num_splits = int(num_splits)
     if num_splits < 1:
         raise ValueError(f"num_splits must be >= 1, got {num_splits}")

@@ -120,6 +120,25 @@ def test_default_split_counts(batch, head_dim, keys, splits):
     assert s == 1 or -(-keys // s) >= (64 if head_dim == 128 else 128)
 
 
+@pytest.mark.parametrize("batch,head_dim,keys,plain,masked,fp32,fp32_masked", [
+    (1, 64, 256, 1, 1, 1, 1), (1, 64, 300, 2, 2, 5, 5), (1, 64, 1024, 8, 8, 8, 16), (1, 64, 1500, 11, 11, 24, 24),
+    (1, 128, 300, 3, 5, 5, 5), (1, 128, 511, 4, 8, 8, 8), (1, 128, 1024, 8, 8, 8, 16), (1, 128, 2048, 32, 32, 32, 32),
+    (1, 256, 128, 1, 1, 1, 1), (1, 256, 200, 4, 4, 4, 4), (1, 256, 300, 5, 5, 5, 5), (1, 256, 1024, 8, 8, 8, 16),
+    # half the CUs have a block: no second split up to 1024 keys, 256 KB of K + V with a mask
+    (16, 64, 1024, 1, 1, 2, 2), (16, 64, 1025, 2, 2, 2, 2), (16, 128, 512, 1, 1, 2, 2), (16, 128, 777, 1, 2, 2, 2),
+    (16, 32, 2048, 1, 1, 2, 2), (16, 32, 4096, 1, 2, 2, 2)])
+def test_split_counts_of_masked_and_fp32_calls(batch, head_dim, keys, plain, masked, fp32, fp32_masked):
+    """Default splits by data type and mask: the single-buffered kernels (fp32, a mask
+    past head_dim 64) and head_dim 256 take more and shorter splits of a short context."""
+    from src import _lib
+    from src.flash_decode import default_num_splits
+    lib, heads = _lib.load(), 24 if head_dim == 128 else 32
+    got = [lib.mi_decode_call_splits(batch, heads, 8, keys, head_dim, code, m)
+           for code, m in ((0, 0), (1, 0), (0, 1), (1, 1), (2, 0), (2, 1))]
+    assert got == [plain, plain, masked, masked, fp32, fp32_masked]
+    assert default_num_splits(batch, heads, 8, keys, head_dim) == plain
+
+
 def test_rope_kv_append_rejects_out_of_capacity():
     from src import _lib
     lib = _lib.load()
