@@ -73,16 +73,16 @@ def supported(M: int, K: int, dtype: torch.dtype, lin, norm_weight=None, *,
 
 def norm_supported(M: int, K: int, dtype: torch.dtype, norm_weight) -> bool:
     """Whether the projections' RMSNorm prologue takes [M, K] rows and this weight."""
-    return (norm_weight.dtype == dtype and norm_weight.is_contiguous()
-            and norm_weight.data_ptr() % 16 == 0 and M * K * 2 <= 64 * 1024
-            and (M <= 8 or K <= 2048))
+    return (M * K * 2 <= 64 * 1024 and (M <= 8 or K <= 2048)
+            and norm_weight.dtype == dtype and norm_weight.is_contiguous()
+            and norm_weight.data_ptr() % 16 == 0)
 
 
 def aligned(x: torch.Tensor) -> bool:
     """Rows of x [M, K] are unit-stride, 16-byte aligned and span less than 2 GB."""
     row, size = x.stride(0), x.element_size()
     return (x.is_cuda and x.stride(1) == 1 and x.data_ptr() % 16 == 0 and (row * size) % 16 == 0
-            and ((x.shape[0] - 1) * row + x.shape[1]) * size < _SPAN)
+            and ((x.size(0) - 1) * row + x.size(1)) * size < _SPAN)
 
 
 def linear_fused(x, lin, *, norm_weight=None, eps: float = 0.0, lin_b=None, residual=None):

@@ -60,7 +60,7 @@ class QuantizedFeedForward(FeedForward):
         GEMM's sizes projections that are not ``_plain``, take the op chain of
         src/model.py:23."""
         x2 = x.reshape(-1, x.shape[-1])
-        w1, w3 = self.w1, self.w3
+        w1, w3 = _children(self, "w1", "w3")
         plain = _plain(w1, w3)
         if (plain and x2.shape[0] <= 16 and w1.weight.shape == w3.weight.shape
                 and _rows_fusable(x2, w1, swiglu=True) and _rows_fusable(x2, w3)):
@@ -82,7 +82,7 @@ class QuantizedFeedForward(FeedForward):
         return out
 
     def down(self, h, residual=None):
-        return _project_residual(self.w2, h, residual)
+        return _project_residual(*_children(self, "w2"), h, residual)
 
 
 def _pairs(*lins):
@@ -192,10 +192,10 @@ class QuantizedTransformerBlock(TransformerBlock):
                 or rope_cos.dtype != dt or attn.head_dim % 16 != 0 or not x.is_contiguous()
                 or not decode_layer.aligned(x.view(B, dim))):
             return None
-        if (rope_cos.stride(1) != 1 or rope_cos.stride() != rope_sin.stride()
-                or rope_sin.dtype != dt or rope_sin.shape[0] != rope_cos.shape[0]
-                or kv_cache.v.dtype != dt or kv_cache.k.stride(4) != 1
-                or kv_cache.k.stride() != kv_cache.v.stride()):
+        kv, rope = kv_cache.k.stride(), rope_cos.stride()
+        if (rope[1] != 1 or rope != rope_sin.stride() or rope_sin.dtype != dt
+                or rope_sin.size(0) != rope_cos.size(0)
+                or kv[4] != 1 or kv != kv_cache.v.stride() or kv_cache.v.dtype != dt):
             return None  # the kernels take one set of strides for each pair
         lins = (*_children(attn, "wq", "wk", "wv", "wo"), *_children(ff, "w1", "w3", "w2"))
         norms = _children(self, "attention_norm", "ffn_norm")
@@ -210,12 +210,12 @@ class QuantizedTransformerBlock(TransformerBlock):
               and sup(B, w1[0].size(0), dt, w2))
         if not ok:
             return None
-        prologue = tuple(decode_layer.norm_supported(B, dim, dt, norm.weight)
-                         for norm in norms)
+        prologue = (decode_layer.norm_supported(B, dim, dt, norms[0].weight),
+                    decode_layer.norm_supported(B, dim, dt, norms[1].weight))
         # past the prologue the op chain served (and at a position outside the cache
         # refused) these rows: it still does where a module's call is observed
-        if not all(prologue) and not (
-                (positions is not None or 0 <= int(start_pos) < kv_cache.k.shape[3])
+        if not (prologue[0] and prologue[1]) and not (
+                (positions is not None or 0 <= int(start_pos) < kv_cache.k.size(3))
                 and _plain(*lins) and _no_hooks(attn, ff, *norms)):
             return None
         return ws, norms, prologue
