@@ -144,7 +144,7 @@ class QuantizedAttention(Attention):
         super().__init__(args, linear)
 
     def out_proj(self, output, residual=None):
-        return _project_residual(self.wo, output, residual)
+        return _project_residual(*_children(self, "wo"), output, residual)
 
     def qkv(self, x):
         """wq, wk and wv in one launch: of the large GEMM (bitwise the three
@@ -152,7 +152,7 @@ class QuantizedAttention(Attention):
         GPU, else of the small-M GEMM; sizes neither takes, and modules that are
         not ``_plain`` at the small-M GEMM's, run one W8A16Linear call each."""
         x2 = x.reshape(-1, x.shape[-1])
-        mats = (self.wq, self.wk, self.wv)
+        mats = _children(self, "wq", "wk", "wv")
         if quant_linear.gemm_multi_worth(x2.shape[0], x2.shape[1],
                                          [m.out_features for m in mats], x.device):
             ys = quant_linear.w8a16_gemm_multi(x2, _pairs(*mats))

@@ -196,11 +196,14 @@ _CUS: dict = {}
 
 def _cu_count(device) -> int:
     """Compute units of `device` (looked up once per device)."""
-    idx = torch.device(device).index
-    idx = torch.cuda.current_device() if idx is None else idx
-    if idx not in _CUS:
-        _CUS[idx] = torch.cuda.get_device_properties(idx).multi_processor_count
-    return _CUS[idx]
+    n = _CUS.get(device)     # a tensor's device, most often
+    if n is None:
+        idx = torch.device(device).index
+        n = torch.cuda.get_device_properties(
+            torch.cuda.current_device() if idx is None else idx).multi_processor_count
+        if idx is not None:
+            _CUS[device] = n
+    return n
 
 
 def w8a16_gemm_residual(x, weight, scales, res, *, splits: int | None = None):
