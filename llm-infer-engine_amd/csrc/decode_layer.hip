@@ -19,9 +19,9 @@
 // reference's separate ops do (src/rope.py:85-86, src/model.py:23, :113-127).
 //
 // GEMV design (MI355X): the int8 weights are the only large operand and are
-// read once.  A workgroup owns a few tiles of 8 (up to 8 token rows) or 16
-// output rows of one (or, for SwiGLU, two) weight matrices and its waves split
-// K.  The products run on v_mfma_f32_16x16x32_{bf16,f16}: weight rows are the A
+// read once.  A workgroup owns a few tiles of 8 (up to 8 token rows, or where
+// larger tiles would leave half the CUs idle) or 16 output rows of one (or, for
+// SwiGLU, two) weight matrices and its waves split K.  The products run on v_mfma_f32_16x16x32_{bf16,f16}: weight rows are the A
 // operand (int8 converted exactly in registers), x^T the B operand with the
 // columns beyond M zero.  A wave issues every load of its K slice before its
 // first MFMA, so the whole matrix is in flight at once (these GEMVs are
@@ -432,7 +432,8 @@ __device__ inline u32x4 rows_hi(const u32x4& a, const u32x4& b) {
 // r and of token row r for each 64-k chunk (two MFMAs); the weights of a pair of
 // chunks are loaded as whole 128-byte lines of 8 rows (rows_lo / rows_hi).  A block has NW waves
 // that split K (SC consecutive chunks each, K = 64 * NW * SC) and owns TPB
-// 16-row tiles of each of its NMAT matrices: every wave reads its slice of x
+// tiles of RT rows (16, or 8 with the other A rows unused) of each of its NMAT
+// matrices: every wave reads its slice of x
 // once, straight into the B registers, for all of the block's tiles.  x is what
 // bounds these calls, not the weights: a block with one tile reads twice as
 // many bytes of x (16 rows of 2 bytes) as of int8 weights, so tiles are grouped
