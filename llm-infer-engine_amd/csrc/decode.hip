@@ -401,10 +401,11 @@ extern "C" int64_t mi_decode_call_splits(int64_t batch, int64_t n_heads, int64_t
     s_keys = (kv_len - 1) / (full - 1);   // ceil(kv_len / s) >= full
     if (kv_len <= 1024) s_keys = std::min(s_keys, (kv_len + 127) / 128);
   } else {
-    // The single-buffered kernels (a mask past head_dim 64, fp32) and 1 KB rows pay a round
-    // trip per few keys: 64 keys a split, 8 splits at most up to 1024 keys.  B1 D128 with a mask, 511
-    // keys 11.8 us with 8 splits, 12.7 with 4; B3, 1024 keys 16.4 with 11, 14.1 with 8;
-    // fp32 B1 D64, 511 keys 8.5 with 8, 9.3 with 4; B2 D256, 300 keys 8.1 with 5, 8.7 with 3.
+    // The single-buffered kernels (a mask past head_dim 64, fp32) and 1 KB rows pay a
+    // round trip per few keys: 64 keys a split, 8 splits at most up to 1024 keys.  B1
+    // D128 with a mask, 511 keys 11.8 us with 8 splits, 12.7 with 4; B3, 1024 keys 16.4
+    // with 11, 14.1 with 8; fp32 B1 D64, 511 keys 8.5 with 8, 9.3 with 4; B2 D256, 300
+    // keys 8.1 with 5, 8.7 with 3.
     s_keys = (kv_len + 63) / 64;
     if (kv_len <= 1024 && !(dtype == MI_DTYPE_F32 && masked != 0))   // B1 D64: 16 11.3 us, 8 12.4
       s_keys = std::min<int64_t>(s_keys, 8);

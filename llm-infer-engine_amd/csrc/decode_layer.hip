@@ -21,12 +21,13 @@
 // GEMV design (MI355X): the int8 weights are the only large operand and are
 // read once.  A workgroup owns a few tiles of 8 (up to 8 token rows, or where
 // larger tiles would leave half the CUs idle) or 16 output rows of one (or, for
-// SwiGLU, two) weight matrices and its waves split K.  The products run on v_mfma_f32_16x16x32_{bf16,f16}: weight rows are the A
-// operand (int8 converted exactly in registers), x^T the B operand with the
-// columns beyond M zero.  A wave issues every load of its K slice before its
-// first MFMA, so the whole matrix is in flight at once (these GEMVs are
-// latency-bound: a few MB each).  With the RMSNorm prologue each wave
-// normalises its own slice of x in registers.
+// SwiGLU, two) weight matrices and its waves split K.  The products run on
+// v_mfma_f32_16x16x32_{bf16,f16}: weight rows are the A operand (int8 converted
+// exactly in registers), x^T the B operand with the columns beyond M zero.  A
+// wave issues every load of its K slice before its first MFMA, so the whole
+// matrix is in flight at once (these GEMVs are latency-bound: a few MB each).
+// With the RMSNorm prologue each wave normalises its own slice of x in
+// registers.
 #include <math.h>
 #include <type_traits>
 
