@@ -233,6 +233,10 @@ def w8a16_gemm_residual(x, weight, scales, res, *, splits: int | None = None):
     return out
 
 
+#: below this K the small-M GEMM never splits it (2048 k a split at least)
+SMALL_GEMM_SPLIT_K = 4096
+
+
 def _small_gemm_takes(M: int, K: int) -> bool:
     """Sizes mi_w8a16_small_gemm is built for (and used for: 17 rows and more)."""
     return _GEMV_MAX_ROWS < M <= 65535 and K % (256 if M <= 64 else 128) == 0
@@ -272,7 +276,8 @@ def small_gemm_fuses(x, mats) -> bool:
     return (_small_gemm_takes(M, K) and len({s.dtype for _, s in mats}) == 1
             and (M >= GEMM_MIN_ROWS or all(K <= t.stride(0) <= (1 << 23) and t.stride(1) == 1
                                            for t in (x, *(w for w, _ in mats))))
-            and all(lib.mi_w8a16_small_gemm_splits(M, w.shape[0], K) == 1 for w, _ in mats))
+            and (K < SMALL_GEMM_SPLIT_K
+                 or all(lib.mi_w8a16_small_gemm_splits(M, w.shape[0], K) == 1 for w, _ in mats)))
 
 
 def gemm_multi_worth(M: int, K: int, out_features, device) -> bool:

@@ -81,6 +81,17 @@ def test_host_tensors_never_reach_a_kernel(monkeypatch):
         kv.update_positions(0, torch.zeros(2, dtype=torch.long), _t(1, 1, 2, 32), _t(1, 1, 2, 32))
 
 
+def test_small_gemm_splits_no_short_k():
+    """small_gemm_fuses asks for split counts only from SMALL_GEMM_SPLIT_K on."""
+    from src import _lib
+    from src.quant_linear import SMALL_GEMM_SPLIT_K
+    splits = _lib.load().mi_w8a16_small_gemm_splits
+    for m in (17, 64, 65, 300, 2000):
+        for n in (16, 512, 2048, 16384):
+            assert splits(m, n, SMALL_GEMM_SPLIT_K - 256) == 1
+    assert splits(48, 2048, SMALL_GEMM_SPLIT_K) > 1
+
+
 def test_model_args_defaults_are_llama_3_2_1b():
     from src.config import ModelArgs
     a = ModelArgs()
